@@ -466,6 +466,32 @@ def test_one_element_path_matches_vector_path(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("V", [1, 7, 9, 4097, 50257])
+def test_backward_rows_at_different_offsets_bitwise(dtype, V):
+    """Rows of logits at every offset within 16 bytes from their gradient's
+    rows give the bits of rows that share it, over row ends, one piece and
+    several, with and without a temperature."""
+    from kernel_opt import _C
+    N = 8
+    per = 16 // torch.empty((), dtype=dtype).element_size()
+    x = seeded_logits((N, V), dtype, seed=62).to(DEV)
+    t = seeded_targets((N,), V, seed=62).to(DEV)
+    gl, ge, gs = (torch.linspace(lo, 0.5, N, device=DEV) for lo in (-0.5, 0.1, 0.2))
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    for temperature in (None, 0.7):
+        outs = [torch.empty(N, device=DEV) for _ in range(3)]
+        _C.fwd_launch(x, t, *outs, temperature=temperature)
+        want = torch.empty((N, V), dtype=dtype, device=DEV)
+        _C.bwd_launch(x, t, outs[2], outs[1], gl, ge, gs, want, temperature=temperature)
+        for off in range(1, per):
+            base = torch.empty(N * V + off, dtype=dtype, device=DEV)
+            shifted = base[off:].view(N, V).copy_(x)
+            got = torch.full((N, V), float("nan"), dtype=dtype, device=DEV)
+            _C.bwd_launch(shifted, t, outs[2], outs[1], gl, ge, gs, got, temperature=temperature)
+            assert torch.equal(got.view(bits), want.view(bits)), (off, temperature)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_special_rows(dtype):
     """Whole row -inf, a NaN, a +inf: same outcome classes as the reference
     v1 kernel (lse -inf / entropy NaN; NaN rows; NaN for +inf)."""

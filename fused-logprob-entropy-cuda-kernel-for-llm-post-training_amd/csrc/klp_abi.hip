@@ -482,23 +482,41 @@ int grpo_setup(const float* logp, const float* old_logp, const float* ref_logp,
     return KLP_OK;
 }
 
-// Fused LM head: vocab tiles per workgroup chunk, chosen so that the grid
-// holds about four rounds of one workgroup per CU (256 CUs).
+// Fused LM head: vocab tiles per workgroup chunk.  A CU holds one workgroup,
+// so the launch takes (rounds of 256 workgroups) * (tiles per workgroup) tile
+// times, plus each round's prologue and merge (about 1/8 of a tile time at
+// dim 3584); of 1..16 tiles the count with the least of that is taken, the
+// fewest tiles on a tie.  1024 tokens of [152064, 3584]: 5 tiles (2 rounds)
+// 828-840 us, 2 tiles (5 rounds) 848-862, 3 tiles (4 rounds, 12 tile times
+// for 9.3 tiles of work per CU) 957, main loop alone.
 void lmh_plan(int64_t n_tokens, int64_t vocab, int64_t* tiles_per_chunk, int64_t* n_chunks) {
+    constexpr int64_t kCus = 256;
     const int64_t tb = klp::lmh_token_blocks(n_tokens);
     const int64_t vt = klp::lmh_vocab_tiles(vocab);
-    int64_t tpc = (tb * vt) / (256 * 4);
-    if (tpc < 1) tpc = 1;
-    if (tpc > 16) tpc = 16;
-    *tiles_per_chunk = tpc;
-    *n_chunks = (vt + tpc - 1) / tpc;
+    int64_t best = 1, best_cost = INT64_MAX;
+    for (int64_t tpc = 1; tpc <= 16 && tpc <= vt; ++tpc) {
+        const int64_t chunks8 = ((vt + tpc - 1) / tpc + 7) / 8 * 8;
+        const int64_t rounds = (chunks8 * tb + kCus - 1) / kCus;
+        const int64_t cost = rounds * (8 * tpc + 1);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = tpc;
+        }
+    }
+    *tiles_per_chunk = best;
+    *n_chunks = (vt + best - 1) / best;
+}
+
+// The chunks' partial states, then the target logits.
+size_t lmh_partials_bytes(int64_t n_tokens, int64_t n_chunks) {
+    return static_cast<size_t>(n_chunks) * static_cast<size_t>(n_tokens) * 4 * sizeof(float);
 }
 
 size_t lmh_workspace_bytes(int64_t n_tokens, int64_t vocab) {
     if (n_tokens <= 0 || vocab <= 0) return 0;
     int64_t tpc, nc;
     lmh_plan(n_tokens, vocab, &tpc, &nc);
-    return static_cast<size_t>(nc) * static_cast<size_t>(n_tokens) * 4 * sizeof(float);
+    return lmh_partials_bytes(n_tokens, nc) + static_cast<size_t>(n_tokens) * sizeof(float);
 }
 
 int ceiling_impl(int mode, const void* src, void* dst, int64_t n_rows, int64_t row_bytes,
@@ -1058,6 +1076,10 @@ int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
                     static_cast<long long>(dim));
     if (ld_hidden < dim || ld_weight < dim || ld_hidden % 8 != 0 || ld_weight % 8 != 0)
         return fail(KLP_EINVAL, "row strides must be >= dim and multiples of 8 elements");
+    // The kernels address 256 rows with 32-bit byte offsets.
+    if (ld_hidden > INT32_MAX / 512 || ld_weight > INT32_MAX / 512)
+        return fail(KLP_EINVAL, "row strides above %d elements are not supported",
+                    INT32_MAX / 512);
     if (n_tokens > (int64_t{1} << 31) - 1 || vocab > (int64_t{1} << 31) - 1)
         return fail(KLP_EINVAL, "n_tokens and vocab must be below 2^31");
     float scale;
@@ -1137,6 +1159,8 @@ int klp_lmh_fwd(const void* hidden, int64_t ld_hidden, const void* weight, int64
                     "workspace missing, too small or not 16-byte aligned: have %zu bytes, need %zu",
                     workspace_bytes, need);
     p.partials = static_cast<float*>(workspace);
+    p.target_logit = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) +
+                                              lmh_partials_bytes(n_tokens, p.n_chunks));
     p.logprob = logprob;
     p.entropy = entropy;
     p.lse = lse;

@@ -214,8 +214,9 @@ struct LmhParams {
     int64_t dim;             // K, a multiple of 64
     const int64_t* targets;  // [n_tokens]
     float scale;             // 1 / temperature
-    float* partials;         // [n_chunks, n_tokens] float4 (m, z, t, target logit)
-    int64_t n_tblocks;       // ceil(n_tokens / 128)
+    float* partials;         // [n_chunks, n_tokens] float4 (m, z, t, unused)
+    float* target_logit;     // [n_tokens], behind the partials; written where a target is valid
+    int64_t n_tblocks;       // ceil(n_tokens / 256)
     int64_t n_vtiles;        // ceil(vocab / 256)
     int64_t tiles_per_chunk;
     int64_t n_chunks;        // ceil(n_vtiles / tiles_per_chunk)

@@ -9,36 +9,51 @@
 // without writing the [N, V] logits anywhere.  hidden is bf16 [N, D] and
 // weight bf16 [V, D] (nn.Linear's layout), both K-contiguous.
 //
-// klp_lmh_kernel<false> (forward): one workgroup (4 waves, 2 x 2) per (token block of
+// klp_lmh_kernel<false, ..> (forward): one workgroup (4 waves, 2 x 2) per (token block of
 // 256, vocab chunk of `tiles_per_chunk` tiles of 256 rows).  Per vocab tile
-// it computes the 256 x 256 block of logits^T with v_mfma_f32_32x32x16_bf16,
-// each wave a 128 x 128 part of it (16 accumulator blocks, 256 AGPRs):
+// it computes the 256 x 256 block of logits^T with v_mfma_f32_16x16x32_bf16,
+// each wave a 128 x 128 part of it (64 accumulator blocks, 256 AGPRs):
 //  - the transposed orientation puts vocab rows on the MFMA's M side, so a
-//    lane's 16 accumulator values all belong to one token (its N column):
-//    the online softmax update runs lane-locally, with no cross-lane
-//    reduction until the end of the chunk;
-//  - K advances in steps of 32 through a ring of 5 LDS stages (32 KB each,
-//    all 160 KB of LDS), filled by direct global -> LDS copies
-//    (global_load_lds_dwordx4, no register staging) 3-4 stages ahead of the
-//    multiply; a slot is refilled once every wave is past the MFMAs of the
-//    stage it held; the ring runs across tile boundaries;
-//  - LDS rows are 64 bytes; the 16-byte chunk index is XOR-swizzled with
+//    lane's accumulators belong to 8 tokens, 32 vocab rows of each: the
+//    online softmax update runs lane-locally, with no cross-lane reduction
+//    until the end of the chunk;
+//  - K advances in stages of 64 columns, a whole 128-byte line of every row,
+//    so that no line is asked for in two halves (with 64-byte stages 40% of
+//    the CU's cycles went to requests waiting behind a pending miss of their
+//    own line);
+//  - the stages go through LDS by direct copies (buffer_load_dwordx4 ... lds,
+//    no register staging), all 160 KB of it: a ring of 3 stages of weight
+//    rows (32 KB each), which come from HBM, and of 2 stages of hidden rows,
+//    which the XCD's L2 holds.  A slot is refilled once every wave has read
+//    the stage it held: weight copies have 1.75 stages to land, hidden ones
+//    0.75.  The rings run across tile boundaries, and past the last stage
+//    the copies go through a descriptor of length 0, which keeps the count
+//    of copies in flight, and with it the vmcnt waits, the same on every path;
+//  - LDS rows are 128 bytes; the 16-byte chunk index is XOR-swizzled with
 //    row bits 0..3 (swz_f) so that the MFMA operand reads are free of bank
 //    conflicts;
-//  - a stage's operands are read in two 16-column halves, ping-ponged: the
-//    MFMAs of one half run while the other half is read from LDS (the next
-//    stage's first half under the current stage's second), one barrier per
-//    stage between the halves;
+//  - operands are read one half stage (32 columns) ahead, two ds_reads per
+//    8 MFMAs in source order, and each copy has a slot between two MFMAs;
+//    there is one barrier per stage, after the last read of the stage;
 //  - after each tile the block's logits are folded into per-lane
-//    (m, z, t) states (absorb() of klp_device.h) and the target logit is
-//    captured if it lies in the tile.
-// At the end of the chunk, lanes l and l+32 (same token) and the two waves
-// of a token half merge; the chunk's partial state per token goes to the
-// workspace.  klp_lmh_combine_kernel merges the chunks of each token (one
+//    (m, z, t) states (absorb() of klp_device.h), 32 values of a token at a
+//    time; only the tile at the vocabulary's end compares rows, and only
+//    tokens whose target lies in the tile look for it.
+// At the end of the chunk the four lanes of a token and the two waves of a
+// token half merge; the chunk's partial state per token goes to the
+// workspace, and a target's logit straight from the lane that holds it.  klp_lmh_combine_kernel merges the chunks of each token (one
 // wave per token, a fixed order) and applies the output formulas.
 //
-// klp_lmh_kernel<true> (backward) runs the same tiles and replaces the fold
+// klp_lmh_kernel<true, ..> (backward) runs the same tiles and replaces the fold
 // with the gradient of klp_bwd, written to d_logits as bf16.
+//
+// Bound: power.  At 1024 tokens of a [152064, 3584] weight the MFMAs take 4/5
+// of the kernel's cycles, and the chip lowers its clock under them: 1.85 GHz,
+// against 2.4 GHz with the copies alone or the MFMAs alone (either of which
+// takes 550-600 us).  The launch pair takes 800 us (1396 TFLOP/s) end to end,
+// where 64-byte stages, 32x32x16 MFMAs and a fold that compared every element
+// with the target took 1239.  32x32x16 MFMAs at this tile and ring: 840-848
+// us against 797-821 for the main loop alone, at 1.62 against 1.85 GHz.
 //
 // Workgroup order: workgroup b runs on XCD b % 8 (round-robin dispatch).
 // Consecutive workgroups of one XCD take the token blocks of one vocab
@@ -50,74 +65,72 @@ namespace klp {
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kVB = 4;              // 32-row vocab blocks per wave
-constexpr int kTB = 4;              // 32-token blocks per wave
-constexpr int kBV = 2 * kVB * 32;   // vocab rows per tile (2 waves along vocab): 256
-constexpr int kBT = 2 * kTB * 32;   // tokens per block (2 waves along tokens): 256
-// K per LDS stage and LDS stages in the ring.  Measured: 64-wide stages (whole
-// 128-byte lines per row, a ring of 2) and non-temporal / sc0 copies were no
-// faster.
-constexpr int kBK = 32;
-constexpr int kRing = 5;
 constexpr int kThreads = 256;
+constexpr int kBlocks = 8;          // 16-row / 16-token MFMA blocks per wave and side
+constexpr int kWaveSide = kBlocks * 16;
+constexpr int kBV = 2 * kWaveSide;  // vocab rows per tile (2 waves along vocab): 256
+constexpr int kBT = 2 * kWaveSide;  // tokens per block (2 waves along tokens): 256
+constexpr int kBK = 64;             // K columns per stage
 constexpr int kRowBytes = kBK * 2;
-constexpr int kChunksPerRow = kRowBytes / 16;
-constexpr int kWBytes = kBV * kRowBytes;
-constexpr int kStageBytes = (kBV + kBT) * kRowBytes;
-// One global_load_lds_dwordx4 moves 64 lanes x 16 B = 1 KB of LDS rows.
-constexpr int kRowsPerCopy = 1024 / kRowBytes;
-constexpr int kWCopies = kBV / kRowsPerCopy / (kThreads / 64);    // per wave per stage
-constexpr int kHCopies = kBT / kRowsPerCopy / (kThreads / 64);
-constexpr int kCopiesPerStage = kWCopies + kHCopies;              // vmcnt units per stage
-static_assert(kRing * kStageBytes <= 160 * 1024, "LDS holds 160 KB");
-static_assert(kCopiesPerStage * (kRing - 2) <= 63, "vmcnt counts up to 63");
+constexpr int kSlotBytes = 256 * kRowBytes;
+constexpr int kWSlots = 3;
+constexpr int kHSlots = 2;
+constexpr int kLdsBytes = (kWSlots + kHSlots) * kSlotBytes;
+static_assert(kLdsBytes <= 160 * 1024, "LDS holds 160 KB");
+// One copy moves 64 lanes x 16 B = 1 KB, 8 LDS rows; the 4 waves' copies of
+// index j cover rows 32 j .. 32 j + 31 of a slot.
+constexpr int kCopies = 8;
 
-// LDS byte offset of 16-byte chunk `c` of row `row`.  The chunk index is
-// XOR-swizzled with f(row) (bits 0..3 of the row only): the MFMA operand
-// reads (one chunk of 16 consecutive rows per pass) are then free of bank
-// conflicts whether the LDS serves 8 or 16 lanes x 16 B per cycle.
-__device__ __forceinline__ int swz_f(int row) {
-    if constexpr (kChunksPerRow == 4) return ((row >> 1) & 3) ^ ((row >> 3) & 1);
-    else return (row & 7) ^ ((row >> 3) & 1);
-}
-__device__ __forceinline__ int swz(int row, int c) {
-    return row * kRowBytes + ((c ^ swz_f(row)) << 4);
+// The 16-byte chunk c of LDS row `row` sits at chunk c ^ swz_f(row): one
+// chunk of 16 consecutive rows, an operand read's quarter wave, then meets
+// every bank once, whether the LDS serves 8 or 16 lanes x 16 B per cycle.
+__device__ __forceinline__ int swz_f(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+
+// s_waitcnt immediate: vmcnt <= vm, lgkmcnt <= lgkm (15: no wait).
+constexpr int waitcnt(int vm, int lgkm) {
+    return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8);
 }
 
-// s_waitcnt with vmcnt = n (0..63) and no wait on the other counters.
-constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-
-// Wait until at most min(N, ahead) stages of copies issued after the
-// current one are outstanding (vmcnt takes an immediate, hence the chain).
-template <int N>
-__device__ __forceinline__ void wait_stages(int ahead) {
-    if constexpr (N > 0) {
-        if (ahead >= N) {
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm(N * kCopiesPerStage));
-            return;
-        }
-        wait_stages<N - 1>(ahead);
-    } else {
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    }
+// acc += a * b (`zero`: acc = a * b), in AGPRs and in place: left to the
+// builtin, the compiler renames the 256 accumulators from MFMA to MFMA and
+// pays for it in moves through VGPRs and spills at every join.  What it would
+// insert around its own MFMAs is then the caller's: the operands come from
+// LDS reads (waited for as any use), an accumulator's own MFMAs are 64 apart,
+// and mfma_drain() comes before other instructions read accumulators.
+__device__ __forceinline__ void mfma_in_place(f32x4& acc, bf16x8 a, bf16x8 b, bool zero) {
+    if (zero)  // a constant at every call
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
+    else
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
+// An accumulator's value, read where it is needed (the compiler would move
+// more than half of them to VGPRs ahead of the fold, and spill).
+__device__ __forceinline__ float acc_value(float acc) {
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc));
+    return v;
+}
+// The wait states between the last MFMA and a VALU read of its result (11 for
+// an MFMA of 8 passes), rounded up.
+__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 7"); }
+
+#define KLP_PIN() __builtin_amdgcn_sched_barrier(0)
 
 }  // namespace
 
 // kGrad == false: the forward (partial states per vocab chunk).
 // kGrad == true: the backward's d_logits: the same logits tiles, turned into
 // the gradient of klp_bwd (grad_one, klp_device.h) and written as bf16.
-template <bool kGrad>
+template <bool kGrad, bool kScaled>
 __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
-    // The ring takes all 160 KB of LDS; the end-of-chunk merge reuses it.
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
+    // The rings take all 160 KB of LDS; the end-of-chunk merge reuses them.
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kLdsBytes];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wv = wave & 1;   // vocab half (128 rows) of the tile
     const int wt = wave >> 1;  // token half (128 tokens) of the block
 
@@ -130,283 +143,302 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     if (chunk >= p.n_chunks) return;  // padding workgroups of the last round
 
     const int64_t tok0 = tb * kBT;
-    const int n_ksteps = static_cast<int>(p.dim / kBK);
+    const int n_k = static_cast<int>(p.dim / kBK);
     const int64_t tile_first = chunk * p.tiles_per_chunk;
     int64_t tile_end = tile_first + p.tiles_per_chunk;
     if (tile_end > p.n_vtiles) tile_end = p.n_vtiles;
-    const int n_stages = static_cast<int>(tile_end - tile_first) * n_ksteps;
 
-    // Copy slots.  Copy q of the W part covers tile rows q * kRowsPerCopy ..
-    // + kRowsPerCopy - 1; this wave issues q = wave + 4j.  Lane l fills LDS
-    // row q * kRowsPerCopy + l / kChunksPerRow, chunk l % kChunksPerRow, which
-    // holds global chunk (l % kChunksPerRow) ^ swz_f(row) of that row (swz_f
-    // reads row bits 0..3, the same for every j).  Rows past the end of the
-    // matrix are clamped to its last row (valid memory; their logits are
-    // masked or their outputs never written).
-    const int lrow = lane / kChunksPerRow;
-    const int gchunk = (lane % kChunksPerRow) ^ swz_f(wave * kRowsPerCopy + lrow);
-    const uint16_t* hsrc[kHCopies];
-#pragma unroll
-    for (int j = 0; j < kHCopies; ++j) {
-        int64_t n = tok0 + (wave + 4 * j) * kRowsPerCopy + lrow;
-        if (n > p.n_tokens - 1) n = p.n_tokens - 1;
-        hsrc[j] = p.hidden + n * p.ld_hidden + gchunk * 8;
-    }
-
-    Stat st[kTB];
-    float xt[kTB];
-    int64_t my_tgt[kTB];
-    RowGrad rg[kTB];
-#pragma unroll
-    for (int j = 0; j < kTB; ++j) {
-        st[j] = stat_empty();
-        xt[j] = 0.0f;
-        const int64_t tok = tok0 + wt * (kTB * 32) + j * 32 + (lane & 31);
-        const bool ok = tok < p.n_tokens;
-        my_tgt[j] = ok ? p.targets[tok] : -1;
-        if constexpr (kGrad) {
-            rg[j] = ok ? row_grad(p.saved_lse[tok], p.saved_entropy[tok],
-                                  p.g_logp ? p.g_logp[tok] : 0.0f,
-                                  p.g_ent ? p.g_ent[tok] : 0.0f, p.g_lse ? p.g_lse[tok] : 0.0f)
-                       : row_grad(0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
-        }
-    }
-
-    // Copies.  Stages run across the chunk's tiles: global stage g is tile
-    // tile_first + g / n_ksteps, K step g % n_ksteps, in ring slot g % kRing.
-    // `issued` stages have been issued; the W sources of the tile being issued
-    // are set once per tile and advanced by kBK columns per stage.
-    int64_t iss_vt = tile_first;
-    int iss_k = 0;
-    int issued = 0;
-    const uint16_t* wsrc[kWCopies];
-    auto point_w = [&]() {
-#pragma unroll
-        for (int j = 0; j < kWCopies; ++j) {
-            int64_t v = iss_vt * kBV + (wave + 4 * j) * kRowsPerCopy + lrow;
-            if (v > p.vocab - 1) v = p.vocab - 1;
-            wsrc[j] = p.weight + v * p.ld_weight + gchunk * 8;
-        }
+    // Copies.  Lane l of wave w fills, with copy j, chunk l % 8 of slot row
+    // 32 j + 8 w + l / 8, which holds global chunk (l % 8) ^ swz_f(row) of
+    // that row (swz_f reads row bits 0..3, the same for every j).  Rows past
+    // the matrix's end lie past the descriptor and read as zeros (their
+    // logits are masked or never written).
+    const int crow = wave * 8 + (lane >> 3);
+    const int cchunk = (lane & 7) ^ swz_f(crow);
+    const uint32_t w_off = static_cast<uint32_t>(crow * p.ld_weight * 2 + cchunk * 16);
+    const uint32_t h_off = static_cast<uint32_t>(crow * p.ld_hidden * 2 + cchunk * 16);
+    const uint32_t w_step = static_cast<uint32_t>(p.ld_weight * 64);  // 32 rows
+    const uint32_t h_step = static_cast<uint32_t>(p.ld_hidden * 64);
+    auto rows_rsrc = [](const uint16_t* base, int64_t rows, int64_t ld) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(base), 0,
+            static_cast<int>((rows < 256 ? rows : 256) * ld * 2), 0x00020000);
     };
-    point_w();
-    // Issue stages up to (not including) `limit`.  A slot may be refilled
-    // once every wave is past the MFMAs of the stage it held: the callers
-    // pass limit = h + 1 + kRing right after a barrier that follows stage h's
-    // MFMAs (the operands of stage h + 1 may still be in flight from LDS, so
-    // its slot stays untouched).
-    auto issue_upto = [&](int limit) {
-        if (limit > n_stages) limit = n_stages;
-        while (issued < limit) {
-            unsigned char* dst = lds + (issued % kRing) * kStageBytes;
-            const int64_t koff = static_cast<int64_t>(iss_k) * kBK;
-#pragma unroll
-            for (int j = 0; j < kWCopies; ++j)
-                __builtin_amdgcn_global_load_lds(wsrc[j] + koff, dst + (wave + 4 * j) * 1024, 16,
-                                                 0, 0);
-#pragma unroll
-            for (int j = 0; j < kHCopies; ++j)
-                __builtin_amdgcn_global_load_lds(hsrc[j] + koff,
-                                                 dst + kWBytes + (wave + 4 * j) * 1024, 16, 0, 0);
-            ++issued;
-            if (++iss_k == n_ksteps) {
-                iss_k = 0;
-                ++iss_vt;
-                point_w();
+    const __amdgpu_buffer_rsrc_t h_rs =
+        rows_rsrc(p.hidden + tok0 * p.ld_hidden, p.n_tokens - tok0, p.ld_hidden);
+    auto tile_rsrc = [&](int64_t vt) {
+        const bool more = vt < tile_end;
+        const int64_t v0 = (more ? vt : tile_first) * kBV;
+        return rows_rsrc(p.weight + v0 * p.ld_weight, more ? p.vocab - v0 : 0, p.ld_weight);
+    };
+    // The stages to be copied next, and their slots.
+    int64_t w_tile = tile_first;
+    int w_k = 0, w_slot = 0, h_k = 0, h_slot = 0;
+    __amdgpu_buffer_rsrc_t w_rs = tile_rsrc(w_tile);
+    typedef __attribute__((address_space(3))) void lds_void;
+    auto copy_w = [&](int j) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            w_rs, (lds_void*)(lds + w_slot * kSlotBytes + (wave + 4 * j) * 1024), 16, w_off,
+            j * w_step + w_k * kRowBytes, 0, 0);
+        if (j == kCopies - 1) {
+            if (++w_k == n_k) {
+                w_k = 0;
+                w_rs = tile_rsrc(++w_tile);
             }
+            w_slot = w_slot == kWSlots - 1 ? 0 : w_slot + 1;
+        }
+    };
+    auto copy_h = [&](int j) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            h_rs, (lds_void*)(lds + (kWSlots + h_slot) * kSlotBytes + (wave + 4 * j) * 1024), 16,
+            h_off, j * h_step + h_k * kRowBytes, 0, 0);
+        if (j == kCopies - 1) {
+            if (++h_k == n_k) h_k = 0;
+            h_slot ^= 1;
         }
     };
 
-    // Operands in two halves of the stage's K (16 columns each, one MFMA K
-    // step), ping-ponged: the MFMAs of one half run while the other half's
-    // operands are read from LDS.  Half 0 of the next stage is read under
-    // half 1's MFMAs, so a stage's first MFMAs find their operands in
-    // registers.  Two halves take the registers one whole stage did.
-    static_assert(kBK == 32, "two 16-column halves per stage");
-    bf16x8 ah[2][kVB], bh[2][kTB];
-    auto read_half = [&](auto half_tag, int stage) {
-        constexpr int H = decltype(half_tag)::value;
-        const unsigned char* wl = lds + (stage % kRing) * kStageBytes;
-        const unsigned char* hl = wl + kWBytes;
-        const int c = H * 2 + (lane >> 5);
-#pragma unroll
-        for (int a = 0; a < kVB; ++a)
-            ah[H][a] = *reinterpret_cast<const bf16x8*>(
-                wl + swz(wv * (kVB * 32) + a * 32 + (lane & 31), c));
-#pragma unroll
-        for (int b = 0; b < kTB; ++b)
-            bh[H][b] = *reinterpret_cast<const bf16x8*>(
-                hl + swz(wt * (kTB * 32) + b * 32 + (lane & 31), c));
+    // Operands.  Block i of a side is rows 16 i .. 16 i + 15 of the wave's
+    // half; lane l holds row l % 16, K columns 8 (l / 16) .. + 7 of the half
+    // stage's 32.
+    const int lrow = lane & 15;
+    const int lq = lane >> 4;
+    const int lf = swz_f(lrow);
+    int rw_slot = 0, rh_slot = 0;  // slots being read
+    auto w_src = [&](int half, int i) {
+        return *reinterpret_cast<const bf16x8*>(lds + rw_slot * kSlotBytes + wv * (kSlotBytes / 2) +
+                                                lrow * kRowBytes +
+                                                (((4 * half) ^ (lq ^ lf)) << 4) + i * 16 * kRowBytes);
     };
-    // Wait until stage `stage` has landed for this wave (at most the stages
-    // issued after it outstanding, up to kRing - 2 of them), then the barrier
-    // makes every wave's copies of it visible.
-    auto sync_stage = [&](int stage) {
-        wait_stages<kRing - 2>(issued - 1 - stage);
-        __builtin_amdgcn_s_barrier();
+    auto h_src = [&](int half, int i) {
+        return *reinterpret_cast<const bf16x8*>(lds + (kWSlots + rh_slot) * kSlotBytes +
+                                                wt * (kSlotBytes / 2) + lrow * kRowBytes +
+                                                (((4 * half) ^ (lq ^ lf)) << 4) + i * 16 * kRowBytes);
     };
-    constexpr int kReadsPerHalf = kVB + kTB;
-    constexpr int kMfmaPerHalf = kVB * kTB;
 
-    issue_upto(kRing);  // prologue: every slot is free
-    int g = 0;          // global stage index, runs across tiles
+    // The lane's 8 tokens: block b's is tok0 + wt * 128 + 16 b + l % 16.
+    const int64_t my_tok = tok0 + wt * kWaveSide + lrow;
+    Stat st[kBlocks];
+    int my_tgt[kBlocks];  // vocab and n_tokens are below 2^31
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+        st[b] = stat_empty();
+        const int64_t tok = my_tok + 16 * b;
+        const int64_t t = tok < p.n_tokens ? p.targets[tok] : -1;
+        my_tgt[b] = t >= 0 && t < p.vocab ? static_cast<int>(t) : -1;
+    }
+
+    // Prologue: stages 0 and 1.  The steady state's order of copies: hidden
+    // of stage g + 2 after the barrier in stage g, weight of stage g + 3 at
+    // the start of stage g + 1.
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) copy_w(j);
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) copy_h(j);
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) copy_w(j);
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) copy_h(j);
+    KLP_PIN();
+    __builtin_amdgcn_s_waitcnt(waitcnt(2 * kCopies, 15));
+    __builtin_amdgcn_s_barrier();
+    KLP_PIN();
+    // Half a stage ahead: all 8 blocks of the token side (two sets, in turn)
+    // and blocks 0..3 of the vocab side; its blocks 4..7 are read under the
+    // MFMAs of 0..3.
+    bf16x8 aw[kBlocks], bh[2][kBlocks];
+#pragma unroll
+    for (int i = 0; i < kBlocks; ++i) bh[0][i] = h_src(0, i);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) aw[i] = w_src(0, i);
+
     for (int64_t vt = tile_first; vt < tile_end; ++vt) {
-        f32x16 acc[kVB][kTB];
+        f32x4 acc[kBlocks][kBlocks];
+        // One stage: 2 x 64 MFMAs, its copies and operand reads placed
+        // between them by hand.
+        auto stage = [&](auto first_tag) {
+            constexpr bool kFirst = decltype(first_tag)::value;
 #pragma unroll
-        for (int a = 0; a < kVB; ++a)
+            for (int q = 0; q < 2; ++q) {
 #pragma unroll
-            for (int b = 0; b < kTB; ++b)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
-
-        auto mfma_half = [&](auto half_tag) {
-            constexpr int H = decltype(half_tag)::value;
-#pragma unroll
-            for (int a = 0; a < kVB; ++a)
-#pragma unroll
-                for (int b = 0; b < kTB; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[H][a], bh[H][b],
-                                                                        acc[a][b], 0, 0, 0);
-        };
-        // One read per MFMA for the first kReadsPerHalf MFMAs, then the rest.
-        auto interleave = [&]() {
-#pragma unroll
-            for (int i = 0; i < kReadsPerHalf; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one DS read
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, kMfmaPerHalf - kReadsPerHalf, 0);
-        };
-        using Half0 = std::integral_constant<int, 0>;
-        using Half1 = std::integral_constant<int, 1>;
-        // Stage g: half 0's MFMAs under half 1's reads; then, when stage g + 1
-        // belongs to this tile, sync on it, top up the ring and read its half
-        // 0 under half 1's MFMAs.
-        auto step = [&](auto prefetch_tag) {
-            constexpr bool kPrefetch = decltype(prefetch_tag)::value;
-            read_half(Half1{}, g);
-            mfma_half(Half0{});
-            interleave();
-            if constexpr (kPrefetch) {
-                sync_stage(g + 1);
-                // Stage g - 1's operand reads all completed before its MFMAs,
-                // which are behind this barrier; stage g's may still be in flight.
-                issue_upto(g + kRing);
-                read_half(Half0{}, g + 1);
-            }
-            mfma_half(Half1{});
-            if constexpr (kPrefetch) interleave();
-            ++g;
-        };
-
-        // The tile's first stage: its half 0.
-        sync_stage(g);
-        issue_upto(g + kRing);  // stage g - 1's MFMAs are behind the barrier
-        read_half(Half0{}, g);
-        for (int kk = 0; kk + 1 < n_ksteps; ++kk) step(std::true_type{});
-        // The tile's last stage reads nothing ahead: the pipeline drains at
-        // the tile's end, so no operands are live across the epilogue.
-        step(std::false_type{});
-
-        const int64_t v0 = vt * kBV;
-        if constexpr (kGrad) {
-            // d_logits of the tile: accumulator r of block (a, b) holds tile
-            // row wv*128 + a*32 + 8*(r/4) + 4*(lane/32) + r%4 of token column
-            // b*32 + lane%32; rows 4q .. 4q + 3 go out as one 8-byte store.
-            const int lrow0 = wv * (kVB * 32) + 4 * (lane >> 5);
-#pragma unroll
-            for (int b = 0; b < kTB; ++b) {
-                const int64_t tok = tok0 + wt * (kTB * 32) + b * 32 + (lane & 31);
-                if (tok >= p.n_tokens) continue;
-                uint16_t* drow = p.d_logits + tok * p.ld_d;
-#pragma unroll
-                for (int a = 0; a < kVB; ++a) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int64_t vq = v0 + lrow0 + a * 32 + 8 * q;
-                        if (vq >= p.vocab) continue;
-                        float d[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            float g = grad_one(acc[a][b][4 * q + i] * p.scale, rg[b]);
-                            if (vq + i == my_tgt[b]) g += rg[b].g_logp;
-                            if (vq + i >= p.vocab) g = 0.0f;
-                            d[i] = g * p.scale;
-                        }
-                        const bf16x2 lo = __builtin_convertvector(f32x2{d[0], d[1]}, bf16x2);
-                        const bf16x2 hi = __builtin_convertvector(f32x2{d[2], d[3]}, bf16x2);
-                        uint2 w;
-                        w.x = __builtin_bit_cast(uint32_t, lo);
-                        w.y = __builtin_bit_cast(uint32_t, hi);
-                        *reinterpret_cast<uint2*>(drow + vq) = w;
+                for (int i = 0; i < 64; ++i) {
+                    const int a = i >> 3, b = i & 7;
+                    if (q == 1 && i == 32) {
+                        // This wave has read all of the stage, and its copies of
+                        // the next one have landed (in flight, at most: the 8
+                        // weight copies after those).  After the barrier so for
+                        // every wave: the stage's slots are free, the next
+                        // stage's are full.
+                        KLP_PIN();
+                        __builtin_amdgcn_s_waitcnt(waitcnt(kCopies, 0));
+                        __builtin_amdgcn_s_barrier();
+                        KLP_PIN();
+                        rw_slot = rw_slot == kWSlots - 1 ? 0 : rw_slot + 1;
+                        rh_slot ^= 1;
                     }
+                    mfma_in_place(acc[a][b], aw[a], bh[q][b], kFirst && q == 0);
+                    if (i < 32) {
+                        if ((i & 7) == 3) aw[4 + a] = w_src(q, 4 + a);
+                        if (q == 0 && (i & 3) == 2) copy_w(i >> 2);
+                    } else {
+                        if ((i & 3) == 1) bh[q ^ 1][(i - 32) >> 2] = h_src(q ^ 1, (i - 32) >> 2);
+                        if ((i & 7) == 7) aw[a - 4] = w_src(q ^ 1, a - 4);
+                        if (q == 1 && (i & 3) == 2) copy_h((i - 32) >> 2);
+                    }
+                    KLP_PIN();
+                }
+            }
+        };
+        stage(std::true_type{});
+        for (int k = 1; k < n_k; ++k) stage(std::false_type{});
+        mfma_drain();
+        KLP_PIN();
+
+        // Accumulator r of block (a, b) holds tile row
+        // wv * 128 + 16 a + 4 (l / 16) + r of the lane's token b.
+        const int64_t v0 = vt * kBV;
+        const int row0 = wv * kWaveSide + 4 * lq;
+        const int64_t left = p.vocab - v0;
+        const int vlim = left < kBV ? static_cast<int>(left) : kBV;
+        if constexpr (kGrad) {
+            // d_logits of the tile; rows 4 l / 16 .. + 3 go out as one 8-byte
+            // store.
+            RowGrad rg[kBlocks];
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                const int64_t tok = my_tok + 16 * b;
+                const bool ok = tok < p.n_tokens;
+                rg[b] = ok ? row_grad(p.saved_lse[tok], p.saved_entropy[tok],
+                                      p.g_logp ? p.g_logp[tok] : 0.0f,
+                                      p.g_ent ? p.g_ent[tok] : 0.0f, p.g_lse ? p.g_lse[tok] : 0.0f)
+                           : row_grad(0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
+            }
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                const int64_t tok = my_tok + 16 * b;
+                if (tok >= p.n_tokens) continue;
+                uint16_t* drow = p.d_logits + tok * p.ld_d + v0 + row0;
+                const int target = my_tgt[b] - static_cast<int>(v0) - row0;
+#pragma unroll
+                for (int a = 0; a < kBlocks; ++a) {
+                    if (16 * a >= vlim - row0) continue;
+                    float d[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float v = acc_value(acc[a][b][i]);
+                        if (kScaled) v *= p.scale;
+                        float g = grad_one(v, rg[b]);
+                        if (16 * a + i == target) g += rg[b].g_logp;
+                        if (16 * a + i >= vlim - row0) g = 0.0f;
+                        d[i] = kScaled ? g * p.scale : g;
+                    }
+                    const bf16x2 lo = __builtin_convertvector(f32x2{d[0], d[1]}, bf16x2);
+                    const bf16x2 hi = __builtin_convertvector(f32x2{d[2], d[3]}, bf16x2);
+                    uint2 w;
+                    w.x = __builtin_bit_cast(uint32_t, lo);
+                    w.y = __builtin_bit_cast(uint32_t, hi);
+                    *reinterpret_cast<uint2*>(drow + 16 * a) = w;
+                    KLP_PIN();
                 }
             }
             continue;
         }
 
-        // Tile done: fold it into the lane's token states, one 32-row block
-        // at a time.  Accumulator r of block (a, b) holds tile row
-        // wv*128 + a*32 + 8*(r/4) + 4*(lane/32) + r%4 (vocab row v0 + that).
-        const int64_t vlim64 = p.vocab - v0;
-        const int vlim = vlim64 < kBV ? static_cast<int>(vlim64) : kBV;
-        const int lrow0 = wv * (kVB * 32) + 4 * (lane >> 5);
+        // Values 8 g .. 8 g + 7 of the lane's 32 of token b.
+        auto values = [&](int b, int g, float* x) {
 #pragma unroll
-        for (int b = 0; b < kTB; ++b) {
-            const int64_t trel64 = my_tgt[b] - v0;
-            const int trel = (trel64 >= 0 && trel64 < kBV) ? static_cast<int>(trel64) : -1;
+            for (int j = 0; j < 8; ++j) {
+                x[j] = acc_value(acc[2 * g + j / 4][b][j % 4]);
+                if (kScaled) x[j] *= p.scale;
+            }
+        };
+        // The target logits the lane holds: of every 16 rows from row0, 0..3.
+        const int first = static_cast<int>(v0) + row0;
 #pragma unroll
-            for (int a = 0; a < kVB; ++a) {
-                float x[16];
+        for (int b = 0; b < kBlocks; ++b) {
+            const int target = my_tgt[b] - first;
+            const bool mine = static_cast<uint32_t>(target) < static_cast<uint32_t>(kWaveSide) &&
+                              (target & 15) < 4;
+            if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
+            float xt = 0.0f;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = lrow0 + a * 32 + 8 * (r / 4) + (r % 4);
-                    const float val = acc[a][b][r] * p.scale;
-                    x[r] = (row < vlim) ? val : -INFINITY;
-                    if (row == trel) xt[b] = val;
+            for (int g = 0; g < 4; ++g) {
+                float x[8];
+                values(b, g, x);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (16 * (2 * g + j / 4) + j % 4 == target) xt = x[j];
+            }
+            if (mine) p.target_logit[my_tok + 16 * b] = xt;
+        }
+        if (vlim < kBV) {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                // Recomputed per token: the 32 lane masks of the comparisons
+                // below would otherwise be kept, and spilled.
+                int last = vlim - row0;
+                asm volatile("" : "+v"(last));
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    float x[8];
+                    values(b, g, x);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (16 * (2 * g + j / 4) + j % 4 >= last) x[j] = -INFINITY;
+                    absorb<8, true>(st[b], x);
+                    KLP_PIN();
                 }
-                absorb<16, true>(st[b], x);
+            }
+        } else {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                const Stat before = st[b];
+                float x[32];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) values(b, g, x + 8 * g);
+                absorb<32, false>(st[b], x);
+                KLP_PIN();
+                if (needs_clamped_rescan(st[b])) {  // a -inf logit
+                    st[b] = before;
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        values(b, g, x);
+                        absorb<8, true>(st[b], x);
+                    }
+                }
             }
         }
     }
 
     if constexpr (kGrad) return;
 
-    // Merge lane l with lane l + 32 (same token, other vocab rows), then the
-    // two vocab-half waves of each token half through LDS (the ring's memory:
-    // every wave is past its last read of it once all reach the barrier).
+    // Merge the four lanes of each token (vocab rows 4 apart), then the two
+    // vocab-half waves of each token half through LDS (the rings' memory:
+    // every wave is past its last read of it, and past its last copy into
+    // it, once all reach the barrier).
+    __builtin_amdgcn_s_waitcnt(waitcnt(0, 15));
     __syncthreads();
     Stat (*merge_stat)[kBT] = reinterpret_cast<Stat (*)[kBT]>(lds);
-    float (*merge_xt)[kBT] = reinterpret_cast<float (*)[kBT]>(lds + 2 * kBT * sizeof(Stat));
 #pragma unroll
-    for (int b = 0; b < kTB; ++b) {
-        Stat o;
-        o.m = __shfl_xor(st[b].m, 32, 64);
-        o.z = __shfl_xor(st[b].z, 32, 64);
-        o.t = __shfl_xor(st[b].t, 32, 64);
-        const float oxt = __shfl_xor(xt[b], 32, 64);
-        st[b] = (lane < 32) ? combine(st[b], o) : combine(o, st[b]);
-        xt[b] += oxt;  // at most one of the two is non-zero
-        if (lane < 32) {
-            const int col = wt * (kTB * 32) + b * 32 + lane;
-            merge_stat[wv][col] = st[b];
-            merge_xt[wv][col] = xt[b];
-        }
+    for (int b = 0; b < kBlocks; ++b) {
+        st[b] = combine(st[b], stat_shfl_xor(st[b], 16));
+        st[b] = combine(st[b], stat_shfl_xor(st[b], 32));
+        if (lane < 16) merge_stat[wv][wt * kWaveSide + 16 * b + lane] = st[b];
     }
     __syncthreads();
-    if (tid < kBT) {
-        const int64_t n = tok0 + tid;
-        if (n < p.n_tokens) {
-            const Stat s = combine(merge_stat[0][tid], merge_stat[1][tid]);
-            float4* slot = reinterpret_cast<float4*>(p.partials) + chunk * p.n_tokens + n;
-            *slot = make_float4(s.m, s.z, s.t, merge_xt[0][tid] + merge_xt[1][tid]);
-        }
+    const int64_t n = tok0 + tid;
+    if (n < p.n_tokens) {
+        const Stat s = combine(merge_stat[0][tid], merge_stat[1][tid]);
+        float4* slot = reinterpret_cast<float4*>(p.partials) + chunk * p.n_tokens + n;
+        *slot = make_float4(s.m, s.z, s.t, 0.0f);
     }
 }
+#undef KLP_PIN
 
 // One wave per token: lane l merges chunks l, l + 64, l + 128, ... in order,
 // the lanes then merge in the fixed xor-butterfly order of wave_reduce (so the
-// result does not depend on timing), and lane 0 takes the target logit from
-// the chunk that holds the target.
+// result does not depend on timing), and lane 0 takes the target logit, which
+// the lane that met it left in the workspace.
 __global__ __launch_bounds__(256) void klp_lmh_combine_kernel(LmhParams p) {
     const int64_t n = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -421,10 +453,7 @@ __global__ __launch_bounds__(256) void klp_lmh_combine_kernel(LmhParams p) {
     if (lane != 0) return;
     const int64_t tgt = p.targets[n];
     float x_target = 0.0f;
-    if (tgt >= 0 && tgt < p.vocab) {
-        const int64_t c = tgt / (static_cast<int64_t>(p.tiles_per_chunk) * kBV);
-        x_target = part[c * p.n_tokens + n].w;
-    }
+    if (tgt >= 0 && tgt < p.vocab) x_target = p.target_logit[n];
     const RowOut o = finalize(acc, x_target);
     p.logprob[n] = o.logp;
     p.entropy[n] = o.ent;
@@ -436,7 +465,7 @@ int64_t lmh_vocab_tiles(int64_t vocab) { return (vocab + kBV - 1) / kBV; }
 
 hipError_t launch_lmh_dlogits(const LmhParams& p, hipStream_t stream) {
     const int64_t chunks8 = (p.n_chunks + 7) / 8 * 8;
-    return launch_kernel(klp_lmh_kernel<true>,
+    return launch_kernel(p.scale != 1.0f ? klp_lmh_kernel<true, true> : klp_lmh_kernel<true, false>,
                          dim3(static_cast<unsigned>(chunks8 * p.n_tblocks)), dim3(kThreads),
                          stream, p);
 }
@@ -446,8 +475,9 @@ hipError_t launch_lmh_fwd(const LmhParams& p, hipStream_t stream) {
     // padding workgroups exit at once.
     const int64_t chunks8 = (p.n_chunks + 7) / 8 * 8;
     const int64_t blocks = chunks8 * p.n_tblocks;
-    hipError_t e = launch_kernel(klp_lmh_kernel<false>, dim3(static_cast<unsigned>(blocks)),
-                                 dim3(kThreads), stream, p);
+    hipError_t e =
+        launch_kernel(p.scale != 1.0f ? klp_lmh_kernel<false, true> : klp_lmh_kernel<false, false>,
+                      dim3(static_cast<unsigned>(blocks)), dim3(kThreads), stream, p);
     if (e != hipSuccess) return e;
     return launch_kernel(klp_lmh_combine_kernel,
                          dim3(static_cast<unsigned>((p.n_tokens + 3) / 4)), dim3(256), stream, p);

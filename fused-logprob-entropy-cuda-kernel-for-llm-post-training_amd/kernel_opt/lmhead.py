@@ -115,6 +115,12 @@ def _ld(t: torch.Tensor) -> int:
     return t.stride(0) if t.size(0) > 1 else t.size(1)
 
 
+def _rows_32bit(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or its contiguous copy where the MFMA kernels' 32-bit offsets
+    within 256 rows would not reach (row strides above 4194303 elements)."""
+    return t if _ld(t) <= (2 ** 31 - 1) // 512 else t.contiguous()
+
+
 # Vocabulary chunk of the chunked head.  Small batches (a chunk of
 # CHUNK_COLS_WIDE columns within CHUNK_WIDE_MAX_BYTES: up to 1024 bf16 tokens)
 # take chunks of CHUNK_COLS_WIDE columns, the last one holding the rest.
@@ -217,6 +223,8 @@ def _backward_chunked(h2, weight, t, T, plan, lse, ent, gl, ge, gs, need_h, need
     dw = torch.empty(V, D, dtype=weight.dtype, device=dev) if need_w else None
     cols = max(n for _, n in plan)
     d_buf = torch.empty(N * (-(-cols // 4) * 4), dtype=weight.dtype, device=dev)
+    if impl == "mfma":
+        h2, weight = _rows_32bit(h2), _rows_32bit(weight)
     lg_buf = torch.empty(N * cols, dtype=h2.dtype, device=dev) if impl == "chunked" else None
     with device_guard(dev.index):
         stream = stream_handle(dev.index)
@@ -328,6 +336,7 @@ def fused_linear_logprob_entropy_forward(hidden: torch.Tensor, weight: torch.Ten
                          out)
         return tuple(out)
     dev = hidden.device
+    h2, weight = _rows_32bit(h2), _rows_32bit(weight)
     with device_guard(dev.index):
         stream = stream_handle(dev.index)
         ws = _workspace(dev, stream, lib.klp_lmh_workspace_bytes(N, V, D))

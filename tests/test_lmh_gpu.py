@@ -67,6 +67,37 @@ def test_matches_oracle(N, V, D):
     check(h, w, t, label=f"{N}x{V}x{D}")
 
 
+@pytest.mark.parametrize("N,V,D", [(256, 256, 64), (255, 257, 64), (257, 255, 128),
+                                   (512, 513, 192), (16, 4096, 64), (300, 70000, 64)])
+def test_tile_and_ring_edges(N, V, D):
+    """Token blocks, vocab tiles and K stages at and around their sizes (256,
+    256 and 64 columns: fewer stages than the rings hold up to several tiles
+    a workgroup), with every row of a tile as some token's target."""
+    h, w, t = make(N, V, D, seed=31 + N + V + D)
+    t = torch.arange(N) * max(1, (V + 255) // 256) % V
+    for temperature in (None, 0.7):
+        check(h, w, t, temperature, label=f"{N}x{V}x{D}")
+
+
+def test_negative_infinite_logits():
+    """Logits of -inf (a weight row with -inf against positive hidden values)
+    drop out of their rows, in full tiles and in the one at the end."""
+    from kernel_opt import fused_linear_logprob_entropy_forward
+    N, V, D = 70, 1000, 64
+    h, w, t = make(N, V, D, seed=33)
+    h[:, 0] = 1.0
+    w[::5, 0] = float("-inf")
+    t = torch.where(t % 5 == 0, t + 1, t)
+    x = (h.double() @ w.double().T)
+    lse = torch.logsumexp(x, 1)
+    p = (x - lse[:, None]).exp()
+    ent = lse - (p * torch.where(torch.isinf(x), torch.zeros_like(x), x)).sum(1)
+    outs = fused_linear_logprob_entropy_forward(h.to(DEV), w.to(DEV), t.to(DEV), impl="mfma")
+    # fp32 sums of 64 products of magnitude up to ~10, as check() bounds them
+    for o, r in zip(outs, (x.gather(1, t[:, None]).squeeze(1) - lse, ent, lse)):
+        assert (o.cpu().double() - r).abs().max() <= 5e-5
+
+
 def test_headline_vocab_and_hidden():
     """Qwen2.5-7B's head: V = 152064, D = 3584, with 300 tokens."""
     h, w, t = make(300, 152064, 3584, seed=7, spike=True)

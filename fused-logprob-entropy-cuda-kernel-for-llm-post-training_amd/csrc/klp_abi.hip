@@ -519,6 +519,65 @@ size_t lmh_workspace_bytes(int64_t n_tokens, int64_t vocab) {
     return lmh_partials_bytes(n_tokens, nc) + static_cast<size_t>(n_tokens) * sizeof(float);
 }
 
+// The LM head's backward products: 256 x 256 tiles, one workgroup per CU.
+constexpr int64_t kHeadTile = 256;
+constexpr int64_t kHeadBK = 64;
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// d_hidden: the K range of one split.  Time in stages of 64 columns (about
+// 1.3 us): rounds of workgroups times a split's stages, about 10 stages a
+// round for filling the rings and storing the tile, and the slabs' write and
+// read at about 5 TB/s.
+int64_t head_dhidden_k_per_split(int64_t n_tokens, int64_t k, int64_t dim) {
+    const int64_t tiles = ceil_div(n_tokens, kHeadTile) * ceil_div(dim, kHeadTile);
+    const int64_t stages = ceil_div(k, kHeadBK);
+    int64_t best = stages, best_cost = INT64_MAX;
+    for (int64_t s = 1; s <= 64 && s <= stages; ++s) {
+        const int64_t per = ceil_div(stages, s);
+        const int64_t splits = ceil_div(stages, per);
+        const int64_t rounds = ceil_div(ceil_div(tiles * splits, 8) * 8, klp::kHeadGemmCus);
+        const int64_t slab = splits * n_tokens * dim / 812500;  // * 8 bytes / 6.5 MB a stage
+        const int64_t cost = rounds * (per + 10) + slab;
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = per;
+        }
+    }
+    return best * kHeadBK;
+}
+
+size_t head_dhidden_workspace_bytes(int64_t n_tokens, int64_t k, int64_t dim) {
+    if (n_tokens <= 0 || k <= 0 || dim <= 0) return 0;
+    const int64_t splits = ceil_div(k, head_dhidden_k_per_split(n_tokens, k, dim));
+    return static_cast<size_t>(splits) * static_cast<size_t>(n_tokens) *
+           static_cast<size_t>(dim) * sizeof(float);
+}
+
+// Checks shared by the two products: sizes, strides, alignment.
+int head_gemm_check(int dtype, const void* d_logits, int64_t ld_d, int64_t n_tokens,
+                    int64_t vocab, const void* other, int64_t ld_other, int64_t dim) {
+    if (dtype != KLP_BF16 && dtype != KLP_FP16)
+        return fail(KLP_EDTYPE, "dtype must be bf16 or fp16");
+    if (n_tokens < 0 || vocab < 1) return fail(KLP_EINVAL, "n_tokens must be >= 0 and vocab >= 1");
+    if (dim < 64 || dim % 64 != 0)
+        return fail(KLP_EINVAL, "dim must be a positive multiple of 64, got %lld",
+                    static_cast<long long>(dim));
+    if (ld_d < ceil_div(vocab, 8) * 8 || ld_other < dim || ld_d % 8 != 0 || ld_other % 8 != 0)
+        return fail(KLP_EINVAL,
+                    "row strides must be multiples of 8 elements, at least dim and vocab rounded "
+                    "up to 8");
+    if (ld_d > INT32_MAX / 512 || ld_other > INT32_MAX / 512)
+        return fail(KLP_EINVAL, "row strides above %d elements are not supported",
+                    INT32_MAX / 512);
+    if (n_tokens > INT32_MAX / 2 || vocab > INT32_MAX / 2 || dim > INT32_MAX / 2)
+        return fail(KLP_EINVAL, "n_tokens, vocab and dim must be below 2^30");
+    if (n_tokens == 0) return KLP_OK;
+    if (d_logits == nullptr || other == nullptr || !aligned(d_logits, 16) || !aligned(other, 16))
+        return fail(KLP_EINVAL, "operands must be non-null and 16-byte aligned");
+    return KLP_OK;
+}
+
 int ceiling_impl(int mode, const void* src, void* dst, int64_t n_rows, int64_t row_bytes,
                  int waves, int unroll, int splits, uint32_t* sink, uint32_t magic,
                  void* stream) {
@@ -1110,11 +1169,14 @@ int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
     return KLP_OK;
 }
 
-int klp_lmh_bwd_logits(const void* hidden, int64_t ld_hidden, const void* weight,
-                       int64_t ld_weight, int64_t n_tokens, int64_t vocab, int64_t dim,
-                       const int64_t* targets, float temperature, const float* lse,
-                       const float* entropy, const float* g_logp, const float* g_ent,
-                       const float* g_lse, void* d_logits, int64_t ld_d, void* stream) {
+// klp_lmh_bwd_logits and klp_lmh_bwd_logits_as.  `pad`: columns are written
+// up to vocab rounded up to it.
+static int lmh_bwd_impl(int dtype, bool rounded, const void* hidden, int64_t ld_hidden,
+                        const void* weight, int64_t ld_weight, int64_t n_tokens, int64_t vocab,
+                        int64_t dim, const int64_t* targets, int64_t vocab_offset,
+                        float temperature, const float* lse, const float* entropy,
+                        const float* g_logp, const float* g_ent, const float* g_lse,
+                        void* d_logits, int64_t ld_d, int64_t pad, void* stream) {
     klp::LmhParams p;
     int rc = lmh_setup(hidden, ld_hidden, weight, ld_weight, n_tokens, vocab, dim, targets,
                        temperature, &p);
@@ -1125,26 +1187,172 @@ int klp_lmh_bwd_logits(const void* hidden, int64_t ld_hidden, const void* weight
     if (g_logp && (rc = check_f32(g_logp, "g_logp")) != KLP_OK) return rc;
     if (g_ent && (rc = check_f32(g_ent, "g_ent")) != KLP_OK) return rc;
     if (g_lse && (rc = check_f32(g_lse, "g_lse")) != KLP_OK) return rc;
-    if (d_logits == nullptr || !aligned(d_logits, 8) || ld_d < vocab || ld_d % 4 != 0)
-        return fail(KLP_EINVAL,
-                    "d_logits must be non-null and 8-byte aligned, with a row stride >= vocab "
-                    "and a multiple of 4 elements");
+    p.target_offset = vocab_offset;
     p.saved_lse = lse;
     p.saved_entropy = entropy;
     p.g_logp = g_logp;
     p.g_ent = g_ent;
     p.g_lse = g_lse;
-    p.d_logits = static_cast<uint16_t*>(d_logits);
-    p.ld_d = ld_d;
+    p.out = static_cast<uint16_t*>(d_logits);
+    p.ld_out = ld_d;
+    p.n_out = ceil_div(vocab, pad) * pad;
+    p.out_align = ld_d % 8 == 0 && aligned(d_logits, 16) ? 16 : 8;
     if (injected_failure("lm-head backward")) return KLP_ELAUNCH;
-    return after_launch(klp::launch_lmh_dlogits(p, static_cast<hipStream_t>(stream)),
-                        "lm-head backward");
+    return after_launch(
+        klp::launch_lmh_dlogits(dtype, rounded, p, static_cast<hipStream_t>(stream)),
+        "lm-head backward");
 }
 
-int klp_lmh_fwd(const void* hidden, int64_t ld_hidden, const void* weight, int64_t ld_weight,
-                int64_t n_tokens, int64_t vocab, int64_t dim, const int64_t* targets,
-                float temperature, float* logprob, float* entropy, float* lse, void* workspace,
-                size_t workspace_bytes, void* stream) {
+int klp_lmh_bwd_logits(const void* hidden, int64_t ld_hidden, const void* weight,
+                       int64_t ld_weight, int64_t n_tokens, int64_t vocab, int64_t dim,
+                       const int64_t* targets, float temperature, const float* lse,
+                       const float* entropy, const float* g_logp, const float* g_ent,
+                       const float* g_lse, void* d_logits, int64_t ld_d, void* stream) {
+    if (n_tokens > 0 && (d_logits == nullptr || !aligned(d_logits, 8) || ld_d < vocab || ld_d % 4 != 0))
+        return fail(KLP_EINVAL,
+                    "d_logits must be non-null and 8-byte aligned, with a row stride >= vocab "
+                    "and a multiple of 4 elements");
+    return lmh_bwd_impl(KLP_BF16, false, hidden, ld_hidden, weight, ld_weight, n_tokens, vocab,
+                        dim, targets, 0, temperature, lse, entropy, g_logp, g_ent, g_lse, d_logits,
+                        ld_d, 4, stream);
+}
+
+static int lmh_as_check(int dtype, int rounded) {
+    if (dtype != KLP_BF16 && !(dtype == KLP_FP16 && rounded))
+        return fail(KLP_EDTYPE, "dtype must be bf16, or fp16 with rounded logits");
+    return KLP_OK;
+}
+
+int klp_lmh_bwd_logits_as(int dtype, int rounded, const void* hidden, int64_t ld_hidden,
+                          const void* weight, int64_t ld_weight, int64_t n_tokens, int64_t vocab,
+                          int64_t dim, const int64_t* targets, int64_t vocab_offset,
+                          float temperature, const float* lse, const float* entropy,
+                          const float* g_logp, const float* g_ent, const float* g_lse,
+                          void* d_logits, int64_t ld_d, void* stream) {
+    int rc = lmh_as_check(dtype, rounded);
+    if (rc != KLP_OK) return rc;
+    if (vocab_offset < 0) return fail(KLP_EINVAL, "vocab_offset must be >= 0");
+    if (n_tokens > 0 && (d_logits == nullptr || !aligned(d_logits, 16) || ld_d % 8 != 0 ||
+                         ld_d < ceil_div(vocab, 8) * 8))
+        return fail(KLP_EINVAL,
+                    "d_logits must be non-null and 16-byte aligned, with a row stride that is a "
+                    "multiple of 8 elements and holds vocab rounded up to 8");
+    return lmh_bwd_impl(dtype, rounded != 0, hidden, ld_hidden, weight, ld_weight, n_tokens, vocab,
+                        dim, targets, vocab_offset, temperature, lse, entropy, g_logp, g_ent,
+                        g_lse, d_logits, ld_d, 8, stream);
+}
+
+int klp_lmh_logits(int dtype, const void* hidden, int64_t ld_hidden, const void* weight,
+                   int64_t ld_weight, int64_t n_tokens, int64_t vocab, int64_t dim, void* logits,
+                   int64_t ld_logits, void* stream) {
+    int rc = lmh_as_check(dtype, 1);
+    if (rc != KLP_OK) return rc;
+    klp::LmhParams p;
+    static const int64_t no_targets = 0;  // not read
+    rc = lmh_setup(hidden, ld_hidden, weight, ld_weight, n_tokens, vocab, dim, &no_targets, 1.0f,
+                   &p);
+    if (rc != KLP_OK) return rc;
+    if (n_tokens == 0) return ok();
+    p.targets = nullptr;
+    if (logits == nullptr || !aligned(logits, 2) || ld_logits < vocab)
+        return fail(KLP_EINVAL, "logits must be non-null, aligned to their elements, with a row "
+                                "stride >= vocab");
+    p.out = static_cast<uint16_t*>(logits);
+    p.ld_out = ld_logits;
+    p.n_out = vocab;
+    p.out_align = ld_logits % 8 == 0 && aligned(logits, 16) ? 16 : 2;
+    if (injected_failure("lm-head logits")) return KLP_ELAUNCH;
+    return after_launch(klp::launch_lmh_logits(dtype, p, static_cast<hipStream_t>(stream)),
+                        "lm-head logits");
+}
+
+size_t klp_head_dhidden_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t dim) {
+    return head_dhidden_workspace_bytes(n_tokens, vocab, dim);
+}
+
+int klp_head_dweight(int dtype, const void* d_logits, int64_t ld_d, int64_t n_tokens,
+                     int64_t vocab, const void* hidden, int64_t ld_hidden, int64_t dim,
+                     void* d_weight, int64_t ld_out, void* stream) {
+    int rc = head_gemm_check(dtype, d_logits, ld_d, n_tokens, vocab, hidden, ld_hidden, dim);
+    if (rc != KLP_OK) return rc;
+    if (n_tokens == 0) return fail(KLP_EINVAL, "n_tokens must be >= 1");
+    if (d_weight == nullptr || !aligned(d_weight, 16) || ld_out < dim || ld_out % 8 != 0)
+        return fail(KLP_EINVAL,
+                    "d_weight must be non-null and 16-byte aligned, with a row stride >= dim and "
+                    "a multiple of 8 elements");
+    klp::HeadGemmParams p{};
+    p.a = static_cast<const uint16_t*>(hidden);
+    p.ld_a = ld_hidden;
+    p.b = static_cast<const uint16_t*>(d_logits);
+    p.ld_b = ld_d;
+    p.m = dim;
+    p.n = vocab;
+    p.k = n_tokens;
+    p.m_tiles = ceil_div(dim, kHeadTile);
+    p.n_tiles = ceil_div(vocab, kHeadTile);
+    p.k_per_split = ceil_div(n_tokens, kHeadBK) * kHeadBK;
+    p.n_items = p.m_tiles * p.n_tiles;
+    p.group = p.n_tiles < klp::kHeadGemmGroup ? p.n_tiles : klp::kHeadGemmGroup;
+    p.out = static_cast<uint16_t*>(d_weight);
+    p.ld_out = ld_out;
+    if (p.n_items > INT32_MAX / 2) return fail(KLP_EINVAL, "too many output tiles");
+    if (injected_failure("lm-head d_weight")) return KLP_ELAUNCH;
+    return after_launch(klp::launch_head_gemm(dtype, p, static_cast<hipStream_t>(stream)),
+                        "lm-head d_weight");
+}
+
+int klp_head_dhidden(int dtype, const void* d_logits, int64_t ld_d, int64_t n_tokens,
+                     int64_t vocab, const void* weight, int64_t ld_weight, int64_t dim,
+                     float* acc, int accumulate, void* d_hidden, void* workspace,
+                     size_t workspace_bytes, void* stream) {
+    int rc = head_gemm_check(dtype, d_logits, ld_d, n_tokens, vocab, weight, ld_weight, dim);
+    if (rc != KLP_OK) return rc;
+    if (n_tokens == 0) return ok();
+    if ((accumulate || d_hidden == nullptr) && (acc == nullptr || !aligned(acc, 16)))
+        return fail(KLP_EINVAL, "acc must be non-null and 16-byte aligned");
+    if (d_hidden != nullptr && !aligned(d_hidden, 16))
+        return fail(KLP_EINVAL, "d_hidden must be 16-byte aligned");
+    const size_t need = head_dhidden_workspace_bytes(n_tokens, vocab, dim);
+    if (workspace == nullptr || workspace_bytes < need || !aligned(workspace, 16))
+        return fail(KLP_EWORKSPACE,
+                    "workspace missing, too small or not 16-byte aligned: have %zu bytes, need %zu",
+                    workspace_bytes, need);
+    klp::HeadGemmParams p{};
+    p.a = static_cast<const uint16_t*>(weight);
+    p.ld_a = ld_weight;
+    p.b = static_cast<const uint16_t*>(d_logits);
+    p.ld_b = ld_d;
+    p.m = dim;
+    p.n = n_tokens;
+    p.k = vocab;
+    p.m_tiles = ceil_div(dim, kHeadTile);
+    p.n_tiles = ceil_div(n_tokens, kHeadTile);
+    p.k_per_split = head_dhidden_k_per_split(n_tokens, vocab, dim);
+    const int64_t splits = ceil_div(vocab, p.k_per_split);
+    p.n_items = p.m_tiles * p.n_tiles * splits;
+    p.group = p.n_tiles < klp::kHeadGemmGroup ? p.n_tiles : klp::kHeadGemmGroup;
+    p.slabs = static_cast<float*>(workspace);
+    if (p.n_items > INT32_MAX / 2) return fail(KLP_EINVAL, "too many output tiles");
+    if (injected_failure("lm-head d_hidden")) return KLP_ELAUNCH;
+    rc = after_launch(klp::launch_head_gemm(dtype, p, static_cast<hipStream_t>(stream)),
+                      "lm-head d_hidden");
+    if (rc != KLP_OK) return rc;
+    klp::HeadSumParams q{};
+    q.slabs = p.slabs;
+    q.n_slabs = static_cast<int>(splits);
+    q.accumulate = accumulate != 0;
+    q.n_vec = n_tokens * dim / 4;
+    q.acc = acc;
+    q.out = static_cast<uint16_t*>(d_hidden);
+    return after_launch(klp::launch_head_sum(dtype, q, static_cast<hipStream_t>(stream)),
+                        "lm-head d_hidden sum");
+}
+
+static int lmh_fwd_impl(int dtype, bool rounded, const void* hidden, int64_t ld_hidden,
+                        const void* weight, int64_t ld_weight, int64_t n_tokens, int64_t vocab,
+                        int64_t dim, const int64_t* targets, float temperature, float* logprob,
+                        float* entropy, float* lse, void* workspace, size_t workspace_bytes,
+                        void* stream) {
     klp::LmhParams p;
     int rc = lmh_setup(hidden, ld_hidden, weight, ld_weight, n_tokens, vocab, dim, targets,
                        temperature, &p);
@@ -1165,8 +1373,29 @@ int klp_lmh_fwd(const void* hidden, int64_t ld_hidden, const void* weight, int64
     p.entropy = entropy;
     p.lse = lse;
     if (injected_failure("lm-head forward")) return KLP_ELAUNCH;
-    return after_launch(klp::launch_lmh_fwd(p, static_cast<hipStream_t>(stream)),
+    return after_launch(klp::launch_lmh_fwd(dtype, rounded, p, static_cast<hipStream_t>(stream)),
                         "lm-head forward");
+}
+
+int klp_lmh_fwd(const void* hidden, int64_t ld_hidden, const void* weight, int64_t ld_weight,
+                int64_t n_tokens, int64_t vocab, int64_t dim, const int64_t* targets,
+                float temperature, float* logprob, float* entropy, float* lse, void* workspace,
+                size_t workspace_bytes, void* stream) {
+    return lmh_fwd_impl(KLP_BF16, false, hidden, ld_hidden, weight, ld_weight, n_tokens, vocab,
+                        dim, targets, temperature, logprob, entropy, lse, workspace,
+                        workspace_bytes, stream);
+}
+
+int klp_lmh_fwd_as(int dtype, int rounded, const void* hidden, int64_t ld_hidden,
+                   const void* weight, int64_t ld_weight, int64_t n_tokens, int64_t vocab,
+                   int64_t dim, const int64_t* targets, float temperature, float* logprob,
+                   float* entropy, float* lse, void* workspace, size_t workspace_bytes,
+                   void* stream) {
+    const int rc = lmh_as_check(dtype, rounded);
+    if (rc != KLP_OK) return rc;
+    return lmh_fwd_impl(dtype, rounded != 0, hidden, ld_hidden, weight, ld_weight, n_tokens, vocab,
+                        dim, targets, temperature, logprob, entropy, lse, workspace,
+                        workspace_bytes, stream);
 }
 
 int klp_ceiling_read(const void* src, int64_t n_rows, int64_t row_bytes, int waves, int unroll,

@@ -203,16 +203,17 @@ struct ScaleParams {
 
 hipError_t launch_scale(int dtype, const ScaleParams& p, hipStream_t stream);
 
-// Fused LM head forward (klp_lmhead.hip).
+// Fused LM head (klp_lmhead.hip).
 struct LmhParams {
-    const uint16_t* hidden;  // bf16 [n_tokens, ld_hidden], first `dim` columns used
+    const uint16_t* hidden;  // [n_tokens, ld_hidden], first `dim` columns used
     int64_t ld_hidden;
-    const uint16_t* weight;  // bf16 [vocab, ld_weight]
+    const uint16_t* weight;  // [vocab, ld_weight]
     int64_t ld_weight;
     int64_t n_tokens;
     int64_t vocab;
     int64_t dim;             // K, a multiple of 64
-    const int64_t* targets;  // [n_tokens]
+    const int64_t* targets;  // [n_tokens]; row targets[n] - target_offset of the weight
+    int64_t target_offset;
     float scale;             // 1 / temperature
     float* partials;         // [n_chunks, n_tokens] float4 (m, z, t, unused)
     float* target_logit;     // [n_tokens], behind the partials; written where a target is valid
@@ -229,13 +230,53 @@ struct LmhParams {
     const float* g_lse;      // nullable
     const float* saved_lse;  // [n_tokens], as the forward wrote it
     const float* saved_entropy;
-    uint16_t* d_logits;      // bf16 [n_tokens, ld_d], ld_d a multiple of 4
-    int64_t ld_d;
+    // d_logits and logits: [n_tokens, ld_out], columns vocab .. n_out - 1
+    // written with zeros; out_align: alignment of every row, 16, 8 or 2 bytes.
+    uint16_t* out;
+    int64_t ld_out;
+    int64_t n_out;
+    int out_align;
 };
 int64_t lmh_token_blocks(int64_t n_tokens);
 int64_t lmh_vocab_tiles(int64_t vocab);
-hipError_t launch_lmh_fwd(const LmhParams& p, hipStream_t stream);
-hipError_t launch_lmh_dlogits(const LmhParams& p, hipStream_t stream);
+// `rounded`: logits rounded once to `dtype` (bf16 or fp16); otherwise bf16
+// operands and float32 logits.
+hipError_t launch_lmh_fwd(int dtype, bool rounded, const LmhParams& p, hipStream_t stream);
+hipError_t launch_lmh_dlogits(int dtype, bool rounded, const LmhParams& p, hipStream_t stream);
+hipError_t launch_lmh_logits(int dtype, const LmhParams& p, hipStream_t stream);
+
+// The LM head's backward products (klp_head_gemm.hip): out[n, m] (or, with
+// `slabs`, float32 slab[split][n, m]) = sum_k a[k, m] * b, b = b[k, n] for
+// 16-bit output and b[n, k] for slabs.  16-bit a, b; strides in elements,
+// multiples of 8; m a multiple of 64; K-contiguous b: k a multiple of 8.
+struct HeadGemmParams {
+    const uint16_t* a;
+    int64_t ld_a;
+    const uint16_t* b;
+    int64_t ld_b;
+    int64_t m, n, k;
+    int64_t m_tiles, n_tiles;  // of 256
+    int64_t k_per_split;       // a multiple of 64 (k without splits)
+    int64_t n_items;           // m_tiles * n_tiles * splits
+    int64_t group;             // row blocks taken together
+    uint16_t* out;             // [n, ld_out]
+    int64_t ld_out;
+    float* slabs;              // [splits][n][m], nullable
+};
+struct HeadSumParams {
+    const float* slabs;
+    int n_slabs;
+    int accumulate;            // add to acc
+    int64_t n_vec;             // n * m / 4
+    float* acc;                // float32 result, and addend with `accumulate`
+    uint16_t* out;             // 16-bit result instead, nullable
+};
+// Workgroups at once: one per CU.
+constexpr int64_t kHeadGemmCus = 256;
+// Row blocks taken together, at most: 6 x 5 tiles are an XCD's 32 at a time.
+constexpr int64_t kHeadGemmGroup = 6;
+hipError_t launch_head_gemm(int dtype, const HeadGemmParams& p, hipStream_t stream);
+hipError_t launch_head_sum(int dtype, const HeadSumParams& p, hipStream_t stream);
 
 // Calibration kernels (klp_ceiling.hip): rows of `row_bytes` (a multiple of
 // 16) at `src` (and `dst`), 16-byte aligned and contiguous; `splits`

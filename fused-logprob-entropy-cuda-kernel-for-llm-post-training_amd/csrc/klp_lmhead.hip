@@ -6,10 +6,10 @@
 //   logits[n, v] = scale * sum_k hidden[n, k] * weight[v, k]      (fp32)
 //   logprob[n] = logits[n, t_n] - lse[n],  entropy[n], lse[n]  as klp_fwd
 //
-// without writing the [N, V] logits anywhere.  hidden is bf16 [N, D] and
-// weight bf16 [V, D] (nn.Linear's layout), both K-contiguous.
+// without writing the [N, V] logits anywhere.  hidden is [N, D] and
+// weight [V, D], bf16 or fp16 (nn.Linear's layout), both K-contiguous.
 //
-// klp_lmh_kernel<false, ..> (forward): one workgroup (4 waves, 2 x 2) per (token block of
+// klp_lmh_kernel, forward (kFold): one workgroup (4 waves, 2 x 2) per (token block of
 // 256, vocab chunk of `tiles_per_chunk` tiles of 256 rows).  Per vocab tile
 // it computes the 256 x 256 block of logits^T with v_mfma_f32_16x16x32_bf16,
 // each wave a 128 x 128 part of it (64 accumulator blocks, 256 AGPRs):
@@ -30,7 +30,7 @@
 //    the copies go through a descriptor of length 0, which keeps the count
 //    of copies in flight, and with it the vmcnt waits, the same on every path;
 //  - LDS rows are 128 bytes; the 16-byte chunk index is XOR-swizzled with
-//    row bits 0..3 (swz_f) so that the MFMA operand reads are free of bank
+//    row bits 1..3 (swz) so that the MFMA operand reads are free of bank
 //    conflicts;
 //  - operands are read one half stage (32 columns) ahead, two ds_reads per
 //    8 MFMAs in source order, and each copy has a slot between two MFMAs;
@@ -44,8 +44,8 @@
 // workspace, and a target's logit straight from the lane that holds it.  klp_lmh_combine_kernel merges the chunks of each token (one
 // wave per token, a fixed order) and applies the output formulas.
 //
-// klp_lmh_kernel<true, ..> (backward) runs the same tiles and replaces the fold
-// with the gradient of klp_bwd, written to d_logits as bf16.
+// The backward (kGradient) runs the same tiles and replaces the fold with the
+// gradient of klp_bwd, written to d_logits; kLogits writes the logits.
 //
 // Bound: power.  At 1024 tokens of a [152064, 3584] weight the MFMAs take 4/5
 // of the kernel's cycles, and the chip lowers its clock under them: 1.85 GHz,
@@ -60,70 +60,27 @@
 // chunk, so the chunk's weight rows are fetched from HBM once per XCD and
 // shared through its L2 by the token blocks running there together.
 #include "klp_launch.h"
+#include "klp_mfma.h"
 
 namespace klp {
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+using namespace mfma;
 
-constexpr int kThreads = 256;
-constexpr int kBlocks = 8;          // 16-row / 16-token MFMA blocks per wave and side
-constexpr int kWaveSide = kBlocks * 16;
-constexpr int kBV = 2 * kWaveSide;  // vocab rows per tile (2 waves along vocab): 256
-constexpr int kBT = 2 * kWaveSide;  // tokens per block (2 waves along tokens): 256
-constexpr int kBK = 64;             // K columns per stage
-constexpr int kRowBytes = kBK * 2;
-constexpr int kSlotBytes = 256 * kRowBytes;
-constexpr int kWSlots = 3;
-constexpr int kHSlots = 2;
-constexpr int kLdsBytes = (kWSlots + kHSlots) * kSlotBytes;
-static_assert(kLdsBytes <= 160 * 1024, "LDS holds 160 KB");
-// One copy moves 64 lanes x 16 B = 1 KB, 8 LDS rows; the 4 waves' copies of
-// index j cover rows 32 j .. 32 j + 31 of a slot.
-constexpr int kCopies = 8;
+constexpr int kBV = kTile;  // vocab rows per tile
+constexpr int kBT = kTile;  // tokens per block
 
-// The 16-byte chunk c of LDS row `row` sits at chunk c ^ swz_f(row): one
-// chunk of 16 consecutive rows, an operand read's quarter wave, then meets
-// every bank once, whether the LDS serves 8 or 16 lanes x 16 B per cycle.
-__device__ __forceinline__ int swz_f(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-
-// s_waitcnt immediate: vmcnt <= vm, lgkmcnt <= lgkm (15: no wait).
-constexpr int waitcnt(int vm, int lgkm) {
-    return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8);
-}
-
-// acc += a * b (`zero`: acc = a * b), in AGPRs and in place: left to the
-// builtin, the compiler renames the 256 accumulators from MFMA to MFMA and
-// pays for it in moves through VGPRs and spills at every join.  What it would
-// insert around its own MFMAs is then the caller's: the operands come from
-// LDS reads (waited for as any use), an accumulator's own MFMAs are 64 apart,
-// and mfma_drain() comes before other instructions read accumulators.
-__device__ __forceinline__ void mfma_in_place(f32x4& acc, bf16x8 a, bf16x8 b, bool zero) {
-    if (zero)  // a constant at every call
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
-    else
-        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
-// An accumulator's value, read where it is needed (the compiler would move
-// more than half of them to VGPRs ahead of the fold, and spill).
-__device__ __forceinline__ float acc_value(float acc) {
-    float v;
-    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc));
-    return v;
-}
-// The wait states between the last MFMA and a VALU read of its result (11 for
-// an MFMA of 8 passes), rounded up.
-__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 7"); }
-
-#define KLP_PIN() __builtin_amdgcn_sched_barrier(0)
+enum : int { kFold = 0, kGradient = 1, kLogits = 2 };
 
 }  // namespace
 
-// kGrad == false: the forward (partial states per vocab chunk).
-// kGrad == true: the backward's d_logits: the same logits tiles, turned into
-// the gradient of klp_bwd (grad_one, klp_device.h) and written as bf16.
-template <bool kGrad, bool kScaled>
+// kMode kFold: the forward (partial states per vocab chunk); kGradient: the
+// backward's d_logits, the same logits tiles turned into the gradient of
+// klp_bwd (grad_one, klp_device.h) and written in DT; kLogits: the logits
+// themselves, rounded to DT (kRound, not scaled).  kRound: each logit is
+// rounded to DT before it is scaled and used, as a GEMM that writes DT does.
+template <int DT, int kMode, bool kRound, bool kScaled>
 __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     // The rings take all 160 KB of LDS; the end-of-chunk merge reuses them.
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kLdsBytes];
@@ -149,12 +106,12 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     if (tile_end > p.n_vtiles) tile_end = p.n_vtiles;
 
     // Copies.  Lane l of wave w fills, with copy j, chunk l % 8 of slot row
-    // 32 j + 8 w + l / 8, which holds global chunk (l % 8) ^ swz_f(row) of
-    // that row (swz_f reads row bits 0..3, the same for every j).  Rows past
+    // 32 j + 8 w + l / 8, which holds global chunk (l % 8) ^ swz(row) of
+    // that row (swz reads row bits 1..3, the same for every j).  Rows past
     // the matrix's end lie past the descriptor and read as zeros (their
     // logits are masked or never written).
     const int crow = wave * 8 + (lane >> 3);
-    const int cchunk = (lane & 7) ^ swz_f(crow);
+    const int cchunk = (lane & 7) ^ swz(crow);
     const uint32_t w_off = static_cast<uint32_t>(crow * p.ld_weight * 2 + cchunk * 16);
     const uint32_t h_off = static_cast<uint32_t>(crow * p.ld_hidden * 2 + cchunk * 16);
     const uint32_t w_step = static_cast<uint32_t>(p.ld_weight * 64);  // 32 rows
@@ -175,7 +132,6 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     int64_t w_tile = tile_first;
     int w_k = 0, w_slot = 0, h_k = 0, h_slot = 0;
     __amdgpu_buffer_rsrc_t w_rs = tile_rsrc(w_tile);
-    typedef __attribute__((address_space(3))) void lds_void;
     auto copy_w = [&](int j) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             w_rs, (lds_void*)(lds + w_slot * kSlotBytes + (wave + 4 * j) * 1024), 16, w_off,
@@ -185,12 +141,12 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
                 w_k = 0;
                 w_rs = tile_rsrc(++w_tile);
             }
-            w_slot = w_slot == kWSlots - 1 ? 0 : w_slot + 1;
+            w_slot = w_slot == kASlots - 1 ? 0 : w_slot + 1;
         }
     };
     auto copy_h = [&](int j) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            h_rs, (lds_void*)(lds + (kWSlots + h_slot) * kSlotBytes + (wave + 4 * j) * 1024), 16,
+            h_rs, (lds_void*)(lds + (kASlots + h_slot) * kSlotBytes + (wave + 4 * j) * 1024), 16,
             h_off, j * h_step + h_k * kRowBytes, 0, 0);
         if (j == kCopies - 1) {
             if (++h_k == n_k) h_k = 0;
@@ -203,15 +159,15 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     // stage's 32.
     const int lrow = lane & 15;
     const int lq = lane >> 4;
-    const int lf = swz_f(lrow);
+    const int lf = swz(lrow);
     int rw_slot = 0, rh_slot = 0;  // slots being read
     auto w_src = [&](int half, int i) {
-        return *reinterpret_cast<const bf16x8*>(lds + rw_slot * kSlotBytes + wv * (kSlotBytes / 2) +
+        return *reinterpret_cast<const operand*>(lds + rw_slot * kSlotBytes + wv * (kSlotBytes / 2) +
                                                 lrow * kRowBytes +
                                                 (((4 * half) ^ (lq ^ lf)) << 4) + i * 16 * kRowBytes);
     };
     auto h_src = [&](int half, int i) {
-        return *reinterpret_cast<const bf16x8*>(lds + (kWSlots + rh_slot) * kSlotBytes +
+        return *reinterpret_cast<const operand*>(lds + (kASlots + rh_slot) * kSlotBytes +
                                                 wt * (kSlotBytes / 2) + lrow * kRowBytes +
                                                 (((4 * half) ^ (lq ^ lf)) << 4) + i * 16 * kRowBytes);
     };
@@ -224,7 +180,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     for (int b = 0; b < kBlocks; ++b) {
         st[b] = stat_empty();
         const int64_t tok = my_tok + 16 * b;
-        const int64_t t = tok < p.n_tokens ? p.targets[tok] : -1;
+        const int64_t t = kMode != kLogits && tok < p.n_tokens ? p.targets[tok] - p.target_offset : -1;
         my_tgt[b] = t >= 0 && t < p.vocab ? static_cast<int>(t) : -1;
     }
 
@@ -239,14 +195,14 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     for (int j = 0; j < kCopies; ++j) copy_w(j);
 #pragma unroll
     for (int j = 0; j < kCopies; ++j) copy_h(j);
-    KLP_PIN();
+    pin();
     __builtin_amdgcn_s_waitcnt(waitcnt(2 * kCopies, 15));
     __builtin_amdgcn_s_barrier();
-    KLP_PIN();
+    pin();
     // Half a stage ahead: all 8 blocks of the token side (two sets, in turn)
     // and blocks 0..3 of the vocab side; its blocks 4..7 are read under the
     // MFMAs of 0..3.
-    bf16x8 aw[kBlocks], bh[2][kBlocks];
+    operand aw[kBlocks], bh[2][kBlocks];
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) bh[0][i] = h_src(0, i);
 #pragma unroll
@@ -269,14 +225,14 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
                         // weight copies after those).  After the barrier so for
                         // every wave: the stage's slots are free, the next
                         // stage's are full.
-                        KLP_PIN();
+                        pin();
                         __builtin_amdgcn_s_waitcnt(waitcnt(kCopies, 0));
                         __builtin_amdgcn_s_barrier();
-                        KLP_PIN();
-                        rw_slot = rw_slot == kWSlots - 1 ? 0 : rw_slot + 1;
+                        pin();
+                        rw_slot = rw_slot == kASlots - 1 ? 0 : rw_slot + 1;
                         rh_slot ^= 1;
                     }
-                    mfma_in_place(acc[a][b], aw[a], bh[q][b], kFirst && q == 0);
+                    mul_add<DT>(acc[a][b], aw[a], bh[q][b], kFirst && q == 0);
                     if (i < 32) {
                         if ((i & 7) == 3) aw[4 + a] = w_src(q, 4 + a);
                         if (q == 0 && (i & 3) == 2) copy_w(i >> 2);
@@ -285,14 +241,14 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
                         if ((i & 7) == 7) aw[a - 4] = w_src(q ^ 1, a - 4);
                         if (q == 1 && (i & 3) == 2) copy_h((i - 32) >> 2);
                     }
-                    KLP_PIN();
+                    pin();
                 }
             }
         };
         stage(std::true_type{});
         for (int k = 1; k < n_k; ++k) stage(std::false_type{});
-        mfma_drain();
-        KLP_PIN();
+        drain();
+        pin();
 
         // Accumulator r of block (a, b) holds tile row
         // wv * 128 + 16 a + 4 (l / 16) + r of the lane's token b.
@@ -300,58 +256,90 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
         const int row0 = wv * kWaveSide + 4 * lq;
         const int64_t left = p.vocab - v0;
         const int vlim = left < kBV ? static_cast<int>(left) : kBV;
-        if constexpr (kGrad) {
-            // d_logits of the tile; rows 4 l / 16 .. + 3 go out as one 8-byte
-            // store.
+        // Values 8 g .. 8 g + 7 of the lane's 32 of token b: rows 16 (2 g) + i
+        // and 16 (2 g + 1) + i beyond row0, i = 0..3.
+        auto values = [&](int b, int g, float* x) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = value(acc[2 * g + j / 4][b][j % 4]);
+            if constexpr (kRound) {
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) round2<DT>(x[j], x[j + 1]);
+            }
+            if constexpr (kScaled) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] *= p.scale;
+            }
+        };
+        if constexpr (kMode != kFold) {
+            // Output columns v0 .. of the lane's tokens; lane quarters trade
+            // halves so that 16 bytes go out a lane, 64 a token and store.  At
+            // the vocabulary's end, or where rows are not 16-byte aligned, 8
+            // bytes a lane or single elements, up to column n_out.
             RowGrad rg[kBlocks];
+            if constexpr (kMode == kGradient) {
+#pragma unroll
+                for (int b = 0; b < kBlocks; ++b) {
+                    const int64_t tok = my_tok + 16 * b;
+                    const bool ok = tok < p.n_tokens;
+                    rg[b] = ok ? row_grad(p.saved_lse[tok], p.saved_entropy[tok],
+                                          p.g_logp ? p.g_logp[tok] : 0.0f,
+                                          p.g_ent ? p.g_ent[tok] : 0.0f,
+                                          p.g_lse ? p.g_lse[tok] : 0.0f)
+                               : row_grad(0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
+                }
+            }
+            const bool whole = vlim == kBV && p.out_align >= 16;
+            const int64_t out_left = p.n_out - v0;
+            const int olim = out_left < kBV ? static_cast<int>(out_left) : kBV;
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) {
                 const int64_t tok = my_tok + 16 * b;
                 const bool ok = tok < p.n_tokens;
-                rg[b] = ok ? row_grad(p.saved_lse[tok], p.saved_entropy[tok],
-                                      p.g_logp ? p.g_logp[tok] : 0.0f,
-                                      p.g_ent ? p.g_ent[tok] : 0.0f, p.g_lse ? p.g_lse[tok] : 0.0f)
-                           : row_grad(0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
-            }
-#pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
-                const int64_t tok = my_tok + 16 * b;
-                if (tok >= p.n_tokens) continue;
-                uint16_t* drow = p.d_logits + tok * p.ld_d + v0 + row0;
+                uint16_t* out = p.out + tok * p.ld_out + v0 + wv * kWaveSide;
                 const int target = my_tgt[b] - static_cast<int>(v0) - row0;
 #pragma unroll
-                for (int a = 0; a < kBlocks; ++a) {
-                    if (16 * a >= vlim - row0) continue;
-                    float d[4];
+                for (int g = 0; g < 4; ++g) {
+                    float x[8];
+                    values(b, g, x);
+                    if constexpr (kMode == kGradient) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float v = acc_value(acc[a][b][i]);
-                        if (kScaled) v *= p.scale;
-                        float g = grad_one(v, rg[b]);
-                        if (16 * a + i == target) g += rg[b].g_logp;
-                        if (16 * a + i >= vlim - row0) g = 0.0f;
-                        d[i] = kScaled ? g * p.scale : g;
+                        for (int j = 0; j < 8; ++j) {
+                            x[j] = grad_one(x[j], rg[b]);
+                            if (16 * (2 * g + j / 4) + j % 4 == target) x[j] += rg[b].g_logp;
+                            if (kScaled) x[j] *= p.scale;
+                        }
                     }
-                    const bf16x2 lo = __builtin_convertvector(f32x2{d[0], d[1]}, bf16x2);
-                    const bf16x2 hi = __builtin_convertvector(f32x2{d[2], d[3]}, bf16x2);
-                    uint2 w;
-                    w.x = __builtin_bit_cast(uint32_t, lo);
-                    w.y = __builtin_bit_cast(uint32_t, hi);
-                    *reinterpret_cast<uint2*>(drow + 16 * a) = w;
-                    KLP_PIN();
+                    const uint32_t lo[2] = {pack2<DT>(x[0], x[1]), pack2<DT>(x[2], x[3])};
+                    const uint32_t hi[2] = {pack2<DT>(x[4], x[5]), pack2<DT>(x[6], x[7])};
+                    if (whole) {
+                        const u32x4 w = gather8(lo, hi);
+                        if (ok) *reinterpret_cast<u32x4*>(out + 32 * g + 8 * lq) = w;
+                    } else if (ok) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const int r0 = 32 * g + 16 * h;
+                            if (r0 >= olim - row0) continue;
+                            uint32_t w[2] = {h ? hi[0] : lo[0], h ? hi[1] : lo[1]};
+                            const int n = vlim - row0 - r0;  // of the 4, the vocabulary's
+                            if (n < 4) w[1] = n == 3 ? w[1] & 0xFFFFu : 0u;
+                            if (n < 2) w[0] = n == 1 ? w[0] & 0xFFFFu : 0u;
+                            uint16_t* at = out + r0 + 4 * lq;
+                            if (p.out_align >= 8 && olim - row0 - r0 >= 4) {
+                                *reinterpret_cast<uint2*>(at) = make_uint2(w[0], w[1]);
+                            } else {
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    if (i < olim - row0 - r0)
+                                        at[i] = static_cast<uint16_t>(w[i / 2] >> (16 * (i & 1)));
+                            }
+                        }
+                    }
+                    pin();
                 }
             }
             continue;
         }
 
-        // Values 8 g .. 8 g + 7 of the lane's 32 of token b.
-        auto values = [&](int b, int g, float* x) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                x[j] = acc_value(acc[2 * g + j / 4][b][j % 4]);
-                if (kScaled) x[j] *= p.scale;
-            }
-        };
         // The target logits the lane holds: of every 16 rows from row0, 0..3.
         const int first = static_cast<int>(v0) + row0;
 #pragma unroll
@@ -386,7 +374,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
                     for (int j = 0; j < 8; ++j)
                         if (16 * (2 * g + j / 4) + j % 4 >= last) x[j] = -INFINITY;
                     absorb<8, true>(st[b], x);
-                    KLP_PIN();
+                    pin();
                 }
             }
         } else {
@@ -397,7 +385,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
 #pragma unroll
                 for (int g = 0; g < 4; ++g) values(b, g, x + 8 * g);
                 absorb<32, false>(st[b], x);
-                KLP_PIN();
+                pin();
                 if (needs_clamped_rescan(st[b])) {  // a -inf logit
                     st[b] = before;
 #pragma unroll
@@ -410,13 +398,15 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
         }
     }
 
-    if constexpr (kGrad) return;
+    // The last copies (of length 0) write zeros to LDS: before it is reused,
+    // or given up.
+    __builtin_amdgcn_s_waitcnt(waitcnt(0, 15));
+    if constexpr (kMode != kFold) return;
 
     // Merge the four lanes of each token (vocab rows 4 apart), then the two
     // vocab-half waves of each token half through LDS (the rings' memory:
     // every wave is past its last read of it, and past its last copy into
     // it, once all reach the barrier).
-    __builtin_amdgcn_s_waitcnt(waitcnt(0, 15));
     __syncthreads();
     Stat (*merge_stat)[kBT] = reinterpret_cast<Stat (*)[kBT]>(lds);
 #pragma unroll
@@ -463,21 +453,41 @@ __global__ __launch_bounds__(256) void klp_lmh_combine_kernel(LmhParams p) {
 int64_t lmh_token_blocks(int64_t n_tokens) { return (n_tokens + kBT - 1) / kBT; }
 int64_t lmh_vocab_tiles(int64_t vocab) { return (vocab + kBV - 1) / kBV; }
 
-hipError_t launch_lmh_dlogits(const LmhParams& p, hipStream_t stream) {
-    const int64_t chunks8 = (p.n_chunks + 7) / 8 * 8;
-    return launch_kernel(p.scale != 1.0f ? klp_lmh_kernel<true, true> : klp_lmh_kernel<true, false>,
-                         dim3(static_cast<unsigned>(chunks8 * p.n_tblocks)), dim3(kThreads),
-                         stream, p);
-}
-
-hipError_t launch_lmh_fwd(const LmhParams& p, hipStream_t stream) {
+template <int DT, int kMode, bool kRound>
+static hipError_t launch_lmh_t(const LmhParams& p, hipStream_t stream) {
     // Round the chunk count up to a multiple of 8 (one per XCD per round);
     // padding workgroups exit at once.
     const int64_t chunks8 = (p.n_chunks + 7) / 8 * 8;
-    const int64_t blocks = chunks8 * p.n_tblocks;
-    hipError_t e =
-        launch_kernel(p.scale != 1.0f ? klp_lmh_kernel<false, true> : klp_lmh_kernel<false, false>,
-                      dim3(static_cast<unsigned>(blocks)), dim3(kThreads), stream, p);
+    const dim3 grid(static_cast<unsigned>(chunks8 * p.n_tblocks));
+    if constexpr (kMode != kLogits) {
+        if (p.scale != 1.0f)
+            return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, true>, grid, dim3(kThreads),
+                                 stream, p);
+    }
+    return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, false>, grid, dim3(kThreads), stream, p);
+}
+
+template <int kMode>
+static hipError_t launch_lmh_mode(int dtype, bool rounded, const LmhParams& p,
+                                  hipStream_t stream) {
+    if (dtype == kFP16 && rounded) return launch_lmh_t<kFP16, kMode, true>(p, stream);
+    if (dtype == kBF16 && rounded) return launch_lmh_t<kBF16, kMode, true>(p, stream);
+    if constexpr (kMode != kLogits) {
+        if (dtype == kBF16) return launch_lmh_t<kBF16, kMode, false>(p, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_lmh_dlogits(int dtype, bool rounded, const LmhParams& p, hipStream_t stream) {
+    return launch_lmh_mode<kGradient>(dtype, rounded, p, stream);
+}
+
+hipError_t launch_lmh_logits(int dtype, const LmhParams& p, hipStream_t stream) {
+    return launch_lmh_mode<kLogits>(dtype, true, p, stream);
+}
+
+hipError_t launch_lmh_fwd(int dtype, bool rounded, const LmhParams& p, hipStream_t stream) {
+    const hipError_t e = launch_lmh_mode<kFold>(dtype, rounded, p, stream);
     if (e != hipSuccess) return e;
     return launch_kernel(klp_lmh_combine_kernel,
                          dim3(static_cast<unsigned>((p.n_tokens + 3) / 4)), dim3(256), stream, p);

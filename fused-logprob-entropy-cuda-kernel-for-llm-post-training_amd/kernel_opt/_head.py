@@ -1,0 +1,89 @@
+"""The LM head's products through the hand-written MFMA kernels
+(csrc/klp_lmhead.hip, csrc/klp_head_gemm.hip): what the chunked head and the
+linear GRPO step run where the operands allow it and the kernels are the
+faster ones.
+
+``mfma_operands``: bf16 / fp16, a hidden size that is a multiple of 64,
+16-byte aligned rows.  Elsewhere (fp32, odd hidden sizes) the callers keep the
+library GEMMs.
+
+``logits_pay`` / ``d_weight_pays`` / ``d_hidden_pays``: small products are one
+launch's time in the library, while a 256 x 256 tile a workgroup leaves most
+of the chip idle there and d_hidden is two launches.  Ours against the library
+(bf16, us, launches queued):
+    N     V       D     logits       d_weight     d_hidden
+    16    16384   512   15 / 6       10 / 11      29 / 21
+    64    16384   512   15 / 6       10 / 9       31 / 68
+    64    16384   1024  23 / 9       11 / 12      27 / 81
+    128   32000   1024  24 / 15      20 / 23      37 / 101
+    256   50240   2048  48 / 57      79 / 104     73 / 207
+    512   32000   1024  32 / 36      39 / 45      50 / 146
+    64    152064  3584  236 / 205
+    192   152064  3584  269 / 287
+    1024  152064  3584  843 / 902    971 / 1198   895 / 1475
+"""
+from __future__ import annotations
+
+import torch
+
+from ._library import DTYPE_CODES, check_status, lib, ptr
+
+_MAX_LD = (2 ** 31 - 1) // 512  # 32-bit byte offsets within 256 rows
+
+
+def row_stride(t: torch.Tensor) -> int:
+    return t.stride(0) if t.size(0) > 1 else t.size(1)
+
+
+def _rows_ok(t: torch.Tensor) -> bool:
+    ld = row_stride(t)
+    return t.data_ptr() % 16 == 0 and ld % 8 == 0 and t.size(1) <= ld <= _MAX_LD
+
+
+def mfma_operands(h2: torch.Tensor, weight: torch.Tensor) -> bool:
+    """True when the MFMA kernels take hidden ``[N, D]`` and weight ``[V, D]``
+    (one dtype, rows with unit stride)."""
+    return (h2.dtype in (torch.bfloat16, torch.float16) and h2.size(0) > 0
+            and h2.size(1) >= 64 and h2.size(1) % 64 == 0 and h2.stride(1) == 1
+            and weight.stride(1) == 1 and _rows_ok(h2) and _rows_ok(weight))
+
+
+def logits_pay(n_tokens: int, vocab: int, dim: int) -> bool:
+    return n_tokens >= 192 and n_tokens * vocab * dim >= 15 << 30 and vocab % 8 == 0
+
+
+def d_weight_pays(vocab: int, dim: int) -> bool:
+    return vocab * dim >= 16 << 20
+
+
+def d_hidden_pays(n_tokens: int, vocab: int, dim: int) -> bool:
+    return n_tokens * vocab * dim >= 1 << 29
+
+
+def logits_into(out: torch.Tensor, h2: torch.Tensor, weight: torch.Tensor, stream) -> None:
+    """``out[:, :] = h2 @ weight^T``, rounded once to the dtype."""
+    check_status(lib.klp_lmh_logits(DTYPE_CODES[h2.dtype], ptr(h2), row_stride(h2), ptr(weight),
+                                    row_stride(weight), h2.size(0), weight.size(0), h2.size(1),
+                                    ptr(out), row_stride(out), stream))
+
+
+def d_weight_into(out: torch.Tensor, d: torch.Tensor, ld_d: int, h2: torch.Tensor,
+                  stream) -> None:
+    """``out = d^T @ h2`` for d_logits ``[N, out.size(0)]`` with row stride
+    ``ld_d``."""
+    check_status(lib.klp_head_dweight(DTYPE_CODES[h2.dtype], ptr(d), ld_d, h2.size(0), out.size(0),
+                                      ptr(h2), row_stride(h2), h2.size(1), ptr(out),
+                                      row_stride(out), stream))
+
+
+def d_hidden_into(out: torch.Tensor | None, acc: torch.Tensor | None, accumulate: bool,
+                  d: torch.Tensor, ld_d: int, n_tokens: int, weight: torch.Tensor,
+                  stream) -> None:
+    """``s = d @ weight`` (+ ``acc`` with ``accumulate``) in float32, into
+    ``out`` (rounded once) or, with ``out`` None, into ``acc``."""
+    V, D = weight.shape
+    nbytes = lib.klp_head_dhidden_workspace_bytes(n_tokens, V, D)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=weight.device)
+    check_status(lib.klp_head_dhidden(DTYPE_CODES[weight.dtype], ptr(d), ld_d, n_tokens, V,
+                                      ptr(weight), row_stride(weight), D, ptr(acc),
+                                      int(accumulate), ptr(out), ptr(ws), nbytes, stream))

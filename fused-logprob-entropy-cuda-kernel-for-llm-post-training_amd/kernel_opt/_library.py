@@ -64,6 +64,15 @@ SIGNATURES = {
                            _vp, _vp, _vp, _vp, _sz, _vp]),
     "klp_lmh_bwd_logits": (_i32, [_vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, ctypes.c_float,
                                   _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "klp_lmh_fwd_as": (_i32, [_i32, _i32, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp,
+                              ctypes.c_float, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "klp_lmh_bwd_logits_as": (_i32, [_i32, _i32, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64,
+                                     ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "klp_lmh_logits": (_i32, [_i32, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp]),
+    "klp_head_dhidden_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "klp_head_dweight": (_i32, [_i32, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _vp]),
+    "klp_head_dhidden": (_i32, [_i32, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _i32, _vp, _vp,
+                                _sz, _vp]),
     "klp_grpo_workspace_bytes": (_sz, [_i64]),
     "klp_grpo_fwd": (_i32, [_vp] * 5 + [_i64, _i64] + [ctypes.c_float] * 4 + [_i32] * 3
                      + [_vp, _vp, _vp, _sz, _vp]),

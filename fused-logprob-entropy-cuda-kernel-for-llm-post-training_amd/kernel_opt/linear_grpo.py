@@ -9,12 +9,14 @@ is known inside the forward (``klp_grpo_step`` writes it in the same pass
 over the logits that computes the log-probabilities), so each chunk of tokens
 goes through
 
-    logits_c  = hidden_c @ weight^T                  (library GEMM, [c, V])
+    logits_c  = hidden_c @ weight^T                  ([c, V])
     klp_grpo_step(logits_c)                          (logp, entropy, loss, d_logits_c)
-    d_hidden_c = d_logits_c @ weight                 (library GEMM)
-    d_weight  += d_logits_c^T @ hidden_c             (library GEMM, float32 accumulator)
+    d_hidden_c = d_logits_c @ weight
+    d_weight  += d_logits_c^T @ hidden_c             (float32 accumulator)
 
-and is dropped before the next chunk: peak memory is two ``[c, V]`` buffers
+(the products through the MFMA kernels of ``_head`` where they take the
+operands, the accumulated d_weight of several chunks and other heads through
+library GEMMs) and is dropped before the next chunk: peak memory is two ``[c, V]`` buffers
 instead of the full logits and their gradient, and the backward has nothing
 left to recompute (it hands over d_hidden and d_weight, scaled by the loss's
 upstream gradient when that is not 1).
@@ -29,7 +31,9 @@ from __future__ import annotations
 
 import torch
 
-from ._library import DTYPE_CODES, lib
+from ._head import (d_hidden_into, d_hidden_pays, d_weight_into, d_weight_pays, logits_into,
+                    logits_pay, mfma_operands)
+from ._library import DTYPE_CODES, device_guard, lib, stream_handle
 from .grpo import fused_grpo_loss
 from .grpo_step import _check_grad_scale, grpo_step_launch, grpo_token_weights, scale_by_upstream
 from .ops import fused_logprob_entropy
@@ -85,7 +89,8 @@ class _FusedLinearGrpoStep(torch.autograd.Function):
         dev = hidden.device
         f32 = lambda: torch.empty(N, dtype=torch.float32, device=dev)  # noqa: E731
         logp, ent, loss_tok = f32(), f32(), f32()
-        d_hidden = torch.empty_like(h2) if need_h else None
+        d_hidden = torch.empty(N, D, dtype=h2.dtype, device=dev) if need_h else None
+        mfma = mfma_operands(h2, weight)
         d_weight = None
         single = chunk >= N
         step_params = (temperature, eps_low, eps_high, beta, 1, grad_scale)  # per-token adv.
@@ -93,7 +98,12 @@ class _FusedLinearGrpoStep(torch.autograd.Function):
             n1 = min(N, n0 + chunk)
             c = n1 - n0
             hc = h2[n0:n1]
-            logits = torch.mm(hc, weight.t())
+            if mfma and logits_pay(c, V, D):
+                logits = torch.empty(c, V, dtype=hc.dtype, device=dev)
+                with device_guard(dev.index):
+                    logits_into(logits, hc, weight, stream_handle(dev.index))
+            else:
+                logits = torch.mm(hc, weight.t())
             lp, en, _lse, lt, d = grpo_step_launch(
                 logits.view(1, c, V), t[n0:n1].view(1, c), old[n0:n1], ref[n0:n1]
                 if ref is not None else None, adv[n0:n1], wts[n0:n1], step_params)
@@ -103,9 +113,18 @@ class _FusedLinearGrpoStep(torch.autograd.Function):
             loss_tok[n0:n1] = lt.view(-1)
             d2 = d.view(c, V)
             if need_h:
-                torch.mm(d2, weight, out=d_hidden[n0:n1])
+                if mfma and d_hidden_pays(c, V, D):
+                    with device_guard(dev.index):
+                        d_hidden_into(d_hidden[n0:n1], None, False, d2, V, c, weight,
+                                      stream_handle(dev.index))
+                else:
+                    torch.mm(d2, weight, out=d_hidden[n0:n1])
             if need_w:
-                if single:
+                if single and mfma and d_weight_pays(V, D):
+                    d_weight = torch.empty(V, D, dtype=weight.dtype, device=dev)
+                    with device_guard(dev.index):
+                        d_weight_into(d_weight, d2, V, hc, stream_handle(dev.index))
+                elif single:
                     d_weight = torch.mm(d2.t(), hc)
                 else:
                     d_weight = _accumulate_f32(d_weight, d2.t(), hc)

@@ -8,38 +8,26 @@ the Liger-style head the reference names as its follow-up
 
 Two implementations:
 
-``impl="chunked"`` (default) walks the vocabulary in chunks
-(:func:`vocab_chunks`: 32768 columns for small batches, ~16K for larger
-ones).  Per chunk a library GEMM writes the chunk's logits (``[N, chunk]``
-in the input dtype, at most 128 MiB) and ``klp_fwd_chunk`` folds them into
-each token's online state; the last chunk's launch merges the chunk states
-in chunk order and writes the outputs.  The weight is read once and the
-logits never exist as one ``[N, V]`` tensor.  The backward recomputes each
-chunk with the same GEMM call (bit-identical logits), applies ``klp_bwd``
-with chunk-relative targets, and accumulates ``d_hidden += d_chunk @
-W_chunk`` (fp32) and ``d_weight[chunk] = d_chunk^T @ hidden``.  Numerics are
-the unfused path's: logits rounded once to the input dtype by the GEMM.
+``impl="chunked"`` (default) rounds each logit once to the input dtype, the
+unfused path's numerics.  bf16 / fp16 heads whose hidden size is a multiple of
+64 (``_head.mfma_operands``) run the hand-written gfx950 kernels: the forward
+is one GEMM with the logprob / entropy reduction as its epilogue
+(klp_lmh_fwd_as, csrc/klp_lmhead.hip), and the backward walks the vocabulary
+in chunks: per chunk the same GEMM again, with the gradient as its epilogue
+(bit-identical logits), then ``d_hidden += d_chunk @ W_chunk`` (fp32) and
+``d_weight[chunk] = d_chunk^T @ hidden`` (csrc/klp_head_gemm.hip).  Other heads
+walk the vocabulary in chunks in the forward too (:func:`vocab_chunks`): a
+library GEMM writes the chunk's logits (``[N, chunk]``, at most 128 MiB) and
+``klp_fwd_chunk`` folds them into each token's online state; the last chunk's
+launch merges the chunk states in chunk order and writes the outputs.  Their
+backward recomputes each chunk with the same GEMM call, applies ``klp_bwd``
+with chunk-relative targets, and runs two library GEMMs.
 
-``impl="mfma"`` is the hand-written gfx950 kernel (klp_lmh_fwd,
-csrc/klp_lmhead.hip): the GEMM with the logprob / entropy reduction as its
-epilogue, logits kept as fp32 MFMA sums (never rounded), bf16 inputs, hidden
-size a multiple of 64.  Its backward recomputes chunks of logits with the
-same MFMA order (klp_lmh_bwd_logits on a slice of the weight) and runs the
-same two library GEMMs per chunk.  It is slower than the library GEMM at
-these shapes (1024 tokens of Qwen2.5-7B's head, bench.py's lm_head leg:
-forward 1.30-1.32 ms, 34% of the bf16 MFMA peak, against 0.93 ms for the
-library GEMM) and is kept as a correct alternative, not tuned further.
+``impl="mfma"`` is the same kernels with the logits kept as fp32 MFMA sums
+(never rounded): bf16 inputs, hidden size a multiple of 64.
 
-At 1024 tokens the chunked forward runs within ~2% of the unfused one, on
-either side from box to box (bench.py's lm_head leg: 0.9356 against 0.9279 ms
-on one box, 0.901-0.954 against 0.911-0.948 ms on three others), while it holds 64 MiB of
-extra memory where the unfused path holds 297 MiB of logits; at 8192 tokens
-6.33 against 6.42 ms, 131 against 2376 MiB.
-
-The backward of either head recomputes the logits, one GEMM more than the
-unfused path's backward: that is the price of not holding them (measured
-forward + backward at 1024 tokens: 4.64-4.72 ms chunked, 3.83-3.87 ms
-unfused, with 135 MiB against 297 MiB beyond the inputs and gradients).  When the loss is
+The backward of either recomputes the logits, one GEMM more than the unfused
+path's backward: that is the price of not holding them.  When the loss is
 known in the forward, :func:`kernel_opt.fused_linear_grpo_step` computes the
 gradients there and needs no recompute.
 
@@ -54,6 +42,8 @@ import threading
 import torch
 
 from . import _C
+from ._head import (d_hidden_into, d_hidden_pays, d_weight_into, d_weight_pays, logits_into,
+                    mfma_operands)
 from ._library import DTYPE_CODES, check_status, device_guard, lib, ptr, stream_handle
 from .linear_grpo import _accumulate_f32
 
@@ -189,12 +179,45 @@ def vocab_chunks(n_tokens: int, vocab: int, elem_bytes: int = 2,
     return plan
 
 
+# Chunk of d_logits of the MFMA backward: as many columns as fit
+# MFMA_CHUNK_BYTES, balanced over the vocabulary in whole 256-column tiles, so
+# that small batches fill the chip (256 tokens over 32768 columns are 128
+# workgroups) and d_hidden's K is long.
+MFMA_CHUNK_BYTES = 64 << 20
+
+
+def _mfma_chunks(n_tokens: int, vocab: int, chunk_vocab: int | None) -> list:
+    """``(first column, width)`` of every chunk of the MFMA backward."""
+    if chunk_vocab is not None:
+        return vocab_chunks(n_tokens, vocab, 2, chunk_vocab)
+    n_chunks = max(1, -(-(n_tokens * vocab * 2) // MFMA_CHUNK_BYTES))
+    cols = -(-(-(-vocab // n_chunks)) // 256) * 256
+    return [(c0, min(cols, vocab - c0)) for c0 in range(0, vocab, cols)]
+
+
 def _chunk_logits(buf, h2, weight, c0, n):
     """logits[:, c0:c0+n] = h2 @ weight[c0:c0+n]^T into a contiguous view of
-    ``buf`` (the same call, hence the same values, in forward and backward)."""
+    ``buf``: the values the chunked head's forward and backward use."""
     out = buf[: h2.size(0) * n].view(h2.size(0), n)
-    torch.mm(h2, weight[c0:c0 + n].t(), out=out)
+    if mfma_operands(h2, weight):
+        with device_guard(h2.device.index):
+            logits_into(out, h2, weight[c0:c0 + n], stream_handle(h2.device.index))
+    else:
+        torch.mm(h2, weight[c0:c0 + n].t(), out=out)
     return out
+
+
+def _forward_mfma(h2, weight, t, T, rounded, out):
+    """The one-GEMM forward; logits rounded to the dtype, or kept in fp32."""
+    dev = h2.device
+    N, V, D = h2.size(0), weight.size(0), h2.size(1)
+    with device_guard(dev.index):
+        stream = stream_handle(dev.index)
+        ws = _workspace(dev, stream, lib.klp_lmh_workspace_bytes(N, V, D))
+        check_status(lib.klp_lmh_fwd_as(DTYPE_CODES[h2.dtype], int(rounded), _ptr(h2), _ld(h2),
+                                        _ptr(weight), _ld(weight), N, V, D, _ptr(t), T,
+                                        _ptr(out[0]), _ptr(out[1]), _ptr(out[2]), _ptr(ws),
+                                        ws.numel(), stream))
 
 
 def _forward_chunked(h2, weight, t, T, plan, out):
@@ -213,38 +236,64 @@ def _forward_chunked(h2, weight, t, T, plan, out):
                                            _ptr(out[1]), _ptr(out[2]), stream))
 
 
-def _backward_chunked(h2, weight, t, T, plan, lse, ent, gl, ge, gs, need_h, need_w, impl):
-    """d_hidden (fp32, or None) and d_weight (weight dtype, or None), one
-    vocabulary chunk of ``plan`` at a time: d_logits exist for one chunk
-    only."""
+def _backward_mfma(h2, weight, t, T, plan, lse, ent, gl, ge, gs, need_h, need_w, rounded):
+    """d_hidden (float32 or the operands' dtype, or None) and d_weight (their
+    dtype, or None), one vocabulary chunk of ``plan`` at a time: d_logits
+    exist for one chunk only."""
+    N, D, V = h2.size(0), h2.size(1), weight.size(0)
+    dev = h2.device
+    code = DTYPE_CODES[h2.dtype]
+    cols = max(n for _, n in plan)
+    own_dh, own_dw = d_hidden_pays(N, cols, D), d_weight_pays(cols, D)
+    dh = torch.empty(N, D, dtype=h2.dtype, device=dev) if need_h and own_dh else None
+    acc = None
+    if need_h and not own_dh:
+        acc = torch.zeros(N, D, dtype=torch.float32, device=dev)
+    elif need_h and len(plan) > 1:
+        acc = torch.empty(N, D, dtype=torch.float32, device=dev)
+    dw = torch.empty(V, D, dtype=weight.dtype, device=dev) if need_w else None
+    d = torch.empty(N * (-(-cols // 8) * 8), dtype=h2.dtype, device=dev)
+    with device_guard(dev.index):
+        stream = stream_handle(dev.index)
+        for c, (c0, n) in enumerate(plan):
+            ld_d = -(-n // 8) * 8
+            w_c = weight[c0:c0 + n]
+            check_status(lib.klp_lmh_bwd_logits_as(
+                code, int(rounded), _ptr(h2), _ld(h2), _ptr(w_c), _ld(weight), N, n, D, _ptr(t),
+                c0, T, _ptr(lse), _ptr(ent), _ptr(gl), _ptr(ge), _ptr(gs), _ptr(d), ld_d, stream))
+            d_c = d[: N * ld_d].view(N, ld_d)[:, :n]
+            if need_h and own_dh:
+                d_hidden_into(dh if c == len(plan) - 1 else None, acc, c > 0, d, ld_d, N, w_c,
+                              stream)
+            elif need_h:
+                _accumulate_f32(acc, d_c, w_c)
+            if need_w and own_dw:
+                d_weight_into(dw[c0:c0 + n], d, ld_d, h2, stream)
+            elif need_w:
+                torch.mm(d_c.t(), h2, out=dw[c0:c0 + n])
+    return acc if need_h and not own_dh else dh, dw
+
+
+def _backward_chunked(h2, weight, t, T, plan, lse, ent, gl, ge, gs, need_h, need_w):
+    """d_hidden (fp32, or None) and d_weight (weight dtype, or None) through
+    library GEMMs, one vocabulary chunk of ``plan`` at a time."""
     N, D, V = h2.size(0), h2.size(1), weight.size(0)
     dev = h2.device
     dh = torch.zeros(N, D, dtype=torch.float32, device=dev) if need_h else None
     dw = torch.empty(V, D, dtype=weight.dtype, device=dev) if need_w else None
     cols = max(n for _, n in plan)
-    d_buf = torch.empty(N * (-(-cols // 4) * 4), dtype=weight.dtype, device=dev)
-    if impl == "mfma":
-        h2, weight = _rows_32bit(h2), _rows_32bit(weight)
-    lg_buf = torch.empty(N * cols, dtype=h2.dtype, device=dev) if impl == "chunked" else None
+    d_buf = torch.empty(N * cols, dtype=weight.dtype, device=dev)
+    lg_buf = torch.empty(N * cols, dtype=h2.dtype, device=dev)
     with device_guard(dev.index):
         stream = stream_handle(dev.index)
         for c0, n in plan:
             tc = t - c0  # chunk-relative: a target outside the chunk adds no one-hot term
-            if impl == "chunked":
-                lg = _chunk_logits(lg_buf, h2, weight, c0, n)
-                d = d_buf[: N * n].view(N, n)
-                check_status(lib.klp_bwd_temp(_ptr(lg), DTYPE_CODES[lg.dtype], N, n,
-                                              *_C.row_layout(lg),
-                                              _ptr(tc), T, _ptr(lse), _ptr(ent), _ptr(gl),
-                                              _ptr(ge), _ptr(gs), _ptr(d), stream))
-            else:
-                ld_d = -(-n // 4) * 4
-                dpad = d_buf[: N * ld_d].view(N, ld_d)
-                w_c = weight[c0:c0 + n]
-                check_status(lib.klp_lmh_bwd_logits(
-                    _ptr(h2), _ld(h2), _ptr(w_c), _ld(weight), N, n, D, _ptr(tc), T, _ptr(lse),
-                    _ptr(ent), _ptr(gl), _ptr(ge), _ptr(gs), _ptr(dpad), ld_d, stream))
-                d = dpad[:, :n]
+            lg = _chunk_logits(lg_buf, h2, weight, c0, n)
+            d = d_buf[: N * n].view(N, n)
+            check_status(lib.klp_bwd_temp(_ptr(lg), DTYPE_CODES[lg.dtype], N, n,
+                                          *_C.row_layout(lg),
+                                          _ptr(tc), T, _ptr(lse), _ptr(ent), _ptr(gl),
+                                          _ptr(ge), _ptr(gs), _ptr(d), stream))
             w_c = weight[c0:c0 + n]
             if need_h:
                 _accumulate_f32(dh, d, w_c)
@@ -283,10 +332,17 @@ class _FusedLinearLogprobEntropy(torch.autograd.Function):
             return None if g is None else g.to(torch.float32, copy=False).reshape(-1).contiguous()
 
         T = 1.0 if ctx.temperature is None else float(ctx.temperature)
-        plan = vocab_chunks(N, V, h2.element_size(), ctx.chunk_vocab)
-        dh, dw = _backward_chunked(h2, weight, t, T, plan, lse.reshape(-1), ent.reshape(-1),
-                                   prep(g_logp), prep(g_ent), prep(g_lse), need_h, need_w,
-                                   ctx.impl)
+        args = (lse.reshape(-1), ent.reshape(-1), prep(g_logp), prep(g_ent), prep(g_lse), need_h,
+                need_w)
+        if ctx.impl == "mfma":
+            h2, weight = _rows_32bit(h2), _rows_32bit(weight)
+        if ctx.impl == "mfma" or mfma_operands(h2, weight):
+            dh, dw = _backward_mfma(h2, weight, t, T, _mfma_chunks(N, V, ctx.chunk_vocab), *args,
+                                    ctx.impl == "chunked")
+        else:
+            dh, dw = _backward_chunked(h2, weight, t, T,
+                                       vocab_chunks(N, V, h2.element_size(), ctx.chunk_vocab),
+                                       *args)
         if dh is not None:
             dh = dh.to(hidden.dtype).reshape(hidden.shape)
         return (dh, dw) + none
@@ -316,8 +372,10 @@ def fused_linear_logprob_entropy_forward(hidden: torch.Tensor, weight: torch.Ten
         temperature: optional T > 0; logits are multiplied by fp32(1/T).
         impl: ``"chunked"`` (bf16 / fp16 / fp32) or ``"mfma"`` (bf16, D a
             multiple of 64, both row strides multiples of 8).
-        chunk_vocab: columns per vocabulary chunk (chunked head, and the
-            backward of both); default :func:`vocab_chunks`.
+        chunk_vocab: columns per vocabulary chunk where a pass walks the
+            vocabulary in chunks (the backward; the forward of heads without
+            MFMA kernels); default :func:`vocab_chunks`, or chunks of 64 MiB
+            of d_logits.
 
     Returns ``(logprob, entropy, lse)``, float32, shaped like ``targets``.
     """
@@ -331,17 +389,13 @@ def fused_linear_logprob_entropy_forward(hidden: torch.Tensor, weight: torch.Ten
     T = 1.0 if temperature is None else float(temperature)
     if not (T > 0.0 and T != float("inf")):
         raise RuntimeError(f"temperature must be finite and > 0, got {T}")
-    if impl == "chunked":
+    if impl == "mfma":
+        _forward_mfma(_rows_32bit(h2), _rows_32bit(weight), t, T, False, out)
+    elif mfma_operands(h2, weight):
+        if chunk_vocab is not None and chunk_vocab < 1:
+            raise ValueError(f"chunk_vocab must be >= 1, got {chunk_vocab}")
+        _forward_mfma(h2, weight, t, T, True, out)
+    else:
         _forward_chunked(h2, weight, t, T, vocab_chunks(N, V, h2.element_size(), chunk_vocab),
                          out)
-        return tuple(out)
-    dev = hidden.device
-    h2, weight = _rows_32bit(h2), _rows_32bit(weight)
-    with device_guard(dev.index):
-        stream = stream_handle(dev.index)
-        ws = _workspace(dev, stream, lib.klp_lmh_workspace_bytes(N, V, D))
-        rc = lib.klp_lmh_fwd(_ptr(h2), _ld(h2), _ptr(weight), _ld(weight),
-                             N, V, D, _ptr(t), T, _ptr(out[0]), _ptr(out[1]), _ptr(out[2]),
-                             _ptr(ws), ws.numel(), stream)
-    check_status(rc)
     return tuple(out)

@@ -463,6 +463,65 @@ int klp_lmh_bwd_logits(const void* hidden, int64_t ld_hidden, const void* weight
                        const float* g_lse, void* d_logits, int64_t ld_d, void* stream);
 
 /*
+ * klp_lmh_fwd and klp_lmh_bwd_logits for `dtype` operands with a choice of
+ * rounding: `rounded` non-zero rounds each logit once to `dtype` before it is
+ * scaled and used (what a GEMM writing `dtype` and klp_fwd / klp_bwd give),
+ * zero keeps the fp32 sums (bf16 operands only).  klp_lmh_bwd_logits_as takes
+ * targets relative to `vocab_offset` (weight row v holds column vocab_offset
+ * + v) and a d_logits of `dtype`, 16-byte aligned, ld_d a multiple of 8 that
+ * holds round_up(vocab, 8) columns; columns vocab .. round_up(vocab, 8) - 1
+ * are written with 0.  klp_lmh_logits writes the rounded logits themselves
+ * ([n_tokens, ld_logits], ld_logits >= vocab): the values the rounded forms
+ * use, bit for bit.
+ */
+int klp_lmh_fwd_as(int dtype, int rounded, const void* hidden, int64_t ld_hidden,
+                   const void* weight, int64_t ld_weight, int64_t n_tokens, int64_t vocab,
+                   int64_t dim, const int64_t* targets, float temperature, float* logprob,
+                   float* entropy, float* lse, void* workspace, size_t workspace_bytes,
+                   void* stream);
+
+int klp_lmh_bwd_logits_as(int dtype, int rounded, const void* hidden, int64_t ld_hidden,
+                          const void* weight, int64_t ld_weight, int64_t n_tokens, int64_t vocab,
+                          int64_t dim, const int64_t* targets, int64_t vocab_offset,
+                          float temperature, const float* lse, const float* entropy,
+                          const float* g_logp, const float* g_ent, const float* g_lse,
+                          void* d_logits, int64_t ld_d, void* stream);
+
+int klp_lmh_logits(int dtype, const void* hidden, int64_t ld_hidden, const void* weight,
+                   int64_t ld_weight, int64_t n_tokens, int64_t vocab, int64_t dim, void* logits,
+                   int64_t ld_logits, void* stream);
+
+/*
+ * The two products that carry d_logits to the LM head's operands, with MFMA
+ * kernels (float32 sums):
+ *   klp_head_dweight:  d_weight[v, d] = sum_n d_logits[n, v] * hidden[n, d],
+ *     rounded once to `dtype`, into [vocab, ld_out];
+ *   klp_head_dhidden:  s[n, d] = (accumulate ? acc[n, d] : 0) +
+ *     sum_v d_logits[n, v] * weight[v, d]; s goes to `acc` (float32, dense
+ *     [n_tokens, dim]), or, with `d_hidden` non-null, rounded once to `dtype`
+ *     into `d_hidden` (dense [n_tokens, dim]) instead (`acc` is then read
+ *     only, and only with `accumulate`).
+ * d_logits [n_tokens, ld_d], hidden [n_tokens, ld_hidden] and weight
+ * [vocab, ld_weight] are bf16 or fp16 (`dtype`), 16-byte aligned, row strides
+ * multiples of 8 elements; dim is a positive multiple of 64.  Columns vocab ..
+ * round_up(vocab, 8) - 1 of d_logits are read by klp_head_dhidden (times
+ * zero: they must be finite) and ld_d must hold them.  The workspace
+ * (klp_head_dhidden_workspace_bytes, 16-byte aligned, no initialisation)
+ * holds float32 partial sums; launches sharing one must be ordered on one
+ * stream.  Sums have a fixed order for given sizes.
+ */
+size_t klp_head_dhidden_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t dim);
+
+int klp_head_dweight(int dtype, const void* d_logits, int64_t ld_d, int64_t n_tokens,
+                     int64_t vocab, const void* hidden, int64_t ld_hidden, int64_t dim,
+                     void* d_weight, int64_t ld_out, void* stream);
+
+int klp_head_dhidden(int dtype, const void* d_logits, int64_t ld_d, int64_t n_tokens,
+                     int64_t vocab, const void* weight, int64_t ld_weight, int64_t dim,
+                     float* acc, int accumulate, void* d_hidden, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
+/*
  * Test hook with no counterpart in the reference: the next `count` compute
  * calls on the calling thread return KLP_ELAUNCH without launching anything,
  * as if hipGetLastError() had reported a failure.  Lets the error path be

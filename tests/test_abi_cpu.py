@@ -592,3 +592,69 @@ def test_noalloc_forward_validation_errors():
     assert fwd(V=0) == KLP_EINVAL and "vocab" in _err()
     assert fwd(x=None) == KLP_EINVAL and "non-null" in _err()
     assert fwd(t=ctypes.c_void_p(0x100004)) == KLP_EINVAL and "targets" in _err()
+
+
+def _head_calls(lib, dtype=0, n=4, v=100, d=64, ld_d=104, ld_o=64, p=P, ws=P, nb=1 << 20, out=P):
+    return {
+        "dweight": lambda: lib.klp_head_dweight(dtype, p, ld_d, n, v, p, ld_o, d, out, d, None),
+        "dhidden": lambda: lib.klp_head_dhidden(dtype, p, ld_d, n, v, p, ld_o, d, p, 0, out, ws, nb,
+                                                None),
+    }
+
+
+@pytest.mark.parametrize("which", ["dweight", "dhidden"])
+@pytest.mark.parametrize("kw,message", [
+    (dict(dtype=2), "bf16 or fp16"),
+    (dict(d=96), "multiple of 64"),
+    (dict(ld_d=100), "multiples of 8"),
+    (dict(ld_d=96), "at least dim and vocab"),
+    (dict(ld_o=8), "at least dim and vocab"),
+    (dict(ld_o=1 << 23), "not supported"),
+    (dict(p=None), "non-null"),
+    (dict(p=ctypes.c_void_p(0x10008)), "16-byte aligned"),
+    (dict(v=0), "vocab >= 1"),
+    (dict(out=ctypes.c_void_p(0x10004)), "16-byte aligned"),
+])
+def test_head_products_reject_bad_arguments(which, kw, message):
+    from kernel_opt._library import lib
+    rc = _head_calls(lib, **kw)[which]()
+    buf = ctypes.create_string_buffer(512)
+    lib.klp_last_error(buf, 512)
+    assert rc != 0 and message in buf.value.decode(), (rc, buf.value)
+
+
+def test_head_dhidden_needs_its_workspace():
+    from kernel_opt._library import lib
+    need = lib.klp_head_dhidden_workspace_bytes(4, 100, 64)
+    assert need > 0 and need % (4 * 64 * 4) == 0
+    assert lib.klp_head_dhidden_workspace_bytes(0, 100, 64) == 0
+    for kw in (dict(ws=None), dict(nb=need - 1)):
+        rc = _head_calls(lib, **kw)["dhidden"]()
+        buf = ctypes.create_string_buffer(512)
+        lib.klp_last_error(buf, 512)
+        assert rc != 0 and "workspace" in buf.value.decode()
+
+
+def test_lm_head_as_rejects_bad_arguments():
+    from kernel_opt._library import lib
+
+    def error():
+        buf = ctypes.create_string_buffer(512)
+        lib.klp_last_error(buf, 512)
+        return buf.value.decode()
+
+    def fwd(dtype, rounded):
+        return lib.klp_lmh_fwd_as(dtype, rounded, P, 64, P, 64, 4, 100, 64, P, 1.0, P, P, P, None, 0,
+                                  None)
+    assert fwd(1, 0) != 0 and "rounded" in error()
+    assert fwd(2, 1) != 0 and "bf16" in error()
+    assert fwd(0, 1) != 0 and "workspace" in error()
+
+    def bwd(ld_d, offset, p=P):
+        return lib.klp_lmh_bwd_logits_as(0, 1, P, 64, P, 64, 4, 100, 64, P, offset, 1.0, P, P, P, P,
+                                         P, p, ld_d, None)
+    assert bwd(100, 0) != 0 and "multiple of 8" in error()
+    assert bwd(96, 0) != 0 and "holds vocab" in error()
+    assert bwd(104, -1) != 0 and "vocab_offset" in error()
+    assert bwd(104, 0, None) != 0 and "non-null" in error()
+    assert lib.klp_lmh_logits(0, P, 64, P, 64, 4, 100, 64, P, 96, None) != 0 and ">= vocab" in error()

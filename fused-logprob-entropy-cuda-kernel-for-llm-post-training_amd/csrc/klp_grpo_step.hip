@@ -13,7 +13,8 @@
 // trainer divides the loss by k gradient-accumulation steps), so that the
 // backward has nothing left to do.
 // The unfused step reads the logits twice (forward, backward) and writes
-// d_logits once; here one workgroup of 1024 threads keeps its whole row in
+// d_logits once; here one workgroup of 1024 threads (256 or 512 where
+// launch_step_dt says so) keeps its whole row in
 // registers, so the logits are read once: 2 passes of HBM traffic instead
 // of 3.  A thread holds up to kGrpoStepMaxVec = 19 16-byte vectors (76 of the
 // 128 VGPRs a 1024-thread workgroup allows; 20 spill): 304 KB per row, a
@@ -128,13 +129,13 @@ __device__ __forceinline__ Stat scan_regs(const u32x4 (&r)[NV], int n_full, bool
 // The target logit comes from the registers: the thread holding it
 // publishes it (a global load issued after the row's loads would make every
 // wave wait for the whole row before its scan).
-template <int DT, int NV, bool kScaled>
+template <int DT, int NV, bool kScaled, int kThreads>
 __device__ __forceinline__ void publish_target(const u32x4 (&r)[NV], int64_t tgt, int tid,
                                                float scale, float* target_logit) {
     constexpr int EPV = Traits<DT>::kPerVec;
     const int64_t tv = tgt / EPV;
-    if (static_cast<int>(tv % kStepThreads) != tid) return;
-    const int kt = static_cast<int>(tv / kStepThreads);
+    if (static_cast<int>(tv % kThreads) != tid) return;
+    const int kt = static_cast<int>(tv / kThreads);
     const int jt = static_cast<int>(tgt - tv * EPV);
     float xt = 0.0f;
 #pragma unroll
@@ -159,15 +160,15 @@ struct StepShared {
 };
 
 // The row's results: the wave reduction (flat: one maximum, one rescale per
-// lane, two sums), the 16 wave states through LDS, merged by wave 0 (each of
-// its 16-lane DPP rows reads all of them and reduces them the same way, every
-// lane ending with the same bits), which computes the
+// lane, two sums), the wave states through LDS, merged by wave 0 (each of its
+// 16-lane DPP rows reads all of them, empty states past the last, and reduces
+// them the same way, every lane ending with the same bits), which computes the
 // row's results and the token's GRPO terms, writes them, and hands the
 // backward's constants to the other waves through LDS.  Both barriers are
 // here; `s` is this thread's state.  With kPublishNext, thread 0 also
 // publishes `next_row` (its claim of the workgroup's next row) between the
 // barriers: every wave read the previous one before the first.
-template <bool kPublishNext>
+template <bool kPublishNext, int kWaves>
 __device__ __forceinline__ RowGrad row_results(const GrpoStepParams& p, int64_t row, Stat s,
                                                bool has_t, const RowInputs& in, bool has_ref,
                                                float eps_low, float eps_high, float beta,
@@ -179,10 +180,11 @@ __device__ __forceinline__ RowGrad row_results(const GrpoStepParams& p, int64_t 
     s = wave_reduce_flat(s);
     if (lane == 0) sh.wave_stat[wave] = s;
     __syncthreads();
-    static_assert(kStepWaves == 16, "one wave state per lane of a DPP row");
+    static_assert(kWaves <= 16, "one wave state per lane of a DPP row");
     if (wave == 0) {
         const RowOut o =
-            finalize(row_reduce_flat(sh.wave_stat[lane & 15]), has_t ? sh.target_logit : 0.0f);
+            finalize(row_reduce_flat((lane & 15) < kWaves ? sh.wave_stat[lane & 15] : stat_empty()),
+                     has_t ? sh.target_logit : 0.0f);
         // GRPO terms of this token (token-level importance weight).
         const TokenLoss tl = grpo_token_loss(eps_low, eps_high, beta, o.logp - in.old_lp,
                                              in.adv, o.logp, in.ref_lp, has_ref);
@@ -236,9 +238,10 @@ __device__ __forceinline__ u32x4 grad_vec(u32x4 v, uint32_t i, const RowGrad& g,
 
 }  // namespace
 
-// One workgroup per row.
-template <int DT, int NV, bool kScaled>
-__global__ __launch_bounds__(kStepThreads) void klp_grpo_step_kernel(GrpoStepParams p) {
+// One workgroup of kThreads threads per row; vector k of a thread is the
+// row's vector tid + k * kThreads (kStepThreads in the comments above).
+template <int DT, int NV, bool kScaled, int kThreads>
+__global__ __launch_bounds__(kThreads) void klp_grpo_step_kernel(GrpoStepParams p) {
     typedef typename Traits<DT>::elem elem;
     constexpr int EPV = Traits<DT>::kPerVec;
     const int tid = threadIdx.x;
@@ -246,8 +249,8 @@ __global__ __launch_bounds__(kStepThreads) void klp_grpo_step_kernel(GrpoStepPar
     const elem* rp = static_cast<const elem*>(p.logits) + row_offset(p.rm, row);
     const uint32_t nvec = static_cast<uint32_t>(p.vocab / EPV);
     const uint32_t row_bytes = nvec * 16u;
-    const int n_full = static_cast<int>(nvec / kStepThreads);
-    const bool has_tail = static_cast<uint32_t>(tid) < nvec - n_full * kStepThreads;
+    const int n_full = static_cast<int>(nvec / kThreads);
+    const bool has_tail = static_cast<uint32_t>(tid) < nvec - n_full * kThreads;
 
     // Every load is issued, unconditionally: a load skipped on some path
     // leaves the number of loads in flight unknown, and the compiler then
@@ -259,7 +262,7 @@ __global__ __launch_bounds__(kStepThreads) void klp_grpo_step_kernel(GrpoStepPar
     u32x4 r[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        r[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, (tid + k * kStepThreads) * 16, 0,
+        r[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, (tid + k * kThreads) * 16, 0,
                                                      kCachePolicyNt);
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -271,8 +274,8 @@ __global__ __launch_bounds__(kStepThreads) void klp_grpo_step_kernel(GrpoStepPar
 
     const Stat s = scan_regs<DT, NV, kScaled>(r, n_full, has_tail, p.scale);
     __shared__ StepShared sh;
-    if (has_t) publish_target<DT, NV, kScaled>(r, in.tgt, tid, p.scale, &sh.target_logit);
-    const RowGrad g = row_results<false>(p, row, s, has_t, in, has_ref, p.eps_low, p.eps_high,
+    if (has_t) publish_target<DT, NV, kScaled, kThreads>(r, in.tgt, tid, p.scale, &sh.target_logit);
+    const RowGrad g = row_results<false, kThreads / 64>(p, row, s, has_t, in, has_ref, p.eps_low, p.eps_high,
                                          p.beta, 0, sh);
 
     // Pass 2: d_logits from the registers.  Stores past the row's end are
@@ -283,7 +286,7 @@ __global__ __launch_bounds__(kStepThreads) void klp_grpo_step_kernel(GrpoStepPar
     const int t_elem = has_t ? static_cast<int>(in.tgt % EPV) : 0;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const uint32_t i = tid + k * kStepThreads;
+        const uint32_t i = tid + k * kThreads;
         if (k <= n_full)
             store_vec_nt(grad_vec<DT, kScaled>(r[k], i, g, t_vec, t_elem, p.scale), ds, i * 16u,
                          0);
@@ -378,12 +381,12 @@ __global__ __launch_bounds__(kStepThreads) void klp_grpo_step_rows_kernel(GrpoSt
         // pending result that a later wait would have to cover, with the
         // output stores in front of it.
         asm volatile("" : "+v"(claimed));
-        if (has_t) publish_target<DT, NV, kScaled>(r, in.tgt, tid, p.scale, &sh.target_logit);
+        if (has_t) publish_target<DT, NV, kScaled, kStepThreads>(r, in.tgt, tid, p.scale, &sh.target_logit);
         // The clip bounds are recomputed per row rather than kept live (and
         // spilled) across the loop.
         float eps_low = p.eps_low, eps_high = p.eps_high, beta = p.beta;
         asm volatile("" : "+s"(eps_low), "+s"(eps_high), "+s"(beta));
-        const RowGrad g = row_results<true>(
+        const RowGrad g = row_results<true, kStepWaves>(
             p, row, s, has_t, in, has_ref, eps_low, eps_high, beta,
             static_cast<int64_t>(gridDim.x) + static_cast<int64_t>(claimed), sh);
 
@@ -490,8 +493,19 @@ static hipError_t launch_step(const GrpoStepParams& p, hipStream_t stream) {
             return launch_kernel(klp_grpo_step_rows_kernel<DT, NV, kScaled>,
                                  dim3(static_cast<unsigned>(wgs)), dim3(kStepThreads), stream, p);
     }
-    return launch_kernel(klp_grpo_step_kernel<DT, NV, kScaled>,
+    return launch_kernel(klp_grpo_step_kernel<DT, NV, kScaled, kStepThreads>,
                          dim3(static_cast<unsigned>(p.n_rows)), dim3(kStepThreads), stream, p);
+}
+
+// One row per workgroup of fewer threads.
+template <int DT, int NV, int kThreads>
+static hipError_t launch_row(const GrpoStepParams& p, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(p.n_rows));
+    if (p.scale != 1.0f)
+        return launch_kernel(klp_grpo_step_kernel<DT, NV, true, kThreads>, grid, dim3(kThreads),
+                             stream, p);
+    return launch_kernel(klp_grpo_step_kernel<DT, NV, false, kThreads>, grid, dim3(kThreads),
+                         stream, p);
 }
 
 template <int DT, int NV>
@@ -511,8 +525,37 @@ static int capacity(int64_t vocab) {
     return 0;
 }
 
+// Threads per row.  A workgroup reads its row, reduces it and writes it in
+// turn, so a CU overlaps those only between rows resident at once: more,
+// smaller workgroups, as long as each still has enough loads in flight.
+//  - Rows of up to 16 KB take 256 threads, up to 32 KB 512 (4 vectors each,
+//    where 1024 threads hold 1-2, idle from 1): bf16, us against 1024 threads,
+//    [8192, 4096] 26.3 / 49.4, [8192, 8192] 45.9 / 76.2, [64, 8192] 6.6 / 7.3,
+//    [2048, 12288] 20.6 / 23.9, [8192, 16384] 89.9 / 101.9, [512, 16384]
+//    7.8 / 9.1; fp32 [4096, 8192] 45.9 / 50.5.  Rows of 32 to 64 KB measured
+//    equal or slower with 256 or 512 ([8192, 32000] 181-186 / 178).
+//  - Rows of 64 to 152 KB take 512 threads when there are more rows than CUs
+//    and fewer than the persistent kernel wants: two rows a CU (128 VGPRs),
+//    where 1024 threads of 70 VGPRs and more fit one.  bf16 [300, 40000]
+//    13.1 / 15.6, [512, 50240] 18.6 / 22.4, [1552, 53440] 64.9 / 72.9, [512,
+//    77824] 27.1 / 31.9; [128, 50240], a row a CU, 10.6 / 9.7.  fp32 has half
+//    the arithmetic to hide: [512, 32000] 22.3 / 23.3, [512, 24576] 15.9 /
+//    18.5, but past 1024 rows of more than 96 KB 74.0 / 72.0 ([1552, 32000]).
+constexpr int64_t kCus = 256;
+
 template <int DT>
 static hipError_t launch_step_dt(const GrpoStepParams& p, hipStream_t stream) {
+    const int64_t nvec = p.vocab / Traits<DT>::kPerVec;
+    if (nvec <= 4 * 256) return launch_row<DT, 4, 256>(p, stream);
+    if (nvec <= 4 * 512) return launch_row<DT, 4, 512>(p, stream);
+    if (nvec > 8 * 512 && nvec <= kGrpoStepMaxVec * 512 && p.n_rows > kCus &&
+        p.n_rows < kPersistMinRowsPerWorkgroup * kCus) {
+        if (nvec <= 12 * 512) return launch_row<DT, 12, 512>(p, stream);
+        if (DT != kFP32 || p.n_rows <= 1024) {
+            if (nvec <= 16 * 512) return launch_row<DT, 16, 512>(p, stream);
+            return launch_row<DT, kGrpoStepMaxVec, 512>(p, stream);
+        }
+    }
     switch (capacity<DT>(p.vocab)) {
         case 4: return launch_step_nv<DT, 4>(p, stream);
         case 8: return launch_step_nv<DT, 8>(p, stream);

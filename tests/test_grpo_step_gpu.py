@@ -574,6 +574,54 @@ def test_persistent_rows_match_one_row_per_workgroup(dtype, B, S, V, temperature
             assert torch.equal(u.view(as_int), v.view(as_int)), name
 
 
+# Rows (in 16-byte vectors) and row counts at the edges of the dispatch: 256
+# threads up to 1024 vectors, 512 up to 2048, 1024 beyond; 512 again for 4097
+# .. 9728 vectors and 257 .. 2047 rows (12, 16 and 19 vectors a thread).
+@pytest.mark.parametrize("dtype,rows,nvec", [
+    (torch.bfloat16, 3, 1), (torch.bfloat16, 9, 255), (torch.float16, 5, 1024),
+    (torch.bfloat16, 7, 1025), (torch.float32, 6, 2048), (torch.bfloat16, 5, 2049),
+    (torch.bfloat16, 257, 4096), (torch.bfloat16, 256, 4097), (torch.bfloat16, 257, 4097),
+    (torch.float16, 300, 6144), (torch.bfloat16, 290, 6145), (torch.bfloat16, 300, 8192),
+    (torch.bfloat16, 260, 8193), (torch.float16, 258, 9728), (torch.bfloat16, 258, 9729),
+    (torch.float32, 1024, 6145), (torch.float32, 1025, 6145), (torch.float32, 1025, 6144),
+    (torch.bfloat16, 2047, 4100), (torch.bfloat16, 2048, 4100)])
+@pytest.mark.parametrize("temperature", [1.0, 0.7])
+def test_threads_per_row(dtype, rows, nvec, temperature):
+    """Every row length and count takes a kernel that gives the forward's
+    logp / entropy / lse (fp32 sums in another order) and, from its own lse,
+    the backward's d_logits bit for bit."""
+    from kernel_opt import _C
+    from kernel_opt._library import KLP_GRPO_STEP_SCHED_BYTES
+    V = nvec * 16 // torch.empty((), dtype=dtype).element_size()
+    g = torch.Generator(device=DEV).manual_seed(nvec)
+    x = (torch.randn(1, rows, V, generator=g, device=DEV) * 2.0).to(dtype)
+    if V > 64:
+        x[0, 1, ::5] = float("-inf")
+    t = torch.randint(0, V, (1, rows), generator=g, device=DEV)
+    t[0, 0], t[0, 2] = V - 1, IGNORE
+    outs = [torch.empty(1, rows, device=DEV) for _ in range(3)]
+    _C.fwd_launch(x, t, *outs, temperature=temperature)
+    # Ratios well inside the clip range, so that d loss / d logp is -w A ratio.
+    old = torch.where(torch.isfinite(outs[0]), outs[0], torch.zeros_like(outs[0])) - 0.05
+    adv = torch.randn(1, rows, generator=g, device=DEV)
+    w = torch.rand(1, rows, generator=g, device=DEV)
+    sched = torch.zeros(KLP_GRPO_STEP_SCHED_BYTES, dtype=torch.uint8, device=DEV)
+    lp, ent, lse, _, d = _step_abi(x, t, old, None, adv, w, temperature, 1, sched)
+    ok = torch.isfinite(outs[0])
+    assert ok.sum() >= rows - 1 and torch.equal(ok, torch.isfinite(lp))
+    for a, b in zip((lp, ent, lse), outs):
+        assert ((a - b)[ok].abs() <= 1e-5).all()
+    from kernel_opt import fused_grpo_loss
+    lpu = lp.detach().clone().requires_grad_(True)
+    loss, _ = fused_grpo_loss(lpu, old, adv, w, eps_low=0.2, eps_high=0.28, loss_type="dapo",
+                              normalizer=1.0)
+    loss.backward()
+    want = torch.empty_like(x)
+    _C.bwd_launch(x, t, lse, ent, lpu.grad, None, None, want, temperature=temperature)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    assert torch.equal(d[ok].view(bits), want[ok].view(bits))
+
+
 def test_persistent_rows_only_where_they_pay():
     """The persistent kernel is used for rows of 8 or more 16-byte vectors
     per thread (bf16 / fp16 V > 32768, fp32 V > 16384), from 8 rows per

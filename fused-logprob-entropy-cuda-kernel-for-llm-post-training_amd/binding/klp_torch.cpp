@@ -445,6 +445,17 @@ struct GrpoArgs {
     int64_t kind, level, per_token;
 };
 
+// The entry points' code of a bool or integer mask's dtype, or -1.
+int mask_dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kBool:
+        case at::kByte: return KLP_MASK_U8;
+        case at::kInt: return KLP_MASK_I32;
+        case at::kLong: return KLP_MASK_I64;
+        default: return -1;
+    }
+}
+
 class FusedGrpoLoss : public torch::autograd::Function<FusedGrpoLoss> {
    public:
     static variable_list forward(AutogradContext* ctx, const at::Tensor& logp, const at::Tensor& old,
@@ -454,7 +465,7 @@ class FusedGrpoLoss : public torch::autograd::Function<FusedGrpoLoss> {
                                  int64_t level, int64_t per_token) {
         const int64_t B = logp.size(0), S = logp.size(1);
         const at::Tensor lp = logp.contiguous();
-        const at::Tensor r = ref.value_or(at::Tensor()), m = mask.value_or(at::Tensor());
+        const at::Tensor r = ref.value_or(at::Tensor()), given = mask.value_or(at::Tensor());
         const auto f32 = at::TensorOptions().dtype(at::kFloat).device(logp.device());
         at::Tensor ws = at::empty({static_cast<int64_t>(klp_grpo_workspace_bytes(B))},
                                   f32.dtype(at::kByte));
@@ -464,12 +475,26 @@ class FusedGrpoLoss : public torch::autograd::Function<FusedGrpoLoss> {
         const c10::hip::HIPGuard guard(static_cast<c10::DeviceIndex>(dev));
         hipStream_t stream =
             c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
-        check_status(klp_grpo_fwd(fptr(lp), fptr(old), fptr(r), fptr(adv), fptr(m), B, S,
-                                  static_cast<float>(eps_low), static_cast<float>(eps_high),
-                                  static_cast<float>(beta), static_cast<float>(norm),
-                                  static_cast<int>(kind), static_cast<int>(level),
-                                  static_cast<int>(per_token), out_ptr(loss), out_ptr(stats),
-                                  ws.data_ptr(), static_cast<size_t>(ws.numel()), stream));
+        // A bool or integer mask is read as it is; the kernel leaves it in
+        // float32 for the backward.
+        const int code = given.defined() ? mask_dtype_code(given.scalar_type()) : -1;
+        at::Tensor m = given;
+        if (code >= 0) {
+            m = at::empty({B, S}, f32);
+            check_status(klp_grpo_fwd_masked(
+                fptr(lp), fptr(old), fptr(r), fptr(adv), given.data_ptr(), code, out_ptr(m), B, S,
+                static_cast<float>(eps_low), static_cast<float>(eps_high),
+                static_cast<float>(beta), static_cast<float>(norm), static_cast<int>(kind),
+                static_cast<int>(level), static_cast<int>(per_token), out_ptr(loss),
+                out_ptr(stats), ws.data_ptr(), static_cast<size_t>(ws.numel()), stream));
+        } else {
+            check_status(klp_grpo_fwd(
+                fptr(lp), fptr(old), fptr(r), fptr(adv), fptr(m), B, S,
+                static_cast<float>(eps_low), static_cast<float>(eps_high),
+                static_cast<float>(beta), static_cast<float>(norm), static_cast<int>(kind),
+                static_cast<int>(level), static_cast<int>(per_token), out_ptr(loss),
+                out_ptr(stats), ws.data_ptr(), static_cast<size_t>(ws.numel()), stream));
+        }
         ctx->save_for_backward({lp, old, r, adv, m, ws});
         ctx->saved_data["args"] = c10::List<double>({eps_low, eps_high, beta, norm,
                                                      static_cast<double>(kind),
@@ -531,7 +556,13 @@ std::vector<at::Tensor> fused_grpo_loss(const at::Tensor& logp, const std::optio
     const bool per_token = advantages.dim() != 1;
     const at::Tensor adv = per_token ? grpo_operand(advantages, "advantages", {B, S}, dev)
                                      : grpo_operand(advantages, "advantages", {B}, dev);
-    const at::Tensor m = grpo_operand(mask, "mask", {B, S}, dev);
+    // A bool or integer mask goes to the kernel as it is, any other in float32.
+    at::Tensor m;
+    if (mask.has_value() && mask->defined() && mask->device() == dev &&
+        mask->sizes() == at::IntArrayRef({B, S}) && mask_dtype_code(mask->scalar_type()) >= 0)
+        m = mask->detach().contiguous();
+    else
+        m = grpo_operand(mask, "mask", {B, S}, dev);
     const at::Tensor r = beta != 0.0 ? grpo_operand(ref, "ref_logp", {B, S}, dev) : at::Tensor();
     if (B == 0 || S == 0)  // no tokens: every normaliser sees an empty (zero) masked sum
         return {logp.sum() * 0.0, at::zeros({4}, logp.options())};
@@ -719,11 +750,7 @@ std::optional<std::vector<at::Tensor>> fused_grpo_step(
     // statement gives inf / negative weights).
     int mask_code = -1;
     if (has_mask) {
-        const auto st = m.scalar_type();
-        mask_code = (st == at::kBool || st == at::kByte) ? KLP_MASK_U8
-                    : st == at::kInt                     ? KLP_MASK_I32
-                    : st == at::kLong                    ? KLP_MASK_I64
-                                                         : -1;
+        mask_code = mask_dtype_code(m.scalar_type());
     }
     const float fixed_scale = static_cast<float>(weight_scale);
     const bool scale_ok = weight_kind != KLP_GRPO_LOSS_FIXED ||

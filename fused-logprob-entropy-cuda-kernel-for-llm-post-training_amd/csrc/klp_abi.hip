@@ -465,6 +465,8 @@ int grpo_setup(const float* logp, const float* old_logp, const float* ref_logp,
     p->ref_logp = ref_logp;
     p->adv = advantages;
     p->mask = mask;
+    p->mask_dtype = klp::kMaskF32;
+    p->mask_out = nullptr;
     p->B = n_seqs;
     p->S = seq_len;
     p->eps_low = eps_low;
@@ -805,6 +807,35 @@ int klp_grpo_fwd(const float* logp, const float* old_logp, const float* ref_logp
     if (rc != KLP_OK) return rc;
     if ((rc = check_f32(loss, "loss")) != KLP_OK) return rc;
     if (stats && (rc = check_f32(stats, "stats")) != KLP_OK) return rc;
+    p.loss = loss;
+    p.stats = stats;
+    if (injected_failure("grpo forward")) return KLP_ELAUNCH;
+    return after_launch(klp::launch_grpo_fwd(p, static_cast<hipStream_t>(stream)),
+                        "grpo forward");
+}
+
+int klp_grpo_fwd_masked(const float* logp, const float* old_logp, const float* ref_logp,
+                        const float* advantages, const void* mask, int mask_dtype,
+                        float* mask_out, int64_t n_seqs, int64_t seq_len, float eps_low,
+                        float eps_high, float beta, float norm_const, int loss_type, int level,
+                        int adv_per_token, float* loss, float* stats, void* workspace,
+                        size_t workspace_bytes, void* stream) {
+    klp::GrpoParams p;
+    int rc = grpo_setup(logp, old_logp, ref_logp, advantages, nullptr, n_seqs, seq_len, eps_low,
+                        eps_high, beta, norm_const, loss_type, level, adv_per_token, workspace,
+                        workspace_bytes, &p);
+    if (rc != KLP_OK) return rc;
+    if (mask_dtype != KLP_MASK_U8 && mask_dtype != KLP_MASK_I32 && mask_dtype != KLP_MASK_I64)
+        return fail(KLP_EDTYPE, "mask dtype must be KLP_MASK_U8, KLP_MASK_I32 or KLP_MASK_I64");
+    const size_t esz = mask_dtype == KLP_MASK_U8 ? 1 : mask_dtype == KLP_MASK_I32 ? 4 : 8;
+    if (mask == nullptr || !aligned(mask, esz))
+        return fail(KLP_EINVAL, "mask must be non-null and aligned to its element size");
+    if ((rc = check_f32(mask_out, "mask_out")) != KLP_OK) return rc;
+    if ((rc = check_f32(loss, "loss")) != KLP_OK) return rc;
+    if (stats && (rc = check_f32(stats, "stats")) != KLP_OK) return rc;
+    p.mask = mask;
+    p.mask_dtype = mask_dtype;
+    p.mask_out = mask_out;
     p.loss = loss;
     p.stats = stats;
     if (injected_failure("grpo forward")) return KLP_ELAUNCH;

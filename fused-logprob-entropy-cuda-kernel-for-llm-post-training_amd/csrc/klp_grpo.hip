@@ -19,9 +19,9 @@
 //
 // Launches: klp_grpo_rows_kernel (one workgroup per row: row sums into the
 // workspace), klp_grpo_finish_kernel (one workgroup: the batch sums in a
-// fixed order, the loss and statistics), klp_grpo_bwd_kernel (one workgroup
-// per row: the gradient, scaled by the upstream gradient of the loss).  All
-// reductions have a fixed order, so results do not depend on timing.
+// fixed order, the loss and statistics), klp_grpo_bwd_kernel (the gradient,
+// scaled by the upstream gradient of the loss).  All reductions have a fixed
+// order, so results do not depend on timing.
 #include <type_traits>
 
 #include "klp_grpo_terms.h"
@@ -32,10 +32,19 @@ namespace klp {
 namespace {
 
 constexpr int kGrpoThreads = 256;
-
-__device__ __forceinline__ float mask_at(const GrpoParams& p, int64_t i) {
-    return p.mask ? p.mask[i] : 1.0f;
-}
+// What bounds the loss is latency: launches, and in few long rows (one
+// workgroup a row, for sums in a fixed order) the chain of loads a thread
+// waits for.  So a thread loads kGrpoUnroll tokens before it uses any, rows of
+// more than kGrpoShortRow tokens, which would take a second such step with
+// kGrpoThreads, have kGrpoLongThreads, and a bool or integer mask is read as
+// it is instead of converted by a launch before.  Rows kernel and backward,
+// bool mask, us before -> after, with the conversion: [8, 512] 3.6 + 3.0 + 3.6
+// -> 4.3 + 3.2, [1, 4749] 9.8 + 7.5 + 3.6 -> 5.3 + 3.6, [64, 4096] 9.2 + 7.9 +
+// 3.9 -> 6.1 + 4.1; the call with its backward, which the host's launches
+// bound, 65.2 -> 61.4 at [8, 512].
+constexpr int kGrpoUnroll = 4;
+constexpr int kGrpoLongThreads = 1024;
+constexpr int64_t kGrpoShortRow = kGrpoThreads * kGrpoUnroll;
 
 __device__ __forceinline__ float adv_at(const GrpoParams& p, int64_t b, int64_t i) {
     return p.adv_per_token ? p.adv[i] : p.adv[b];
@@ -48,9 +57,9 @@ __device__ __forceinline__ TokenLoss token_loss(const GrpoParams& p, float w, fl
 
 // Block-wide sums of K values, fixed order (xor-shuffle tree within waves,
 // waves in order through LDS).  Every thread returns the totals.
-template <int K>
+template <int kThreads, int K>
 __device__ __forceinline__ void block_sum(float (&v)[K]) {
-    __shared__ float red[kGrpoThreads / 64][K];
+    __shared__ float red[kThreads / 64][K];
     __shared__ float tot[K];
 #pragma unroll
     for (int k = 0; k < K; ++k)
@@ -66,7 +75,7 @@ __device__ __forceinline__ void block_sum(float (&v)[K]) {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             float s = red[0][k];
-            for (int w = 1; w < kGrpoThreads / 64; ++w) s += red[w][k];
+            for (int w = 1; w < kThreads / 64; ++w) s += red[w][k];
             tot[k] = s;
         }
     }
@@ -76,17 +85,52 @@ __device__ __forceinline__ void block_sum(float (&v)[K]) {
     __syncthreads();
 }
 
+// A token's inputs.
+struct TokenIn {
+    float m, lp, lo, adv, lr;
+};
+
+// Calls use(i, token) for the tokens s = first, first + step, .. < end of row
+// b, in that order, the loads of kGrpoUnroll of them before the first use.
+template <typename Mask, typename Use>
+__device__ __forceinline__ void for_tokens(const GrpoParams& p, int64_t b, bool has_ref,
+                                           int64_t first, int64_t step, int64_t end, Use use) {
+    const int64_t base = b * p.S;
+    const Mask* mask = static_cast<const Mask*>(p.mask);
+    for (int64_t s0 = first; s0 < end; s0 += kGrpoUnroll * step) {
+        TokenIn t[kGrpoUnroll] = {};
+        Mask m[kGrpoUnroll] = {};
+#pragma unroll
+        for (int k = 0; k < kGrpoUnroll; ++k) {
+            const int64_t s = s0 + k * step;
+            if (s >= end) break;
+            const int64_t i = base + s;
+            m[k] = mask ? mask[i] : Mask{1};
+            t[k].lp = p.logp[i];
+            t[k].lo = p.old_logp[i];
+            t[k].adv = adv_at(p, b, i);
+            t[k].lr = has_ref ? p.ref_logp[i] : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < kGrpoUnroll; ++k) {
+            const int64_t s = s0 + k * step;
+            if (s >= end) break;
+            t[k].m = static_cast<float>(m[k]);
+            use(base + s, t[k]);
+        }
+    }
+}
+
 // The row's log importance weight at sequence level: masked mean of lp - lo.
+template <int kThreads, typename Mask>
 __device__ __forceinline__ void row_sequence_weight(const GrpoParams& p, int64_t b, float* w_row,
                                                     float* m_row) {
-    const int64_t base = b * p.S;
     float v[2] = {0.0f, 0.0f};
-    for (int64_t s = threadIdx.x; s < p.S; s += kGrpoThreads) {
-        const float m = mask_at(p, base + s);
-        v[0] += (p.logp[base + s] - p.old_logp[base + s]) * m;
-        v[1] += m;
-    }
-    block_sum<2>(v);
+    for_tokens<Mask>(p, b, false, threadIdx.x, kThreads, p.S, [&](int64_t, const TokenIn& t) {
+        v[0] += (t.lp - t.lo) * t.m;
+        v[1] += t.m;
+    });
+    block_sum<kThreads>(v);
     *m_row = v[1];
     *w_row = v[0] / fmaxf(v[1], 1.0f);
 }
@@ -98,27 +142,26 @@ __device__ __forceinline__ void row_sequence_weight(const GrpoParams& p, int64_t
 //   row b:  [0] sum loss*m  [1] sum m  [2] sum kl*m  [3] sum low*m
 //           [4] sum high*m
 //   tail :  [0] sum m over the batch
-__global__ __launch_bounds__(kGrpoThreads) void klp_grpo_rows_kernel(GrpoParams p) {
+// With p.mask_out the mask goes there in float32 (for the backward, which is
+// then independent of the caller's mask).
+template <int kThreads, typename Mask>
+__global__ __launch_bounds__(kThreads) void klp_grpo_rows_kernel(GrpoParams p) {
     const int64_t b = blockIdx.x;
-    const int64_t base = b * p.S;
     const bool has_ref = p.ref_logp != nullptr && p.beta != 0.0f;
     float w_row = 0.0f, m_row = 0.0f;
-    if (p.level == KLP_GRPO_SEQUENCE) row_sequence_weight(p, b, &w_row, &m_row);
+    if (p.level == KLP_GRPO_SEQUENCE) row_sequence_weight<kThreads, Mask>(p, b, &w_row, &m_row);
     float v[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t s = threadIdx.x; s < p.S; s += kGrpoThreads) {
-        const int64_t i = base + s;
-        const float m = mask_at(p, i);
-        const float lp = p.logp[i];
-        const float w = (p.level == KLP_GRPO_SEQUENCE) ? w_row : lp - p.old_logp[i];
-        const TokenLoss t = token_loss(p, w, adv_at(p, b, i), lp,
-                                       has_ref ? p.ref_logp[i] : 0.0f, has_ref);
-        v[0] += t.loss * m;
-        v[1] += m;
-        v[2] += t.kl * m;
-        v[3] += t.low * m;
-        v[4] += t.high * m;
-    }
-    block_sum<5>(v);
+    for_tokens<Mask>(p, b, has_ref, threadIdx.x, kThreads, p.S, [&](int64_t i, const TokenIn& in) {
+        const float w = (p.level == KLP_GRPO_SEQUENCE) ? w_row : in.lp - in.lo;
+        const TokenLoss t = token_loss(p, w, in.adv, in.lp, in.lr, has_ref);
+        if (p.mask_out) p.mask_out[i] = in.m;
+        v[0] += t.loss * in.m;
+        v[1] += in.m;
+        v[2] += t.kl * in.m;
+        v[3] += t.low * in.m;
+        v[4] += t.high * in.m;
+    });
+    block_sum<kThreads>(v);
     if (threadIdx.x == 0) {
         float* row = p.ws + b * kGrpoRowWords;
 #pragma unroll
@@ -141,7 +184,7 @@ __global__ __launch_bounds__(kGrpoThreads) void klp_grpo_finish_kernel(GrpoParam
         v[4] += row[3];
         v[5] += row[4];
     }
-    block_sum<6>(v);
+    block_sum<kGrpoThreads>(v);
     if (threadIdx.x != 0) return;
     float loss;
     if (p.loss_type == KLP_GRPO_LOSS_GRPO) loss = v[0] / static_cast<float>(p.B);
@@ -160,9 +203,11 @@ __global__ __launch_bounds__(kGrpoThreads) void klp_grpo_finish_kernel(GrpoParam
 
 // d loss / d lp for every token, times the upstream gradient of the loss
 // (a device scalar, or 1 when null).  Reads the row sums of the forward.
-__global__ __launch_bounds__(kGrpoThreads) void klp_grpo_bwd_kernel(GrpoParams p) {
+// Token level: pieces of kThreads * kGrpoUnroll tokens of the row, dealt over
+// blockIdx.y; sequence level: one workgroup a row.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void klp_grpo_bwd_kernel(GrpoParams p) {
     const int64_t b = blockIdx.x;
-    const int64_t base = b * p.S;
     const bool has_ref = p.ref_logp != nullptr && p.beta != 0.0f;
     const float g = p.grad_loss ? p.grad_loss[0] : 1.0f;
     // Weight of a token's loss in the batch loss, per unit mask.
@@ -179,34 +224,28 @@ __global__ __launch_bounds__(kGrpoThreads) void klp_grpo_bwd_kernel(GrpoParams p
         // Every token shares w = sum_s (lp - lo) m / max(sum m, 1): the
         // ratio term's gradient is (sum_s' scale m_s' dw_s') * m_s / max(sum m, 1).
         float w_row, m_row;
-        row_sequence_weight(p, b, &w_row, &m_row);
+        row_sequence_weight<kThreads, float>(p, b, &w_row, &m_row);
         float v[1] = {0.0f};
-        for (int64_t s = threadIdx.x; s < p.S; s += kGrpoThreads) {
-            const int64_t i = base + s;
-            const float m = mask_at(p, i);
-            const TokenLoss t = token_loss(p, w_row, adv_at(p, b, i), p.logp[i],
-                                           has_ref ? p.ref_logp[i] : 0.0f, has_ref);
-            v[0] += t.dw * m;
-        }
-        block_sum<1>(v);
+        for_tokens<float>(p, b, has_ref, threadIdx.x, kThreads, p.S, [&](int64_t, const TokenIn& in) {
+            v[0] += token_loss(p, w_row, in.adv, in.lp, in.lr, has_ref).dw * in.m;
+        });
+        block_sum<kThreads>(v);
         const float row_term = v[0] * scale / fmaxf(m_row, 1.0f);
-        for (int64_t s = threadIdx.x; s < p.S; s += kGrpoThreads) {
-            const int64_t i = base + s;
-            const float m = mask_at(p, i);
-            const TokenLoss t = token_loss(p, w_row, adv_at(p, b, i), p.logp[i],
-                                           has_ref ? p.ref_logp[i] : 0.0f, has_ref);
-            p.d_logp[i] = row_term * m + t.dlp * m * scale;
-        }
+        for_tokens<float>(p, b, has_ref, threadIdx.x, kThreads, p.S, [&](int64_t i, const TokenIn& in) {
+            const TokenLoss t = token_loss(p, w_row, in.adv, in.lp, in.lr, has_ref);
+            p.d_logp[i] = row_term * in.m + t.dlp * in.m * scale;
+        });
         return;
     }
-    for (int64_t s = threadIdx.x; s < p.S; s += kGrpoThreads) {
-        const int64_t i = base + s;
-        const float m = mask_at(p, i);
-        const float lp = p.logp[i];
-        const TokenLoss t = token_loss(p, lp - p.old_logp[i], adv_at(p, b, i), lp,
-                                       has_ref ? p.ref_logp[i] : 0.0f, has_ref);
-        p.d_logp[i] = (t.dw + t.dlp) * m * scale;
-    }
+    constexpr int64_t kSpan = kThreads * kGrpoUnroll;
+    for (int64_t first = blockIdx.y * kSpan; first < p.S; first += gridDim.y * kSpan)
+        for_tokens<float>(p, b, has_ref, first + threadIdx.x, kThreads,
+                          first + kSpan < p.S ? first + kSpan : p.S,
+                          [&](int64_t i, const TokenIn& in) {
+                              const TokenLoss t = token_loss(p, in.lp - in.lo, in.adv, in.lp,
+                                                             in.lr, has_ref);
+                              p.d_logp[i] = (t.dw + t.dlp) * in.m * scale;
+                          });
 }
 
 namespace {
@@ -415,15 +454,38 @@ hipError_t launch_grpo_token_weights(const TokenWeightsParams& p, hipStream_t st
     }
 }
 
+template <typename Mask>
+static hipError_t launch_grpo_rows(const GrpoParams& p, hipStream_t stream) {
+    const dim3 rows(static_cast<unsigned>(p.B));
+    return p.S <= kGrpoShortRow
+               ? launch_kernel(klp_grpo_rows_kernel<kGrpoThreads, Mask>, rows, dim3(kGrpoThreads),
+                               stream, p)
+               : launch_kernel(klp_grpo_rows_kernel<kGrpoLongThreads, Mask>, rows,
+                               dim3(kGrpoLongThreads), stream, p);
+}
+
 hipError_t launch_grpo_fwd(const GrpoParams& p, hipStream_t stream) {
-    hipError_t e = launch_kernel(klp_grpo_rows_kernel, dim3(static_cast<unsigned>(p.B)),
-                                 dim3(kGrpoThreads), stream, p);
+    const hipError_t e = p.mask_dtype == KLP_MASK_U8    ? launch_grpo_rows<uint8_t>(p, stream)
+                         : p.mask_dtype == KLP_MASK_I32 ? launch_grpo_rows<int32_t>(p, stream)
+                         : p.mask_dtype == KLP_MASK_I64 ? launch_grpo_rows<int64_t>(p, stream)
+                                                        : launch_grpo_rows<float>(p, stream);
     if (e != hipSuccess) return e;
     return launch_kernel(klp_grpo_finish_kernel, dim3(1), dim3(kGrpoThreads), stream, p);
 }
 
 hipError_t launch_grpo_bwd(const GrpoParams& p, hipStream_t stream) {
-    return launch_kernel(klp_grpo_bwd_kernel, dim3(static_cast<unsigned>(p.B)),
+    const unsigned rows = static_cast<unsigned>(p.B);
+    if (p.level == KLP_GRPO_SEQUENCE)
+        return p.S <= kGrpoShortRow
+                   ? launch_kernel(klp_grpo_bwd_kernel<kGrpoThreads>, dim3(rows),
+                                   dim3(kGrpoThreads), stream, p)
+                   : launch_kernel(klp_grpo_bwd_kernel<kGrpoLongThreads>, dim3(rows),
+                                   dim3(kGrpoLongThreads), stream, p);
+    const int64_t span = int64_t{kGrpoThreads} * kGrpoUnroll;
+    const int64_t pieces = p.S < 1 ? 1 : (p.S + span - 1) / span;
+    // 65535: the grid's second dimension; longer rows loop.
+    return launch_kernel(klp_grpo_bwd_kernel<kGrpoThreads>,
+                         dim3(rows, static_cast<unsigned>(pieces < 65535 ? pieces : 65535)),
                          dim3(kGrpoThreads), stream, p);
 }
 

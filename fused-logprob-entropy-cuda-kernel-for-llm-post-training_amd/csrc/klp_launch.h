@@ -111,7 +111,9 @@ struct GrpoParams {
     const float* old_logp;
     const float* ref_logp;   // nullable
     const float* adv;        // [B], or [B, S] when adv_per_token
-    const float* mask;       // nullable (all ones)
+    const void* mask;        // nullable (all ones), of mask_dtype
+    int mask_dtype;          // KLP_MASK_U8 / _I32 / _I64, or kMaskF32
+    float* mask_out;         // forward: the mask in float32, nullable
     int64_t B;
     int64_t S;
     float eps_low;
@@ -127,6 +129,7 @@ struct GrpoParams {
     const float* grad_loss;  // backward: device scalar, nullable (1)
     float* d_logp;           // backward: [B, S]
 };
+constexpr int kMaskF32 = -1;
 // Workspace words per row of the GRPO loss (5 used, padded).
 constexpr int kGrpoRowWords = 8;
 

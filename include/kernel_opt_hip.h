@@ -294,6 +294,18 @@ int klp_grpo_fwd(const float* logp, const float* old_logp, const float* ref_logp
                  void* workspace, size_t workspace_bytes,
                  void* stream);
 
+/* klp_grpo_fwd for a bool / uint8, int32 or int64 mask (KLP_MASK_U8 / _I32 /
+ * _I64, below), which it reads as it is and writes to `mask_out` (float32
+ * [n_seqs, seq_len]): the mask klp_grpo_bwd then takes. */
+int klp_grpo_fwd_masked(const float* logp, const float* old_logp, const float* ref_logp,
+                        const float* advantages, const void* mask, int mask_dtype,
+                        float* mask_out, int64_t n_seqs, int64_t seq_len,
+                        float eps_low, float eps_high, float beta, float norm_const,
+                        int loss_type, int level, int adv_per_token,
+                        float* loss, float* stats,
+                        void* workspace, size_t workspace_bytes,
+                        void* stream);
+
 int klp_grpo_bwd(const float* logp, const float* old_logp, const float* ref_logp,
                  const float* advantages, const float* mask,
                  int64_t n_seqs, int64_t seq_len,

@@ -141,3 +141,33 @@ def test_invalid_arguments_raise():
         fused_grpo_loss(lp, lp, adv, loss_type="dapo")
     with pytest.raises(RuntimeError, match="shape"):
         fused_grpo_loss(lp, lp[:1], adv)
+
+
+@pytest.mark.parametrize("dtype", [torch.bool, torch.uint8, torch.int32, torch.int64])
+@pytest.mark.parametrize("level", ["token", "sequence"])
+@pytest.mark.parametrize("B,S", [(3, 1), (2, 255), (3, 1024), (2, 1025), (1, 4749)])
+def test_integer_masks_match_float_bitwise(B, S, level, dtype):
+    """A bool or integer mask, read as it is, gives the float32 mask's loss,
+    statistics and gradient exactly, on both sides of the row length where
+    the threads per row change; its values need not be 0 and 1, and it need
+    not be contiguous.  Changing it after the forward changes nothing."""
+    from kernel_opt import fused_grpo_loss
+    new, old, ref, adv, mask = case(B, S, 11, adv_per_token=True)
+    t = lambda a: torch.tensor(a, device=DEV)
+    top = 1 if dtype == torch.bool else 3
+    m = t(mask) * torch.randint(1, top + 1, (B, S), device=DEV)
+    strided = torch.empty(S, B, dtype=dtype, device=DEV).t().copy_(m)
+
+    def go(m):
+        lp = torch.tensor(new, device=DEV, requires_grad=True)
+        loss, stats = fused_grpo_loss(lp, t(old), t(adv), m, t(ref), beta=0.04,
+                                      importance_level=level)
+        if m is strided:
+            m.zero_()
+        loss.backward()
+        return loss.detach(), stats, lp.grad
+
+    expect = go(m)
+    for given in (m.to(dtype), strided):
+        for a, b in zip(go(given), expect):
+            assert torch.equal(a, b)

@@ -484,29 +484,47 @@ int grpo_setup(const float* logp, const float* old_logp, const float* ref_logp,
     return KLP_OK;
 }
 
-// Fused LM head: vocab tiles per workgroup chunk.  A CU holds one workgroup,
-// so the launch takes (rounds of 256 workgroups) * (tiles per workgroup) tile
-// times, plus each round's prologue and merge (about 1/8 of a tile time at
-// dim 3584); of 1..16 tiles the count with the least of that is taken, the
-// fewest tiles on a tie.  1024 tokens of [152064, 3584]: 5 tiles (2 rounds)
-// 828-840 us, 2 tiles (5 rounds) 848-862, 3 tiles (4 rounds, 12 tile times
-// for 9.3 tiles of work per CU) 957, main loop alone.
-void lmh_plan(int64_t n_tokens, int64_t vocab, int64_t* tiles_per_chunk, int64_t* n_chunks) {
+// Fused LM head: tokens per workgroup and vocab tiles per workgroup chunk.  A
+// CU holds one workgroup, so the launch takes (rounds of 256 workgroups) *
+// (tiles per workgroup) tile times, plus each round's prologue and merge
+// (about 1/8 of a tile time at dim 3584); of 256 and 128 tokens and 1..16
+// tiles the pair with the least of that is taken, 256 tokens and the fewest
+// tiles on a tie.  1024 tokens of [152064, 3584]: 5 tiles (2 rounds) 828-840
+// us, 2 tiles (5 rounds) 848-862, 3 tiles (4 rounds, 12 tile times for 9.3
+// tiles of work per CU) 957, main loop alone.  A tile of 128 tokens takes 5/8
+// of one of 256 (1024 tokens as 8 blocks of 128: 980 us against 794; the
+// weight rows are read from LDS for half as many MFMAs).  Forward, us, 256 /
+// 128 tokens a workgroup:
+//   N     [152064, 3584]  [50240, 2048]  [32000, 4096]  [16384, 512]
+//   16    232 / 191       52 / 39        79 / 53        22 / 22
+//   128   238 / 209       53 / 41        79 / 61        24 / 23
+//   200   259 / 278       52 / 55        80 / 62        24 / 23
+//   320   395 / 399       89 / 77        94 / 100       24 / 23
+//   512   424 / 517       97 / 103       101 / 112      24 / 23
+//   1280                  209 / 231      250 / 286      38 / 33
+struct LmhPlan {
+    int block_tokens;
+    int64_t tiles_per_chunk;
+    int64_t n_chunks;
+};
+LmhPlan lmh_plan(int64_t n_tokens, int64_t vocab) {
     constexpr int64_t kCus = 256;
-    const int64_t tb = klp::lmh_token_blocks(n_tokens);
     const int64_t vt = klp::lmh_vocab_tiles(vocab);
-    int64_t best = 1, best_cost = INT64_MAX;
-    for (int64_t tpc = 1; tpc <= 16 && tpc <= vt; ++tpc) {
-        const int64_t chunks8 = ((vt + tpc - 1) / tpc + 7) / 8 * 8;
-        const int64_t rounds = (chunks8 * tb + kCus - 1) / kCus;
-        const int64_t cost = rounds * (8 * tpc + 1);
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = tpc;
+    LmhPlan best{256, 1, vt};
+    int64_t best_cost = INT64_MAX;
+    for (int block : {256, 128}) {
+        const int64_t tb = (n_tokens + block - 1) / block;
+        for (int64_t tpc = 1; tpc <= 16 && tpc <= vt; ++tpc) {
+            const int64_t n_chunks = (vt + tpc - 1) / tpc;
+            const int64_t rounds = ((n_chunks + 7) / 8 * 8 * tb + kCus - 1) / kCus;
+            const int64_t cost = rounds * ((block == 256 ? 8 : 5) * tpc + 1);
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = LmhPlan{block, tpc, n_chunks};
+            }
         }
     }
-    *tiles_per_chunk = best;
-    *n_chunks = (vt + best - 1) / best;
+    return best;
 }
 
 // The chunks' partial states, then the target logits.
@@ -516,9 +534,7 @@ size_t lmh_partials_bytes(int64_t n_tokens, int64_t n_chunks) {
 
 size_t lmh_workspace_bytes(int64_t n_tokens, int64_t vocab) {
     if (n_tokens <= 0 || vocab <= 0) return 0;
-    int64_t tpc, nc;
-    lmh_plan(n_tokens, vocab, &tpc, &nc);
-    return lmh_partials_bytes(n_tokens, nc) + static_cast<size_t>(n_tokens) * sizeof(float);
+    return lmh_partials_bytes(n_tokens, lmh_plan(n_tokens, vocab).n_chunks) + static_cast<size_t>(n_tokens) * sizeof(float);
 }
 
 // The LM head's backward products: 256 x 256 tiles, one workgroup per CU.
@@ -1190,9 +1206,12 @@ int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
     p->dim = dim;
     p->targets = targets;
     p->scale = scale;
-    p->n_tblocks = klp::lmh_token_blocks(n_tokens);
+    const LmhPlan plan = lmh_plan(n_tokens, vocab);
+    p->block_tokens = plan.block_tokens;
+    p->n_tblocks = (n_tokens + plan.block_tokens - 1) / plan.block_tokens;
     p->n_vtiles = klp::lmh_vocab_tiles(vocab);
-    lmh_plan(n_tokens, vocab, &p->tiles_per_chunk, &p->n_chunks);
+    p->tiles_per_chunk = plan.tiles_per_chunk;
+    p->n_chunks = plan.n_chunks;
     const int64_t blocks = (p->n_chunks + 7) / 8 * 8 * p->n_tblocks;
     if (blocks > (int64_t{1} << 31) - 1)
         return fail(KLP_EINVAL, "grid of %lld workgroups is too large",

@@ -220,7 +220,8 @@ struct LmhParams {
     float scale;             // 1 / temperature
     float* partials;         // [n_chunks, n_tokens] float4 (m, z, t, unused)
     float* target_logit;     // [n_tokens], behind the partials; written where a target is valid
-    int64_t n_tblocks;       // ceil(n_tokens / 256)
+    int block_tokens;        // tokens per workgroup: 256 or 128
+    int64_t n_tblocks;       // ceil(n_tokens / block_tokens)
     int64_t n_vtiles;        // ceil(vocab / 256)
     int64_t tiles_per_chunk;
     int64_t n_chunks;        // ceil(n_vtiles / tiles_per_chunk)
@@ -240,7 +241,6 @@ struct LmhParams {
     int64_t n_out;
     int out_align;
 };
-int64_t lmh_token_blocks(int64_t n_tokens);
 int64_t lmh_vocab_tiles(int64_t vocab);
 // `rounded`: logits rounded once to `dtype` (bf16 or fp16); otherwise bf16
 // operands and float32 logits.

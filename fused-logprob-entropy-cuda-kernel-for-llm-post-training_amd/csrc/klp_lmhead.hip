@@ -12,7 +12,9 @@
 // klp_lmh_kernel, forward (kFold): one workgroup (4 waves, 2 x 2) per (token block of
 // 256, vocab chunk of `tiles_per_chunk` tiles of 256 rows).  Per vocab tile
 // it computes the 256 x 256 block of logits^T with v_mfma_f32_16x16x32_bf16,
-// each wave a 128 x 128 part of it (64 accumulator blocks, 256 AGPRs):
+// each wave a 128 x 128 part of it (64 accumulator blocks, 256 AGPRs).  Where
+// that leaves less for the matrix cores to do (few tokens, or a remainder
+// block that would be mostly padding) token blocks of 128, a wave 128 x 64:
 //  - the transposed orientation puts vocab rows on the MFMA's M side, so a
 //    lane's accumulators belong to 8 tokens, 32 vocab rows of each: the
 //    online softmax update runs lane-locally, with no cross-lane reduction
@@ -41,8 +43,9 @@
 //    tokens whose target lies in the tile look for it.
 // At the end of the chunk the four lanes of a token and the two waves of a
 // token half merge; the chunk's partial state per token goes to the
-// workspace, and a target's logit straight from the lane that holds it.  klp_lmh_combine_kernel merges the chunks of each token (one
-// wave per token, a fixed order) and applies the output formulas.
+// workspace, and a target's logit straight from the lane that holds it.
+// klp_lmh_combine_kernel merges the chunks of each token (one wave per token,
+// a fixed order) and applies the output formulas.
 //
 // The backward (kGradient) runs the same tiles and replaces the fold with the
 // gradient of klp_bwd, written to d_logits; kLogits writes the logits.
@@ -53,7 +56,9 @@
 // takes 550-600 us).  The launch pair takes 800 us (1396 TFLOP/s) end to end,
 // where 64-byte stages, 32x32x16 MFMAs and a fold that compared every element
 // with the target took 1239.  32x32x16 MFMAs at this tile and ring: 840-848
-// us against 797-821 for the main loop alone, at 1.62 against 1.85 GHz.
+// us against 797-821 for the main loop alone, at 1.62 against 1.85 GHz.  Up
+// to 128 tokens the weight's bytes bound it: 16 tokens 191 us (5.7 TB/s) with
+// blocks of 128, 232 with blocks of 256.
 //
 // Workgroup order: workgroup b runs on XCD b % 8 (round-robin dispatch).
 // Consecutive workgroups of one XCD take the token blocks of one vocab
@@ -69,7 +74,6 @@ namespace {
 using namespace mfma;
 
 constexpr int kBV = kTile;  // vocab rows per tile
-constexpr int kBT = kTile;  // tokens per block
 
 enum : int { kFold = 0, kGradient = 1, kLogits = 2 };
 
@@ -80,10 +84,19 @@ enum : int { kFold = 0, kGradient = 1, kLogits = 2 };
 // klp_bwd (grad_one, klp_device.h) and written in DT; kLogits: the logits
 // themselves, rounded to DT (kRound, not scaled).  kRound: each logit is
 // rounded to DT before it is scaled and used, as a GEMM that writes DT does.
-template <int DT, int kMode, bool kRound, bool kScaled>
+// kTokBlocks: 16-token blocks per wave, 8 or 4 (256 or 128 tokens a workgroup).
+template <int DT, int kMode, bool kRound, bool kScaled, int kTokBlocks>
 __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
-    // The rings take all 160 KB of LDS; the end-of-chunk merge reuses them.
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[kLdsBytes];
+    constexpr int kTokSide = 16 * kTokBlocks;  // a wave's tokens
+    constexpr int kBT = 2 * kTokSide;          // the workgroup's
+    constexpr int kTokSlot = kBT * kRowBytes;
+    constexpr int kTokRing = kASlots * kSlotBytes;  // LDS offset of the hidden rows' ring
+    // MFMAs per half stage, and between two of its 8 weight copies.
+    constexpr int kSteps = kBlocks * kTokBlocks;
+    constexpr int kCopyStep = kSteps / 2 / kCopies;
+    // The rings (with 8 token blocks all 160 KB of LDS); the end-of-chunk
+    // merge reuses them.
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kTokRing + kBSlots * kTokSlot];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -116,17 +129,17 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     const uint32_t h_off = static_cast<uint32_t>(crow * p.ld_hidden * 2 + cchunk * 16);
     const uint32_t w_step = static_cast<uint32_t>(p.ld_weight * 64);  // 32 rows
     const uint32_t h_step = static_cast<uint32_t>(p.ld_hidden * 64);
-    auto rows_rsrc = [](const uint16_t* base, int64_t rows, int64_t ld) {
+    auto rows_rsrc = [](const uint16_t* base, int64_t rows, int64_t ld, int64_t most) {
         return __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint16_t*>(base), 0,
-            static_cast<int>((rows < 256 ? rows : 256) * ld * 2), 0x00020000);
+            static_cast<int>((rows < most ? rows : most) * ld * 2), 0x00020000);
     };
     const __amdgpu_buffer_rsrc_t h_rs =
-        rows_rsrc(p.hidden + tok0 * p.ld_hidden, p.n_tokens - tok0, p.ld_hidden);
+        rows_rsrc(p.hidden + tok0 * p.ld_hidden, p.n_tokens - tok0, p.ld_hidden, kBT);
     auto tile_rsrc = [&](int64_t vt) {
         const bool more = vt < tile_end;
         const int64_t v0 = (more ? vt : tile_first) * kBV;
-        return rows_rsrc(p.weight + v0 * p.ld_weight, more ? p.vocab - v0 : 0, p.ld_weight);
+        return rows_rsrc(p.weight + v0 * p.ld_weight, more ? p.vocab - v0 : 0, p.ld_weight, kBV);
     };
     // The stages to be copied next, and their slots.
     int64_t w_tile = tile_first;
@@ -146,9 +159,9 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     };
     auto copy_h = [&](int j) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            h_rs, (lds_void*)(lds + (kASlots + h_slot) * kSlotBytes + (wave + 4 * j) * 1024), 16,
+            h_rs, (lds_void*)(lds + kTokRing + h_slot * kTokSlot + (wave + 4 * j) * 1024), 16,
             h_off, j * h_step + h_k * kRowBytes, 0, 0);
-        if (j == kCopies - 1) {
+        if (j == kTokBlocks - 1) {
             if (++h_k == n_k) h_k = 0;
             h_slot ^= 1;
         }
@@ -167,17 +180,17 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
                                                 (((4 * half) ^ (lq ^ lf)) << 4) + i * 16 * kRowBytes);
     };
     auto h_src = [&](int half, int i) {
-        return *reinterpret_cast<const operand*>(lds + (kASlots + rh_slot) * kSlotBytes +
-                                                wt * (kSlotBytes / 2) + lrow * kRowBytes +
+        return *reinterpret_cast<const operand*>(lds + kTokRing + rh_slot * kTokSlot +
+                                                wt * (kTokSlot / 2) + lrow * kRowBytes +
                                                 (((4 * half) ^ (lq ^ lf)) << 4) + i * 16 * kRowBytes);
     };
 
-    // The lane's 8 tokens: block b's is tok0 + wt * 128 + 16 b + l % 16.
-    const int64_t my_tok = tok0 + wt * kWaveSide + lrow;
-    Stat st[kBlocks];
-    int my_tgt[kBlocks];  // vocab and n_tokens are below 2^31
+    // The lane's tokens: block b's is tok0 + wt * kTokSide + 16 b + l % 16.
+    const int64_t my_tok = tok0 + wt * kTokSide + lrow;
+    Stat st[kTokBlocks];
+    int my_tgt[kTokBlocks];  // vocab and n_tokens are below 2^31
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b) {
+    for (int b = 0; b < kTokBlocks; ++b) {
         st[b] = stat_empty();
         const int64_t tok = my_tok + 16 * b;
         const int64_t t = kMode != kLogits && tok < p.n_tokens ? p.targets[tok] - p.target_offset : -1;
@@ -190,36 +203,36 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
 #pragma unroll
     for (int j = 0; j < kCopies; ++j) copy_w(j);
 #pragma unroll
-    for (int j = 0; j < kCopies; ++j) copy_h(j);
+    for (int j = 0; j < kTokBlocks; ++j) copy_h(j);
 #pragma unroll
     for (int j = 0; j < kCopies; ++j) copy_w(j);
 #pragma unroll
-    for (int j = 0; j < kCopies; ++j) copy_h(j);
+    for (int j = 0; j < kTokBlocks; ++j) copy_h(j);
     pin();
-    __builtin_amdgcn_s_waitcnt(waitcnt(2 * kCopies, 15));
+    __builtin_amdgcn_s_waitcnt(waitcnt(kCopies + kTokBlocks, 15));
     __builtin_amdgcn_s_barrier();
     pin();
-    // Half a stage ahead: all 8 blocks of the token side (two sets, in turn)
+    // Half a stage ahead: all blocks of the token side (two sets, in turn)
     // and blocks 0..3 of the vocab side; its blocks 4..7 are read under the
     // MFMAs of 0..3.
-    operand aw[kBlocks], bh[2][kBlocks];
+    operand aw[kBlocks], bh[2][kTokBlocks];
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) bh[0][i] = h_src(0, i);
+    for (int i = 0; i < kTokBlocks; ++i) bh[0][i] = h_src(0, i);
 #pragma unroll
     for (int i = 0; i < 4; ++i) aw[i] = w_src(0, i);
 
     for (int64_t vt = tile_first; vt < tile_end; ++vt) {
-        f32x4 acc[kBlocks][kBlocks];
-        // One stage: 2 x 64 MFMAs, its copies and operand reads placed
+        f32x4 acc[kBlocks][kTokBlocks];
+        // One stage: 2 x kSteps MFMAs, its copies and operand reads placed
         // between them by hand.
         auto stage = [&](auto first_tag) {
             constexpr bool kFirst = decltype(first_tag)::value;
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
 #pragma unroll
-                for (int i = 0; i < 64; ++i) {
-                    const int a = i >> 3, b = i & 7;
-                    if (q == 1 && i == 32) {
+                for (int i = 0; i < kSteps; ++i) {
+                    const int a = i / kTokBlocks, b = i % kTokBlocks;
+                    if (q == 1 && i == kSteps / 2) {
                         // This wave has read all of the stage, and its copies of
                         // the next one have landed (in flight, at most: the 8
                         // weight copies after those).  After the barrier so for
@@ -233,13 +246,14 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
                         rh_slot ^= 1;
                     }
                     mul_add<DT>(acc[a][b], aw[a], bh[q][b], kFirst && q == 0);
-                    if (i < 32) {
-                        if ((i & 7) == 3) aw[4 + a] = w_src(q, 4 + a);
-                        if (q == 0 && (i & 3) == 2) copy_w(i >> 2);
+                    if (i < kSteps / 2) {
+                        if (b == kTokBlocks / 2 - 1) aw[4 + a] = w_src(q, 4 + a);
+                        if (q == 0 && i % kCopyStep == kCopyStep / 2) copy_w(i / kCopyStep);
                     } else {
-                        if ((i & 3) == 1) bh[q ^ 1][(i - 32) >> 2] = h_src(q ^ 1, (i - 32) >> 2);
-                        if ((i & 7) == 7) aw[a - 4] = w_src(q ^ 1, a - 4);
-                        if (q == 1 && (i & 3) == 2) copy_h((i - 32) >> 2);
+                        const int n = (i - kSteps / 2) / 4;
+                        if (i % 4 == 1) bh[q ^ 1][n] = h_src(q ^ 1, n);
+                        if (b == kTokBlocks - 1) aw[a - 4] = w_src(q ^ 1, a - 4);
+                        if (q == 1 && i % 4 == 2) copy_h(n);
                     }
                     pin();
                 }
@@ -278,7 +292,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
             RowGrad rg[kBlocks];
             if constexpr (kMode == kGradient) {
 #pragma unroll
-                for (int b = 0; b < kBlocks; ++b) {
+                for (int b = 0; b < kTokBlocks; ++b) {
                     const int64_t tok = my_tok + 16 * b;
                     const bool ok = tok < p.n_tokens;
                     rg[b] = ok ? row_grad(p.saved_lse[tok], p.saved_entropy[tok],
@@ -292,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
             const int64_t out_left = p.n_out - v0;
             const int olim = out_left < kBV ? static_cast<int>(out_left) : kBV;
 #pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
+            for (int b = 0; b < kTokBlocks; ++b) {
                 const int64_t tok = my_tok + 16 * b;
                 const bool ok = tok < p.n_tokens;
                 uint16_t* out = p.out + tok * p.ld_out + v0 + wv * kWaveSide;
@@ -343,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
         // The target logits the lane holds: of every 16 rows from row0, 0..3.
         const int first = static_cast<int>(v0) + row0;
 #pragma unroll
-        for (int b = 0; b < kBlocks; ++b) {
+        for (int b = 0; b < kTokBlocks; ++b) {
             const int target = my_tgt[b] - first;
             const bool mine = static_cast<uint32_t>(target) < static_cast<uint32_t>(kWaveSide) &&
                               (target & 15) < 4;
@@ -361,7 +375,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
         }
         if (vlim < kBV) {
 #pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
+            for (int b = 0; b < kTokBlocks; ++b) {
                 // Recomputed per token: the 32 lane masks of the comparisons
                 // below would otherwise be kept, and spilled.
                 int last = vlim - row0;
@@ -379,7 +393,7 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
             }
         } else {
 #pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
+            for (int b = 0; b < kTokBlocks; ++b) {
                 const Stat before = st[b];
                 float x[32];
 #pragma unroll
@@ -410,20 +424,19 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     __syncthreads();
     Stat (*merge_stat)[kBT] = reinterpret_cast<Stat (*)[kBT]>(lds);
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b) {
+    for (int b = 0; b < kTokBlocks; ++b) {
         st[b] = combine(st[b], stat_shfl_xor(st[b], 16));
         st[b] = combine(st[b], stat_shfl_xor(st[b], 32));
-        if (lane < 16) merge_stat[wv][wt * kWaveSide + 16 * b + lane] = st[b];
+        if (lane < 16) merge_stat[wv][wt * kTokSide + 16 * b + lane] = st[b];
     }
     __syncthreads();
     const int64_t n = tok0 + tid;
-    if (n < p.n_tokens) {
+    if (tid < kBT && n < p.n_tokens) {
         const Stat s = combine(merge_stat[0][tid], merge_stat[1][tid]);
         float4* slot = reinterpret_cast<float4*>(p.partials) + chunk * p.n_tokens + n;
         *slot = make_float4(s.m, s.z, s.t, 0.0f);
     }
 }
-#undef KLP_PIN
 
 // One wave per token: lane l merges chunks l, l + 64, l + 128, ... in order,
 // the lanes then merge in the fixed xor-butterfly order of wave_reduce (so the
@@ -450,21 +463,27 @@ __global__ __launch_bounds__(256) void klp_lmh_combine_kernel(LmhParams p) {
     p.lse[n] = o.lse;
 }
 
-int64_t lmh_token_blocks(int64_t n_tokens) { return (n_tokens + kBT - 1) / kBT; }
 int64_t lmh_vocab_tiles(int64_t vocab) { return (vocab + kBV - 1) / kBV; }
 
-template <int DT, int kMode, bool kRound>
-static hipError_t launch_lmh_t(const LmhParams& p, hipStream_t stream) {
+template <int DT, int kMode, bool kRound, bool kScaled>
+static hipError_t launch_lmh_s(const LmhParams& p, hipStream_t stream) {
     // Round the chunk count up to a multiple of 8 (one per XCD per round);
     // padding workgroups exit at once.
     const int64_t chunks8 = (p.n_chunks + 7) / 8 * 8;
     const dim3 grid(static_cast<unsigned>(chunks8 * p.n_tblocks));
+    if (p.block_tokens == 128)
+        return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 4>, grid, dim3(kThreads),
+                             stream, p);
+    return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 8>, grid, dim3(kThreads),
+                         stream, p);
+}
+
+template <int DT, int kMode, bool kRound>
+static hipError_t launch_lmh_t(const LmhParams& p, hipStream_t stream) {
     if constexpr (kMode != kLogits) {
-        if (p.scale != 1.0f)
-            return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, true>, grid, dim3(kThreads),
-                                 stream, p);
+        if (p.scale != 1.0f) return launch_lmh_s<DT, kMode, kRound, true>(p, stream);
     }
-    return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, false>, grid, dim3(kThreads), stream, p);
+    return launch_lmh_s<DT, kMode, kRound, false>(p, stream);
 }
 
 template <int kMode>

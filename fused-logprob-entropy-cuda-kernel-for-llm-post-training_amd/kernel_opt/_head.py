@@ -18,9 +18,17 @@ of the chip idle there and d_hidden is two launches.  Ours against the library
     128   32000   1024  24 / 15      20 / 23      37 / 101
     256   50240   2048  48 / 57      79 / 104     73 / 207
     512   32000   1024  32 / 36      39 / 45      50 / 146
-    64    152064  3584  236 / 205
+    64    152064  3584  203 / 204
     192   152064  3584  269 / 287
+    320   152064  3584  417 / 423
+    320   50240   2048  72 / 72
+    320   32000   4096  90 / 75
+    320   128256  1024  107 / 101
+    512   32000   4096  102 / 98
+    512   50240   2048  92 / 101
     1024  152064  3584  843 / 902    971 / 1198   895 / 1475
+The logits' token blocks of 256 (or 128) do a remainder's work in full: the
+library is ahead where fewer than 7/10 of the padded tokens are real ones.
 """
 from __future__ import annotations
 
@@ -49,7 +57,9 @@ def mfma_operands(h2: torch.Tensor, weight: torch.Tensor) -> bool:
 
 
 def logits_pay(n_tokens: int, vocab: int, dim: int) -> bool:
-    return n_tokens >= 192 and n_tokens * vocab * dim >= 15 << 30 and vocab % 8 == 0
+    padded = -(-n_tokens // 256) * 256
+    return (10 * n_tokens >= 7 * padded and n_tokens * vocab * dim >= 15 << 30
+            and vocab % 8 == 0)
 
 
 def d_weight_pays(vocab: int, dim: int) -> bool:

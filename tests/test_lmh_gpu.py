@@ -68,10 +68,12 @@ def test_matches_oracle(N, V, D):
 
 
 @pytest.mark.parametrize("N,V,D", [(256, 256, 64), (255, 257, 64), (257, 255, 128),
-                                   (512, 513, 192), (16, 4096, 64), (300, 70000, 64)])
+                                   (512, 513, 192), (16, 4096, 64), (300, 70000, 64),
+                                   (127, 257, 64), (128, 70000, 192), (129, 513, 128),
+                                   (384, 4097, 64), (385, 8192, 64)])
 def test_tile_and_ring_edges(N, V, D):
-    """Token blocks, vocab tiles and K stages at and around their sizes (256,
-    256 and 64 columns: fewer stages than the rings hold up to several tiles
+    """Token blocks, vocab tiles and K stages at and around their sizes (256
+    or 128, 256 and 64 columns: fewer stages than the rings hold up to several tiles
     a workgroup), with every row of a tile as some token's target."""
     h, w, t = make(N, V, D, seed=31 + N + V + D)
     t = torch.arange(N) * max(1, (V + 255) // 256) % V

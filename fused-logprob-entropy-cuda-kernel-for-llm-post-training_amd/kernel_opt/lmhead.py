@@ -179,19 +179,35 @@ def vocab_chunks(n_tokens: int, vocab: int, elem_bytes: int = 2,
     return plan
 
 
-# Chunk of d_logits of the MFMA backward: as many columns as fit
-# MFMA_CHUNK_BYTES, balanced over the vocabulary in whole 256-column tiles, so
-# that small batches fill the chip (256 tokens over 32768 columns are 128
-# workgroups) and d_hidden's K is long.
+# Chunk of d_logits of the MFMA backward, in whole 256-column tiles.  Up to
+# 1024 tokens equal chunks within 64 MiB.  Above, 128 MiB: fewer chunks make
+# d_hidden's K longer and the passes over its float32 accumulator fewer, and
+# their 256 x 256 tiles are a whole number of rounds of the 256 CUs, as nearly
+# as they fit, the last chunk holding the rest.  Forward + backward, ms, equal
+# chunks within 64 MiB / whole rounds within 128 MiB:
+#   [152064, 3584]   700 tokens  2.81-2.88 / 3.00-3.03   1024  3.78-3.79 / 3.81-3.82
+#                   1500         5.72-5.76 / 5.53-5.54   2048  7.51-7.53 / 7.20
+#                   4096       14.21-14.32 / 14.04-14.08 8192  34.7 / 29.1
+#   [100000, 1024]  2000         1.90 / 1.62-1.63
+#   [50240, 2048]   2048         1.59 / 1.47             1024  0.87-0.88 / 0.85-0.86
+MFMA_CHUNK_TOKENS = 1024
 MFMA_CHUNK_BYTES = 64 << 20
+MFMA_CHUNK_MAX_BYTES = 128 << 20
 
 
 def _mfma_chunks(n_tokens: int, vocab: int, chunk_vocab: int | None) -> list:
     """``(first column, width)`` of every chunk of the MFMA backward."""
     if chunk_vocab is not None:
         return vocab_chunks(n_tokens, vocab, 2, chunk_vocab)
-    n_chunks = max(1, -(-(n_tokens * vocab * 2) // MFMA_CHUNK_BYTES))
-    cols = -(-(-(-vocab // n_chunks)) // 256) * 256
+    if n_tokens <= MFMA_CHUNK_TOKENS:
+        n_chunks = max(1, -(-(n_tokens * vocab * 2) // MFMA_CHUNK_BYTES))
+        cols = -(-(-(-vocab // n_chunks)) // 256) * 256
+    else:
+        tiles = MFMA_CHUNK_MAX_BYTES // (2 * n_tokens * 256)
+        if tiles * 256 < vocab:
+            token_blocks = -(-n_tokens // 256)
+            tiles = max(1, tiles * token_blocks // 256 * 256 // token_blocks)
+        cols = tiles * 256
     return [(c0, min(cols, vocab - c0)) for c0 in range(0, vocab, cols)]
 
 

@@ -4,6 +4,7 @@ from __future__ import annotations
 import math
 
 import numpy as np
+import pytest
 import torch
 
 from oracle import lmh_oracle
@@ -134,3 +135,16 @@ def test_vocab_chunk_plan():
     assert [n for _, n in vocab_chunks(1024, 100, chunk_vocab=1000)] == [100]
     # fp32 halves the columns that fit the small-batch rule
     assert vocab_chunk(1024, 152064, elem_bytes=4) != 32768
+
+
+@pytest.mark.parametrize("n_tokens", [1, 255, 1024, 1025, 2048, 8192, 70000, 300000])
+@pytest.mark.parametrize("vocab", [1, 256, 16384, 50257, 152064])
+def test_mfma_backward_chunks_cover_the_vocabulary(n_tokens, vocab):
+    from kernel_opt.lmhead import MFMA_CHUNK_MAX_BYTES, _mfma_chunks
+    plan = _mfma_chunks(n_tokens, vocab, None)
+    assert [c0 for c0, _ in plan] == [sum(n for _, n in plan[:i]) for i in range(len(plan))]
+    assert sum(n for _, n in plan) == vocab and min(n for _, n in plan) >= 1
+    cols = plan[0][1]
+    assert cols == vocab or cols % 256 == 0
+    # one tile of columns, or within the limit
+    assert cols <= 256 or 2 * n_tokens * cols <= MFMA_CHUNK_MAX_BYTES

@@ -811,10 +811,9 @@ def shard_timing(dev, K, N=32768, V=151936, P=8):
 def lmhead_timing(dev, N=1024, V=152064, D=3584, K=5, rounds=6):
     """The fused LM head against the unfused path on Qwen2.5-7B's head shape
     with C2's 1024 tokens (and 8x that), random weights.  Three paths:
-    "chunked" (the default: a library GEMM per vocabulary chunk, then
-    klp_fwd_shard / klp_fwd_shard_merge; the backward recomputes each chunk),
-    "mfma" (klp_lmh_fwd, the hand-written GEMM with the reduction as its
-    epilogue) and "unfused" (a bf16 library matmul to the [N, V] logits, then
+    "chunked" (the default: the MFMA kernels with each logit rounded to the
+    dtype; the backward recomputes them per vocabulary chunk), "mfma" (the
+    same with fp32 logits) and "unfused" (a bf16 library matmul to the [N, V] logits, then
     klp_fwd / klp_bwd).  Forward, and forward + backward with upstream
     gradients on logprob and entropy; medians over interleaved rounds of K
     calls; peak memory beyond the inputs (and, for the backward, beyond the
@@ -903,7 +902,7 @@ def lmhead_timing(dev, N=1024, V=152064, D=3584, K=5, rounds=6):
         runs.append(run)
         del h, t, gl, ge
         torch.cuda.empty_cache()
-    # GRPO on the head: the chunked LM head + fused step (library GEMMs and
+    # GRPO on the head: the chunked LM head + fused step (GEMMs and
     # klp_grpo_step per chunk of tokens) against the unfused path (bf16
     # matmul to the full logits, the logprob op, the GRPO loss, backward), at
     # this token count and at 8x it.
@@ -974,15 +973,16 @@ def lmhead_timing(dev, N=1024, V=152064, D=3584, K=5, rounds=6):
            "roofline_fwd": {"bound": "mfma", "achieved": c["fwd_tflops"],
                             "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                             "frac": round(c["fwd_tflops"] / MFMA_BF16_PEAK_TFLOPS, 4)},
-           "note": "fused = the chunked head (default); mfma = klp_lmh_fwd with the "
+           "note": "fused = the default head (MFMA kernels, each logit rounded to the "
+                   "dtype); mfma = the same with fp32 logits; both with a "
                    "vocabulary-chunked backward; unfused = bf16 library matmul to [N, V] "
                    "logits, then klp_fwd / klp_bwd; medians of 6 interleaved rounds of 5 "
                    "calls, the order reversed every round",
            "grpo_step": {
                "runs": grpo_heads,
                "note": "fused_linear_grpo_step (chunks of the given token count, 'default' "
-                       "its own chunking: library "
-                       "GEMMs + klp_grpo_step, d_hidden / d_weight computed in the forward), "
+                       "its own chunking: MFMA or "
+                       "library GEMMs + klp_grpo_step, d_hidden / d_weight computed in the forward), "
                        "and vocab_chunked_head (fused_linear_logprob_entropy, the "
                        "vocabulary-chunked head, + fused_grpo_loss + backward), "
                        "against matmul + fused_logprob_entropy + fused_grpo_loss + backward; "

@@ -41,7 +41,7 @@ constexpr int kGrpoThreads = 256;
 // bool mask, us before -> after, with the conversion: [8, 512] 3.6 + 3.0 + 3.6
 // -> 4.3 + 3.2, [1, 4749] 9.8 + 7.5 + 3.6 -> 5.3 + 3.6, [64, 4096] 9.2 + 7.9 +
 // 3.9 -> 6.1 + 4.1; the call with its backward, which the host's launches
-// bound, 65.2 -> 61.4 at [8, 512].
+// bound, 65.2 -> 61.4 at [16, 2048].
 constexpr int kGrpoUnroll = 4;
 constexpr int kGrpoLongThreads = 1024;
 constexpr int64_t kGrpoShortRow = kGrpoThreads * kGrpoUnroll;

@@ -658,3 +658,19 @@ def test_lm_head_as_rejects_bad_arguments():
     assert bwd(104, -1) != 0 and "vocab_offset" in error()
     assert bwd(104, 0, None) != 0 and "non-null" in error()
     assert lib.klp_lmh_logits(0, P, 64, P, 64, 4, 100, 64, P, 96, None) != 0 and ">= vocab" in error()
+
+
+@pytest.mark.parametrize("kw,message", [
+    (dict(dtype=3), "mask dtype"), (dict(mask=None), "mask"), (dict(dtype=2, mask=4), "mask"),
+    (dict(mask_out=None), "mask_out"), (dict(B=0), "n_seqs"), (dict(loss=None), "loss")])
+def test_grpo_masked_forward_rejects_bad_arguments(kw, message):
+    from kernel_opt._library import lib
+    P = 0x100000
+    ws = lib.klp_grpo_workspace_bytes(4)
+    a = dict(dtype=0, mask=P, mask_out=P, B=4, loss=P)
+    a.update(kw)
+    rc = lib.klp_grpo_fwd_masked(P, P, None, P, a["mask"], a["dtype"], a["mask_out"], a["B"], 10,
+                                 0.2, 0.2, 0.0, 1.0, 1, 0, 0, a["loss"], None, P, ws, None)
+    buf = ctypes.create_string_buffer(512)
+    lib.klp_last_error(buf, 512)
+    assert rc != 0 and message in buf.value.decode(), (rc, buf.value)

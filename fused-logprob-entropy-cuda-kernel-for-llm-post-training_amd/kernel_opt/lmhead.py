@@ -36,9 +36,6 @@ old-policy and reference log-probabilities).
 """
 from __future__ import annotations
 
-import collections
-import threading
-
 import torch
 
 from . import _C
@@ -52,29 +49,6 @@ __all__ = ["fused_linear_logprob_entropy", "fused_linear_logprob_entropy_forward
 
 
 _ptr = ptr
-
-
-# Forward workspaces, one per (device, stream), the 16 most recently used
-# kept (as kernel_opt._C keeps its split-row workspaces).
-_ws_lock = threading.Lock()
-_ws: collections.OrderedDict = collections.OrderedDict()
-_WS_KEEP = 16
-
-
-def _workspace(dev, stream, nbytes):
-    """The workspace of (device, raw handle of its current stream), allocated
-    on that stream."""
-    key = (dev.index, stream)
-    with _ws_lock:
-        buf = _ws.get(key)
-        if buf is None or buf.numel() < nbytes:
-            with torch.cuda.stream(torch.cuda.current_stream(dev)):
-                buf = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
-            _ws[key] = buf
-        _ws.move_to_end(key)
-        while len(_ws) > _WS_KEEP:
-            _ws.popitem(last=False)
-        return buf
 
 
 def _check(hidden, weight, targets, impl):
@@ -229,7 +203,9 @@ def _forward_mfma(h2, weight, t, T, rounded, out):
     N, V, D = h2.size(0), weight.size(0), h2.size(1)
     with device_guard(dev.index):
         stream = stream_handle(dev.index)
-        ws = _workspace(dev, stream, lib.klp_lmh_workspace_bytes(N, V, D))
+        # From the allocator on every call: a captured call's then belongs to
+        # its graph, and no later call can replace it under a replay.
+        ws = torch.empty(lib.klp_lmh_workspace_bytes(N, V, D), dtype=torch.uint8, device=dev)
         check_status(lib.klp_lmh_fwd_as(DTYPE_CODES[h2.dtype], int(rounded), _ptr(h2), _ld(h2),
                                         _ptr(weight), _ld(weight), N, V, D, _ptr(t), T,
                                         _ptr(out[0]), _ptr(out[1]), _ptr(out[2]), _ptr(ws),

@@ -456,3 +456,33 @@ def test_chunked_holds_no_full_logits():
     grads = w.grad.numel() * 2 + h.grad.numel() * 2
     bwd_extra = torch.cuda.max_memory_allocated() - base - grads
     assert bwd_extra < full // 2, f"backward peak {bwd_extra / 2**20:.0f} MiB beyond the grads"
+
+
+@pytest.mark.parametrize("impl", ["chunked", "mfma"])
+def test_captured_forward_keeps_its_workspace(impl):
+    """A captured forward replays to the eager outputs, with larger eager
+    calls (whose workspaces are larger) and allocations between the replays."""
+    from kernel_opt import fused_linear_logprob_entropy_forward
+    h, w, t = (x.to(DEV) for x in make(300, 5000, 128, seed=41))
+    big = [x.to(DEV) for x in make(700, 40000, 128, seed=42)]
+    run = lambda *a: fused_linear_logprob_entropy_forward(*a, impl=impl)  # noqa: E731
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run(h, w, t)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        outs = run(h, w, t)
+    for k in range(4):
+        with torch.cuda.stream(side):
+            run(*big)
+            junk = torch.full((1 << 20,), float("nan"), device=DEV)
+        torch.cuda.synchronize()
+        h.copy_(torch.roll(h, 1, 0))
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(outs, run(h, w, t)):
+            assert torch.equal(a, b)
+        del junk

@@ -50,8 +50,8 @@ def _rows_ok(t: torch.Tensor) -> bool:
 
 def mfma_operands(h2: torch.Tensor, weight: torch.Tensor) -> bool:
     """True when the MFMA kernels take hidden ``[N, D]`` and weight ``[V, D]``
-    (one dtype, rows with unit stride)."""
-    return (h2.dtype in (torch.bfloat16, torch.float16) and h2.size(0) > 0
+    (one dtype, one device, rows with unit stride)."""
+    return (h2.device == weight.device and h2.dtype in (torch.bfloat16, torch.float16) and h2.size(0) > 0
             and h2.size(1) >= 64 and h2.size(1) % 64 == 0 and h2.stride(1) == 1
             and weight.stride(1) == 1 and _rows_ok(h2) and _rows_ok(weight))
 

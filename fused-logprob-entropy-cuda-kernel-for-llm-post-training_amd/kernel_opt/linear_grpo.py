@@ -204,6 +204,8 @@ def fused_linear_grpo_step(hidden: torch.Tensor, weight: torch.Tensor, targets: 
         raise RuntimeError(f"hidden must be [B, S, D], got shape {tuple(hidden.shape)}")
     if not (hidden.is_cuda and weight.is_cuda and targets.is_cuda):
         raise RuntimeError("hidden, weight and targets must be GPU tensors")
+    if not (weight.device == hidden.device and targets.device == hidden.device):
+        raise RuntimeError("hidden, weight and targets must be on the same device")
     B, S, D = hidden.shape
     if weight.dim() != 2 or weight.size(1) != D:
         raise RuntimeError(f"weight must be [V, {D}], got {tuple(weight.shape)}")

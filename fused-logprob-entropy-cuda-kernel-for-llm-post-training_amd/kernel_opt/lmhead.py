@@ -56,6 +56,8 @@ def _check(hidden, weight, targets, impl):
         raise ValueError(f"impl must be 'chunked' or 'mfma', got {impl!r}")
     if not (hidden.is_cuda and weight.is_cuda and targets.is_cuda):
         raise RuntimeError("hidden, weight and targets must be GPU tensors")
+    if not (weight.device == hidden.device and targets.device == hidden.device):
+        raise RuntimeError("hidden, weight and targets must be on the same device")
     if impl == "mfma" and (hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16):
         raise RuntimeError("hidden and weight must be bfloat16")
     if hidden.dtype not in DTYPE_CODES or weight.dtype != hidden.dtype:

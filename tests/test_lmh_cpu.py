@@ -137,6 +137,34 @@ def test_vocab_chunk_plan():
     assert vocab_chunk(1024, 152064, elem_bytes=4) != 32768
 
 
+@pytest.mark.parametrize("elsewhere", ["hidden", "weight", "targets"])
+def test_operands_on_two_devices_are_refused(elsewhere):
+    """Refused before any launch, by every entry point of the head: the kernels
+    get raw pointers and run on one device's stream.  Shape-only tensors stand
+    for those of two GPUs."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    import kernel_opt
+    from kernel_opt._head import mfma_operands
+    with FakeTensorMode():
+        dev = {k: "cuda:1" if k == elsewhere else "cuda:0" for k in ("hidden", "weight", "targets")}
+        h = torch.empty(1, 1024, 1024, dtype=torch.bfloat16, device=dev["hidden"])
+        w = torch.empty(32000, 1024, dtype=torch.bfloat16, device=dev["weight"])
+        t = torch.empty(1, 1024, dtype=torch.int64, device=dev["targets"])
+        old = torch.empty(1, 1024, device=dev["hidden"])
+        adv = torch.empty(1, device=dev["hidden"])
+        for impl in ("chunked", "mfma"):
+            with pytest.raises(RuntimeError, match="same device"):
+                kernel_opt.fused_linear_logprob_entropy_forward(h, w, t, impl=impl)
+            with pytest.raises(RuntimeError, match="same device"):
+                kernel_opt.fused_linear_logprob_entropy(h, w, t, impl=impl)
+        for level in ("token", "sequence"):
+            with pytest.raises(RuntimeError, match="same device"):
+                kernel_opt.fused_linear_grpo_step(h, w, t, old, adv, importance_level=level)
+        if elsewhere != "targets":
+            assert not mfma_operands(h.view(-1, 1024), w)
+
+
 @pytest.mark.parametrize("n_tokens", [1, 255, 1024, 1025, 2048, 8192, 70000, 300000])
 @pytest.mark.parametrize("vocab", [1, 256, 16384, 50257, 152064])
 def test_mfma_backward_chunks_cover_the_vocabulary(n_tokens, vocab):

@@ -36,7 +36,7 @@ import torch
 
 from ._library import DTYPE_CODES, check_status, lib, ptr
 
-_MAX_LD = (2 ** 31 - 1) // 512  # 32-bit byte offsets within 256 rows
+MAX_LD = (2 ** 31 - 1) // 512  # 32-bit byte offsets within 256 rows
 
 
 def row_stride(t: torch.Tensor) -> int:
@@ -45,7 +45,7 @@ def row_stride(t: torch.Tensor) -> int:
 
 def _rows_ok(t: torch.Tensor) -> bool:
     ld = row_stride(t)
-    return t.data_ptr() % 16 == 0 and ld % 8 == 0 and t.size(1) <= ld <= _MAX_LD
+    return t.data_ptr() % 16 == 0 and ld % 8 == 0 and t.size(1) <= ld <= MAX_LD
 
 
 def mfma_operands(h2: torch.Tensor, weight: torch.Tensor) -> bool:

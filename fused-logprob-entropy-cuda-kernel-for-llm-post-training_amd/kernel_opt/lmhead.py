@@ -39,8 +39,8 @@ from __future__ import annotations
 import torch
 
 from . import _C
-from ._head import (d_hidden_into, d_hidden_pays, d_weight_into, d_weight_pays, logits_into,
-                    mfma_operands)
+from ._head import (MAX_LD, d_hidden_into, d_hidden_pays, d_weight_into, d_weight_pays,
+                    logits_into, mfma_operands)
 from ._library import DTYPE_CODES, check_status, device_guard, lib, ptr, stream_handle
 from .linear_grpo import _accumulate_f32
 
@@ -84,7 +84,7 @@ def _ld(t: torch.Tensor) -> int:
 def _rows_32bit(t: torch.Tensor) -> torch.Tensor:
     """``t``, or its contiguous copy where the MFMA kernels' 32-bit offsets
     within 256 rows would not reach (row strides above 4194303 elements)."""
-    return t if _ld(t) <= (2 ** 31 - 1) // 512 else t.contiguous()
+    return t if _ld(t) <= MAX_LD else t.contiguous()
 
 
 # Vocabulary chunk of the chunked head.  Small batches (a chunk of
@@ -169,12 +169,15 @@ def vocab_chunks(n_tokens: int, vocab: int, elem_bytes: int = 2,
 MFMA_CHUNK_TOKENS = 1024
 MFMA_CHUNK_BYTES = 64 << 20
 MFMA_CHUNK_MAX_BYTES = 128 << 20
+# A chunk's columns are the row stride of its d_logits, which the products
+# address with 32-bit offsets: few tokens of millions of columns take several.
+MFMA_CHUNK_MAX_COLS = MAX_LD // 256 * 256
 
 
 def _mfma_chunks(n_tokens: int, vocab: int, chunk_vocab: int | None) -> list:
     """``(first column, width)`` of every chunk of the MFMA backward."""
     if chunk_vocab is not None:
-        return vocab_chunks(n_tokens, vocab, 2, chunk_vocab)
+        return vocab_chunks(n_tokens, vocab, 2, min(chunk_vocab, MFMA_CHUNK_MAX_COLS))
     if n_tokens <= MFMA_CHUNK_TOKENS:
         n_chunks = max(1, -(-(n_tokens * vocab * 2) // MFMA_CHUNK_BYTES))
         cols = -(-(-(-vocab // n_chunks)) // 256) * 256
@@ -184,6 +187,7 @@ def _mfma_chunks(n_tokens: int, vocab: int, chunk_vocab: int | None) -> list:
             token_blocks = -(-n_tokens // 256)
             tiles = max(1, tiles * token_blocks // 256 * 256 // token_blocks)
         cols = tiles * 256
+    cols = min(cols, MFMA_CHUNK_MAX_COLS)
     return [(c0, min(cols, vocab - c0)) for c0 in range(0, vocab, cols)]
 
 

@@ -176,3 +176,15 @@ def test_mfma_backward_chunks_cover_the_vocabulary(n_tokens, vocab):
     assert cols == vocab or cols % 256 == 0
     # one tile of columns, or within the limit
     assert cols <= 256 or 2 * n_tokens * cols <= MFMA_CHUNK_MAX_BYTES
+
+
+@pytest.mark.parametrize("n_tokens,chunk_vocab", [(1, None), (4, None), (1, 5000000),
+                                                   (2000, 4194303)])
+def test_mfma_backward_chunks_stay_within_the_row_stride(n_tokens, chunk_vocab):
+    """Millions of columns: every chunk's d_logits rows, padded to 8 columns,
+    are within the stride that the products take."""
+    from kernel_opt.lmhead import _mfma_chunks
+    plan = _mfma_chunks(n_tokens, 9000001, chunk_vocab)
+    assert [c0 for c0, _ in plan] == [sum(n for _, n in plan[:i]) for i in range(len(plan))]
+    assert sum(n for _, n in plan) == 9000001
+    assert max(-(-n // 8) * 8 for _, n in plan) <= (2 ** 31 - 1) // 512

@@ -95,7 +95,6 @@ __device__ __forceinline__ void bwd_piece(const BwdParams& p, const u32x4* vin, 
 template <int DT, int WAVES, int U, bool kNtStore, bool kScaled>
 __global__ __launch_bounds__(WAVES * 64) void klp_bwd_kernel(BwdParams p) {
     typedef typename Traits<DT>::elem elem;
-    constexpr int NTHREADS = WAVES * 64;
     constexpr int EPV = Traits<DT>::kPerVec;
     constexpr int ESZ = 16 / EPV;
 

@@ -477,7 +477,9 @@ class FusedGrpoLoss : public torch::autograd::Function<FusedGrpoLoss> {
             c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
         // A bool or integer mask is read as it is; the kernel leaves it in
         // float32 for the backward.
-        const int code = given.defined() ? mask_dtype_code(given.scalar_type()) : -1;
+        const int code = !given.defined()                      ? -1
+                         : given.scalar_type() == at::kBool ? KLP_MASK_BOOL
+                                                            : mask_dtype_code(given.scalar_type());
         at::Tensor m = given;
         if (code >= 0) {
             m = at::empty({B, S}, f32);

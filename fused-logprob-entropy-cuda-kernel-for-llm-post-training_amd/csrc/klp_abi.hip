@@ -841,9 +841,13 @@ int klp_grpo_fwd_masked(const float* logp, const float* old_logp, const float* r
                         eps_high, beta, norm_const, loss_type, level, adv_per_token, workspace,
                         workspace_bytes, &p);
     if (rc != KLP_OK) return rc;
-    if (mask_dtype != KLP_MASK_U8 && mask_dtype != KLP_MASK_I32 && mask_dtype != KLP_MASK_I64)
-        return fail(KLP_EDTYPE, "mask dtype must be KLP_MASK_U8, KLP_MASK_I32 or KLP_MASK_I64");
-    const size_t esz = mask_dtype == KLP_MASK_U8 ? 1 : mask_dtype == KLP_MASK_I32 ? 4 : 8;
+    const size_t esz = mask_dtype == KLP_MASK_U8 || mask_dtype == KLP_MASK_BOOL ? 1
+                       : mask_dtype == KLP_MASK_I32                            ? 4
+                       : mask_dtype == KLP_MASK_I64                            ? 8
+                                                                               : 0;
+    if (esz == 0)
+        return fail(KLP_EDTYPE, "mask dtype must be KLP_MASK_BOOL, KLP_MASK_U8, KLP_MASK_I32 or "
+                                "KLP_MASK_I64");
     if (mask == nullptr || !aligned(mask, esz))
         return fail(KLP_EINVAL, "mask must be non-null and aligned to its element size");
     if ((rc = check_f32(mask_out, "mask_out")) != KLP_OK) return rc;

@@ -92,6 +92,12 @@ __device__ __forceinline__ void block_sum(float (&v)[K]) {
     __syncthreads();
 }
 
+// A bool mask's element: any byte but 0 is true, as in torch's conversions.
+struct MaskBool {
+    uint8_t byte;
+    __device__ explicit operator float() const { return byte ? 1.0f : 0.0f; }
+};
+
 // A token's inputs.
 struct TokenIn {
     float m, lp, lo, adv, lr;
@@ -472,7 +478,8 @@ static hipError_t launch_grpo_rows(const GrpoParams& p, hipStream_t stream) {
 }
 
 hipError_t launch_grpo_fwd(const GrpoParams& p, hipStream_t stream) {
-    const hipError_t e = p.mask_dtype == KLP_MASK_U8    ? launch_grpo_rows<uint8_t>(p, stream)
+    const hipError_t e = p.mask_dtype == KLP_MASK_BOOL  ? launch_grpo_rows<MaskBool>(p, stream)
+                         : p.mask_dtype == KLP_MASK_U8  ? launch_grpo_rows<uint8_t>(p, stream)
                          : p.mask_dtype == KLP_MASK_I32 ? launch_grpo_rows<int32_t>(p, stream)
                          : p.mask_dtype == KLP_MASK_I64 ? launch_grpo_rows<int64_t>(p, stream)
                                                         : launch_grpo_rows<float>(p, stream);

@@ -112,7 +112,7 @@ struct GrpoParams {
     const float* ref_logp;   // nullable
     const float* adv;        // [B], or [B, S] when adv_per_token
     const void* mask;        // nullable (all ones), of mask_dtype
-    int mask_dtype;          // KLP_MASK_U8 / _I32 / _I64, or kMaskF32
+    int mask_dtype;          // KLP_MASK_BOOL / _U8 / _I32 / _I64, or kMaskF32
     float* mask_out;         // forward: the mask in float32, nullable
     int64_t B;
     int64_t S;

@@ -294,9 +294,9 @@ int klp_grpo_fwd(const float* logp, const float* old_logp, const float* ref_logp
                  void* workspace, size_t workspace_bytes,
                  void* stream);
 
-/* klp_grpo_fwd for a bool / uint8, int32 or int64 mask (KLP_MASK_U8 / _I32 /
- * _I64, below), which it reads as it is and writes to `mask_out` (float32
- * [n_seqs, seq_len]): the mask klp_grpo_bwd then takes. */
+/* klp_grpo_fwd for a bool, uint8, int32 or int64 mask (KLP_MASK_BOOL / _U8 /
+ * _I32 / _I64, below), which it reads as it is and writes to `mask_out`
+ * (float32 [n_seqs, seq_len]): the mask klp_grpo_bwd then takes. */
 int klp_grpo_fwd_masked(const float* logp, const float* old_logp, const float* ref_logp,
                         const float* advantages, const void* mask, int mask_dtype,
                         float* mask_out, int64_t n_seqs, int64_t seq_len,
@@ -397,7 +397,8 @@ int klp_grpo_step(const void* logits, int dtype, int64_t n_rows, int64_t vocab,
 enum klp_mask_dtype {
     KLP_MASK_U8 = 0,
     KLP_MASK_I32 = 1,
-    KLP_MASK_I64 = 2
+    KLP_MASK_I64 = 2,
+    KLP_MASK_BOOL = 4 /* bytes, any but 0 counts as 1; klp_grpo_fwd_masked only */
 };
 
 #define KLP_GRPO_TOKEN_WEIGHTS_WORKSPACE_BYTES 8192

@@ -171,3 +171,21 @@ def test_integer_masks_match_float_bitwise(B, S, level, dtype):
     for given in (m.to(dtype), strided):
         for a, b in zip(go(given), expect):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,S", [(2, 255), (2, 1025)])
+def test_bool_mask_of_any_bytes(B, S):
+    """A bool mask made from bytes other than 0 and 1 counts as torch converts
+    it, every byte but 0 as 1."""
+    from kernel_opt import fused_grpo_loss
+    new, old, ref, adv, _ = case(B, S, 19, adv_per_token=True)
+    t = lambda a: torch.tensor(a, device=DEV)
+    byte = (torch.arange(B * S, device=DEV).view(B, S) % 4 * 85).to(torch.uint8)  # 0, 85, 170, 255
+    outs = []
+    for m in (byte.view(torch.bool), byte.ne(0).float()):
+        lp = torch.tensor(new, device=DEV, requires_grad=True)
+        loss, stats = fused_grpo_loss(lp, t(old), t(adv), m, t(ref), beta=0.04)
+        loss.backward()
+        outs.append((loss.detach(), stats, lp.grad))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)

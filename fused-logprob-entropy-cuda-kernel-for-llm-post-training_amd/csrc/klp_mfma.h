@@ -42,10 +42,14 @@ __device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
 // acc += a * b (`zero`: acc = a * b), in AGPRs and in place: left to the
 // builtin, the compiler renames the 256 accumulators from MFMA to MFMA and
 // pays for it in moves through VGPRs and spills at every join (436-920 bytes
-// of scratch in the LM head's forward, 970 against 800 us).  What it would
-// insert around its own MFMAs is then the caller's: the operands come from
-// LDS reads (waited for as any use), an accumulator's own MFMAs are 64 apart,
-// and drain() comes before other instructions read accumulators.
+// of scratch in the LM head's forward, 970 against 800 us).  The wait states
+// it would insert around its own MFMAs are then the caller's: the operands
+// come straight from LDS reads (waited for as any use), so that no VALU
+// instruction writes one in the 2 wait states before; an accumulator's own
+// MFMAs are a half stage apart, 64 or, with blocks of 128 tokens, 32; and
+// drain() comes before other instructions read accumulators.  The compiler
+// is free to move a register in between: tests/test_mfma_hazards_cpu.py looks
+// for that in the generated code.
 template <int DT>
 __device__ __forceinline__ void mul_add(f32x4& acc, operand a, operand b, bool zero) {
     if constexpr (DT == kBF16) {
@@ -126,8 +130,15 @@ __device__ __forceinline__ int swz_k(int k) { return (k & 3) | (((k >> 3) & 1) <
 // In asm because the compiler, which cannot tell the rings' slots apart, puts
 // s_waitcnt vmcnt(0) between a copy it knows of and a following transposing
 // read; nothing is loaded into registers here, and the callers count their
-// copies and wait for them (also before the kernel ends).  The s_nop is the
-// wait state between writing M0 and a copy that reads it.
+// copies and wait for them (also before the kernel ends).  The compiler sees
+// no memory instruction, so its wait states are ours: the s_nop is the 1 from
+// writing M0 to a copy that reads it; of the 5 from a VALU instruction that
+// wrote the descriptor or an offset (the reload of a spilled SGPR) it is the
+// second.  All 5 here (s_nop 3) cost the training passes at [152064, 3584]
+// 1.3% (head 3727 -> 3778 us, linear step 2768 -> 2805).  In the generated
+// code no such write stands that close, and M0, which cannot be named as
+// clobbered (it is reserved), has no other use in the kernel that calls this:
+// tests/test_mfma_hazards_cpu.py checks both.
 __device__ __forceinline__ void copy_to_lds(u32x4 rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
     asm volatile(
         "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"

@@ -487,21 +487,30 @@ int grpo_setup(const float* logp, const float* old_logp, const float* ref_logp,
 // Fused LM head: tokens per workgroup and vocab tiles per workgroup chunk.  A
 // CU holds one workgroup, so the launch takes (rounds of 256 workgroups) *
 // (tiles per workgroup) tile times, plus each round's prologue and merge
-// (about 1/8 of a tile time at dim 3584); of 256 and 128 tokens and 1..16
-// tiles the pair with the least of that is taken, 256 tokens and the fewest
-// tiles on a tie.  1024 tokens of [152064, 3584]: 5 tiles (2 rounds) 828-840
-// us, 2 tiles (5 rounds) 848-862, 3 tiles (4 rounds, 12 tile times for 9.3
-// tiles of work per CU) 957, main loop alone.  A tile of 128 tokens takes 5/8
-// of one of 256 (1024 tokens as 8 blocks of 128: 980 us against 794; the
-// weight rows are read from LDS for half as many MFMAs).  Forward, us, 256 /
-// 128 tokens a workgroup:
+// (about 1/8 of a tile time at dim 3584); of 256, 192 and 128 tokens and 1..16
+// tiles the pair with the least of that is taken, the larger block and the
+// fewest tiles on a tie.  1024 tokens of [152064, 3584]: 10 tiles (1 round)
+// 784-800 us, 5 tiles (2 rounds) 786-800, 2 tiles (5 rounds) 803-829, 4 tiles
+// (3 rounds, 12 tile times for 9.3 tiles of work per CU) 871-875, 3 tiles (4
+// rounds, 12 as well) 893-896.
+// A tile of 192 tokens takes 13/16, one of 128 5/8 of one of 256 (1024 tokens
+// as 8 blocks of 128: 973-991 us; the weight rows are read from LDS for half
+// as many MFMAs).  Blocks of 192 are for a last block that would be mostly
+// padding: 300 tokens of [152064, 3584] 331-338 us with 5 tiles of 192,
+// 412-415 with 5 of 256, 391-395 with 8 of 128.  Forward, us, 256 / 128
+// tokens a workgroup:
 //   N     [152064, 3584]  [50240, 2048]  [32000, 4096]  [16384, 512]
 //   16    232 / 191       52 / 39        79 / 53        22 / 22
 //   128   238 / 209       53 / 41        79 / 61        24 / 23
 //   200   259 / 278       52 / 55        80 / 62        24 / 23
-//   320   395 / 399       89 / 77        94 / 100       24 / 23
 //   512   424 / 517       97 / 103       101 / 112      24 / 23
 //   1280                  209 / 231      250 / 286      38 / 33
+// and 256 or 128, as the rule without 192 chose / the rule:
+//   N     [152064, 3584]  [151936, 2048]  [32000, 4096]  [100000, 1024]
+//   260   429-432 / 373   238 / 201
+//   320   432 / 368                       106 / 92       86 / 86
+//   560   603 / 517                                      129 / 111
+//   1100  958 / 940                                      224 / 206
 struct LmhPlan {
     int block_tokens;
     int64_t tiles_per_chunk;
@@ -512,12 +521,14 @@ LmhPlan lmh_plan(int64_t n_tokens, int64_t vocab) {
     const int64_t vt = klp::lmh_vocab_tiles(vocab);
     LmhPlan best{256, 1, vt};
     int64_t best_cost = INT64_MAX;
-    for (int block : {256, 128}) {
+    for (int block : {256, 192, 128}) {
         const int64_t tb = (n_tokens + block - 1) / block;
         for (int64_t tpc = 1; tpc <= 16 && tpc <= vt; ++tpc) {
             const int64_t n_chunks = (vt + tpc - 1) / tpc;
             const int64_t rounds = ((n_chunks + 7) / 8 * 8 * tb + kCus - 1) / kCus;
-            const int64_t cost = rounds * ((block == 256 ? 8 : 5) * tpc + 1);
+            // In sixteenths of a 256-token tile's time.
+            const int64_t tile = block == 256 ? 16 : block == 192 ? 13 : 10;
+            const int64_t cost = rounds * (tile * tpc + 2);
             if (cost < best_cost) {
                 best_cost = cost;
                 best = LmhPlan{block, tpc, n_chunks};

@@ -220,7 +220,7 @@ struct LmhParams {
     float scale;             // 1 / temperature
     float* partials;         // [n_chunks, n_tokens] float4 (m, z, t, unused)
     float* target_logit;     // [n_tokens], behind the partials; written where a target is valid
-    int block_tokens;        // tokens per workgroup: 256 or 128
+    int block_tokens;        // tokens per workgroup: 256, 192 or 128
     int64_t n_tblocks;       // ceil(n_tokens / block_tokens)
     int64_t n_vtiles;        // ceil(vocab / 256)
     int64_t tiles_per_chunk;

@@ -14,7 +14,8 @@
 // it computes the 256 x 256 block of logits^T with v_mfma_f32_16x16x32_bf16,
 // each wave a 128 x 128 part of it (64 accumulator blocks, 256 AGPRs).  Where
 // that leaves less for the matrix cores to do (few tokens, or a remainder
-// block that would be mostly padding) token blocks of 128, a wave 128 x 64:
+// block that would be mostly padding) token blocks of 192 or 128, a wave
+// 128 x 96 or 128 x 64:
 //  - the transposed orientation puts vocab rows on the MFMA's M side, so a
 //    lane's accumulators belong to 8 tokens, 32 vocab rows of each: the
 //    online softmax update runs lane-locally, with no cross-lane reduction
@@ -58,7 +59,9 @@
 // with the target took 1239.  32x32x16 MFMAs at this tile and ring: 840-848
 // us against 797-821 for the main loop alone, at 1.62 against 1.85 GHz.  Up
 // to 128 tokens the weight's bytes bound it: 16 tokens 191 us (5.7 TB/s) with
-// blocks of 128, 232 with blocks of 256.
+// blocks of 128, 232 with blocks of 256.  257-384 tokens, two blocks of 192:
+// 300 tokens 368 us, 432 with blocks of 256, most of the second one padding
+// (the library's GEMM per vocabulary chunk, which this kernel replaced: 401).
 //
 // Workgroup order: workgroup b runs on XCD b % 8 (round-robin dispatch).
 // Consecutive workgroups of one XCD take the token blocks of one vocab
@@ -84,7 +87,8 @@ enum : int { kFold = 0, kGradient = 1, kLogits = 2 };
 // klp_bwd (grad_one, klp_device.h) and written in DT; kLogits: the logits
 // themselves, rounded to DT (kRound, not scaled).  kRound: each logit is
 // rounded to DT before it is scaled and used, as a GEMM that writes DT does.
-// kTokBlocks: 16-token blocks per wave, 8 or 4 (256 or 128 tokens a workgroup).
+// kTokBlocks: 16-token blocks per wave, 8, 6 or 4 (256, 192 or 128 tokens a
+// workgroup).
 template <int DT, int kMode, bool kRound, bool kScaled, int kTokBlocks>
 __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     constexpr int kTokSide = 16 * kTokBlocks;  // a wave's tokens
@@ -471,6 +475,9 @@ static hipError_t launch_lmh_s(const LmhParams& p, hipStream_t stream) {
     // padding workgroups exit at once.
     const int64_t chunks8 = (p.n_chunks + 7) / 8 * 8;
     const dim3 grid(static_cast<unsigned>(chunks8 * p.n_tblocks));
+    if (p.block_tokens == 192)
+        return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 6>, grid, dim3(kThreads),
+                             stream, p);
     if (p.block_tokens == 128)
         return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 4>, grid, dim3(kThreads),
                              stream, p);

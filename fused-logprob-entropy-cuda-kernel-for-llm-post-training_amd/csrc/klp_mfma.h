@@ -46,7 +46,8 @@ __device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
 // it would insert around its own MFMAs are then the caller's: the operands
 // come straight from LDS reads (waited for as any use), so that no VALU
 // instruction writes one in the 2 wait states before; an accumulator's own
-// MFMAs are a half stage apart, 64 or, with blocks of 128 tokens, 32; and
+// MFMAs are a half stage apart, 64 or, with blocks of 192 or 128 tokens, 48
+// or 32; and
 // drain() comes before other instructions read accumulators.  The compiler
 // is free to move a register in between: tests/test_mfma_hazards_cpu.py looks
 // for that in the generated code.

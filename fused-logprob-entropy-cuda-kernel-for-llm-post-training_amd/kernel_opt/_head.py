@@ -27,7 +27,7 @@ of the chip idle there and d_hidden is two launches.  Ours against the library
     512   32000   4096  102 / 98
     512   50240   2048  92 / 101
     1024  152064  3584  843 / 902    971 / 1198   895 / 1475
-The logits' token blocks of 256 (or 128) do a remainder's work in full: the
+The logits' token blocks of 256 (192, 128) do a remainder's work in full: the
 library is ahead where fewer than 7/10 of the padded tokens are real ones.
 """
 from __future__ import annotations

@@ -40,7 +40,7 @@ import torch
 
 from . import _C
 from ._head import (MAX_LD, d_hidden_into, d_hidden_pays, d_weight_into, d_weight_pays,
-                    logits_into, mfma_operands)
+                    mfma_operands)
 from ._library import DTYPE_CODES, check_status, device_guard, lib, ptr, stream_handle
 from .linear_grpo import _accumulate_f32
 
@@ -193,13 +193,10 @@ def _mfma_chunks(n_tokens: int, vocab: int, chunk_vocab: int | None) -> list:
 
 def _chunk_logits(buf, h2, weight, c0, n):
     """logits[:, c0:c0+n] = h2 @ weight[c0:c0+n]^T into a contiguous view of
-    ``buf``: the values the chunked head's forward and backward use."""
+    ``buf`` through the library: the same call, hence the same values, in the
+    forward and the backward of heads without MFMA kernels."""
     out = buf[: h2.size(0) * n].view(h2.size(0), n)
-    if mfma_operands(h2, weight):
-        with device_guard(h2.device.index):
-            logits_into(out, h2, weight[c0:c0 + n], stream_handle(h2.device.index))
-    else:
-        torch.mm(h2, weight[c0:c0 + n].t(), out=out)
+    torch.mm(h2, weight[c0:c0 + n].t(), out=out)
     return out
 
 

@@ -8,10 +8,11 @@ entropy and lse inherit at most the largest logit error of their row plus the
 fp32 softmax noise.  Per token:
     |ours - oracle| <= 2e-5 + 8 * 2^-24 * sqrt(D / 16) * max_v sum_k |h_k w_k|.
 
-Chunked head (impl="chunked", the default): the library GEMM rounds each
-logit once to the input dtype, so the bar is the logprob kernels' own bar on
-those logits (the float64 logits oracle, oracle/klp_oracle.py, on the chunk
-GEMMs' output), plus a float64 check of the head itself whose bound follows
+Chunked head (impl="chunked", the default): each logit is rounded once to the
+input dtype, by the MFMA kernels or, for the operands they do not take, by the
+library GEMM, so the bar is the logprob kernels' own bar on those logits (the
+float64 logits oracle, oracle/klp_oracle.py, on the logits that klp_lmh_logits
+or the chunk GEMMs write), plus a float64 check of the head itself whose bound follows
 from the logit rounding: with every logit within eps of exact, lse moves by
 at most eps, logp by 2 eps and the entropy by eps * sqrt(Var_p(x)) to first
 order (the derivative of H is -p_v (x_v - mean_p x)).
@@ -70,10 +71,11 @@ def test_matches_oracle(N, V, D):
 @pytest.mark.parametrize("N,V,D", [(256, 256, 64), (255, 257, 64), (257, 255, 128),
                                    (512, 513, 192), (16, 4096, 64), (300, 70000, 64),
                                    (127, 257, 64), (128, 70000, 192), (129, 513, 128),
-                                   (384, 4097, 64), (385, 8192, 64)])
+                                   (384, 4097, 64), (385, 8192, 64), (140, 60000, 64),
+                                   (191, 70000, 64), (192, 70001, 128), (383, 70000, 64)])
 def test_tile_and_ring_edges(N, V, D):
-    """Token blocks, vocab tiles and K stages at and around their sizes (256
-    or 128, 256 and 64 columns: fewer stages than the rings hold up to several tiles
+    """Token blocks, vocab tiles and K stages at and around their sizes (256,
+    192 or 128, 256 and 64 columns: fewer stages than the rings hold up to several tiles
     a workgroup), with every row of a tile as some token's target."""
     h, w, t = make(N, V, D, seed=31 + N + V + D)
     t = torch.arange(N) * max(1, (V + 255) // 256) % V
@@ -172,7 +174,7 @@ def test_invalid_arguments_raise():
 
 
 # ---------------------------------------------------------------------------
-# Backward (klp_lmh_bwd_logits + library GEMMs)
+# Backward (klp_lmh_bwd_logits, then the two products)
 # ---------------------------------------------------------------------------
 def _grads(N, V, seed):
     g = torch.Generator().manual_seed(seed)
@@ -279,19 +281,25 @@ def test_backward_matches_unfused_path(impl):
 
 
 # ---------------------------------------------------------------------------
-# Chunked head (library GEMM per vocabulary chunk + klp_fwd_shard / merge)
+# Chunked head (MFMA kernels, or a library GEMM and klp_fwd_chunk per chunk)
 # ---------------------------------------------------------------------------
 SIG_BITS = {torch.bfloat16: 8, torch.float16: 11, torch.float32: 24}
 
 
 def _chunk_logits(hd, wd, plan):
-    """The logits the chunked head computes: the same GEMM call per chunk of
-    ``plan`` (a vocab_chunks list, or a width for equal chunks; the GEMM is
-    deterministic, so the values are bit-identical to the head's own),
-    concatenated."""
-    from kernel_opt import lmhead
+    """The logits the chunked head computes: klp_lmh_logits' where the MFMA
+    kernels take the operands (the same values for every chunk), else the same
+    library GEMM per chunk of ``plan`` (a vocab_chunks list, or a width for
+    equal chunks; the GEMM is deterministic, so the values are bit-identical
+    to the head's own), concatenated."""
+    from kernel_opt import _head, lmhead
+    from kernel_opt._library import stream_handle
     h2 = hd.reshape(-1, hd.size(-1))
     N, V = h2.size(0), wd.size(0)
+    if _head.mfma_operands(h2, wd):
+        out = torch.empty(N, V, dtype=hd.dtype, device=DEV)
+        _head.logits_into(out, h2, wd, stream_handle(0))
+        return out
     if isinstance(plan, int):
         plan = [(c0, min(plan, V - c0)) for c0 in range(0, V, plan)]
     parts = []
@@ -313,17 +321,29 @@ CHUNK_CASES = [  # N, V, D, dtype, chunk_vocab, temperature
     (64, 5000, 96, torch.float16, 1024, 1.3),
     (50, 2001, 80, torch.float32, 500, None),
     (300, 20000, 512, torch.bfloat16, None, None),
+    # hidden sizes that the library takes; the default plan in three chunks
+    (40, 70001, 80, torch.bfloat16, None, None),
+    (90, 3001, 80, torch.bfloat16, 700, 0.7),
 ]
 
 
 @pytest.mark.parametrize("N,V,D,dtype,chunk,T", CHUNK_CASES)
 def test_chunked_forward(N, V, D, dtype, chunk, T, oracle):
+    from kernel_opt import _head
+    h, w, t = make(N, V, D, seed=40 + N + V, dtype=dtype)
+    hd, wd = h.to(DEV), w.to(DEV)
+    assert _head.mfma_operands(hd, wd) == (dtype != torch.float32 and D % 64 == 0)
+    _check_chunked_forward(h, w, t, hd, wd, chunk, T, oracle)
+
+
+def _check_chunked_forward(h, w, t, hd, wd, chunk, T, oracle):
+    """``hd``, ``wd``: the operands on the GPU, in the layout under test."""
     from kernel_opt import fused_linear_logprob_entropy_forward, vocab_chunks
     from klp_testutil import FWD_TOL
-    h, w, t = make(N, V, D, seed=40 + N + V, dtype=dtype)
+    (N, D), V, dtype = h.shape, w.size(0), h.dtype
     t[::7] = -100
     t[3::11] = V
-    hd, wd, td = h.to(DEV), w.to(DEV), t.to(DEV)
+    td = t.to(DEV)
     lp, ent, lse = fused_linear_logprob_entropy_forward(hd, wd, td, T, chunk_vocab=chunk)
     x = _chunk_logits(hd, wd, vocab_chunks(N, V, h.element_size(), chunk))
     # (1) the logprob bar on the logits the chunks computed
@@ -390,6 +410,9 @@ BWD_CASES = [  # N, V, D, dtype, chunk_vocab, temperature, need_w
     (33, 2001, 64, torch.bfloat16, 333, None, False),
     (100, 3000, 128, torch.float16, 1024, 1.3, True),
     (50, 2001, 80, torch.float32, 500, None, True),
+    # hidden sizes that the library takes; the default plan in three chunks
+    (50, 2001, 80, torch.bfloat16, 500, 0.7, True),
+    (40, 70001, 96, torch.float16, None, None, True),
 ]
 
 
@@ -399,13 +422,22 @@ def test_chunked_backward(N, V, D, dtype, chunk, T, need_w, oracle):
     logits: d_logits within one rounding to the input dtype (plus the fp32
     evaluation noise of its row), carried through the two products, whose
     outputs are rounded once more and accumulate in fp32."""
-    from kernel_opt import fused_linear_logprob_entropy, vocab_chunks
+    from kernel_opt import _head
     h, w, t = make(N, V, D, seed=60 + N, dtype=dtype)
+    hd, wd = h.to(DEV), w.to(DEV)
+    assert _head.mfma_operands(hd, wd) == (dtype != torch.float32 and D % 64 == 0)
+    _check_chunked_backward(h, w, t, hd, wd, chunk, T, need_w, oracle)
+
+
+def _check_chunked_backward(h, w, t, hd, wd, chunk, T, need_w, oracle):
+    """``hd``, ``wd``: the operands on the GPU, in the layout under test."""
+    from kernel_opt import fused_linear_logprob_entropy, vocab_chunks
+    N, V, dtype = h.size(0), w.size(0), h.dtype
     t[::9] = -100
     t[1::13] = V
     gl, ge, gs = _grads(N, V, 61)
-    hd = h.to(DEV).requires_grad_(True)
-    wd = w.to(DEV).requires_grad_(need_w)
+    hd.requires_grad_(True)
+    wd.requires_grad_(need_w)
     td = t.to(DEV)
     lp, ent, lse = fused_linear_logprob_entropy(hd, wd, td, T, chunk_vocab=chunk)
     ((lp * gl.to(DEV)).sum() + (ent * ge.to(DEV)).sum() + (lse * gs.to(DEV)).sum()).backward()
@@ -429,6 +461,27 @@ def test_chunked_backward(N, V, D, dtype, chunk, T, need_w, oracle):
         assert np.all(err_w <= bound_w), f"d_weight: {(err_w / bound_w).max():.3g}x the bound"
     else:
         assert wd.grad is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("stride,first", [(132, 0), (136, 1), (128, 4)])
+@pytest.mark.parametrize("which", ["hidden", "weight"])
+def test_unaligned_rows_take_the_library(dtype, stride, first, which, oracle):
+    """A hidden size that the kernels take, in rows that are not 16-byte
+    aligned: a row stride or a first element that is not a multiple of 8."""
+    from kernel_opt import _head
+
+    def place(x, moved):
+        if not moved:
+            return x.to(DEV)
+        buf = torch.zeros(x.size(0) * stride + first, dtype=dtype, device=DEV)
+        return buf[first:].as_strided(x.shape, (stride, 1), first).copy_(x)
+
+    h, w, t = make(70, 1501, 128, seed=71, dtype=dtype)
+    hd, wd = place(h, which == "hidden"), place(w, which == "weight")
+    assert not _head.mfma_operands(hd, wd)
+    _check_chunked_forward(h, w, t.clone(), hd, wd, 400, 0.7, oracle)
+    _check_chunked_backward(h, w, t, hd, wd, 400, 0.7, True, oracle)
 
 
 def test_chunked_holds_no_full_logits():

@@ -9,6 +9,11 @@ Bars:
     same chunk GEMMs (grpo_step_launch with the same per-token weights, then
     d_hidden = d_logits @ W and d_weight accumulated chunk by chunk in float32):
     equal, so the chunking itself adds nothing;
+    (both of these at sizes whose products the library runs);
+  * the same with the logits, d_hidden and d_weight kernels selected: loss,
+    logp and entropy equal to the per-chunk composition on klp_lmh_logits'
+    logits, d_hidden and d_weight within the float32 sums' bound of float64
+    products of its d_logits;
   * a small case against the float64 oracle (oracle/grpo_step_oracle.py on the
     GEMM's bf16 logits, then float64 products): logp / entropy within 2e-5,
     the loss within 1e-5 relative, d_hidden and d_weight within
@@ -191,24 +196,68 @@ def test_frozen_weight_and_scaled_loss():
     assert torch.equal(hc.grad, hb.grad) and torch.equal(wc.grad, wb.grad)
 
 
+@pytest.mark.parametrize("B,S,D,V,chunk", [(2, 256, 1088, 30008, 512), (1, 1204, 1088, 100008, 512)])
+def test_kernels_products_match_float64(B, S, D, V, chunk):
+    """The MFMA kernels in their places, one chunk and several with a shorter
+    last one (d_weight then accumulates through the library)."""
+    from kernel_opt import _head
+    from kernel_opt._library import stream_handle
+    from kernel_opt.grpo_step import grpo_step_launch, grpo_token_weights
+    ko = _ko()
+    h, w, t, mask, adv, old, ref = make(B, S, D, V, seed=41)
+    N = B * S
+    chunks = [(n0, min(N, n0 + chunk)) for n0 in range(0, N, chunk)]
+    assert _head.mfma_operands(h.view(N, D), w) and _head.d_weight_pays(V, D)
+    for n0, n1 in chunks:
+        assert _head.logits_pay(n1 - n0, V, D) and _head.d_hidden_pays(n1 - n0, V, D)
+    ha = h.clone().requires_grad_(True)
+    wa = w.clone().requires_grad_(True)
+    loss, lp, ent = ko.fused_linear_grpo_step(ha, wa, t, old, adv, mask, ref, chunk_tokens=chunk,
+                                              **KW)
+    loss.backward()
+    h2 = h.view(N, D)
+    wts = grpo_token_weights(mask, "grpo").reshape(-1).contiguous()
+    adv_t = adv.unsqueeze(1).expand(B, S).reshape(-1).contiguous()
+    flat = lambda x: x.reshape(-1).contiguous()  # noqa: E731
+    lps, ents, lts = [], [], []
+    w64 = w.double()
+    dw, dw_mag = torch.zeros_like(w64), torch.zeros_like(w64)
+    for n0, n1 in chunks:
+        c = n1 - n0
+        logits = torch.empty(c, V, dtype=h.dtype, device=DEV)
+        _head.logits_into(logits, h2[n0:n1], w, stream_handle(0))
+        a, b, _, lt, d = grpo_step_launch(logits.view(1, c, V), flat(t)[n0:n1].view(1, c),
+                                          flat(old)[n0:n1], flat(ref)[n0:n1], adv_t[n0:n1],
+                                          wts[n0:n1], (1.0, 0.2, 0.28, 0.04, 1, 1.0))
+        lps.append(a.view(-1)); ents.append(b.view(-1)); lts.append(lt.view(-1))
+        d64, h64 = d.view(c, V).double(), h2[n0:n1].double()
+        exact, mag = d64 @ w64, d64.abs() @ w64.abs()
+        err = (ha.grad.view(N, D)[n0:n1].double() - exact).abs()
+        # V products summed in float32 and one rounding to bf16
+        assert torch.all(err <= V * 2.0 ** -24 * mag + 2.0 ** -8 * exact.abs() + 1e-30)
+        dw += d64.t() @ h64
+        dw_mag += d64.t().abs() @ h64.abs()
+    assert torch.equal(lp.view(-1), torch.cat(lps)) and torch.equal(ent.view(-1), torch.cat(ents))
+    assert torch.equal(loss, torch.cat(lts).sum())
+    err = (wa.grad.double() - dw).abs()
+    assert torch.all(err <= N * 2.0 ** -24 * dw_mag + 2.0 ** -8 * dw.abs() + 1e-30)
+
+
 def test_qwen_head_shape_chunks():
     """Qwen2.5-7B's head (D = 3584, V = 152064) with 1024 tokens in chunks of
-    384 against one chunk: the loss within 1e-5 relative; logp / entropy equal
-    where the chunk GEMMs reproduce the full GEMM's logits, else within twice
-    the row's largest logit difference (logp and H move by at most that)."""
+    384 against one chunk.  klp_lmh_logits sums every logit in the same order
+    whatever the chunk, so the losses agree within 1e-5 relative and logp /
+    entropy within the 2e-5 of their reductions."""
+    from kernel_opt import _head
     ko = _ko()
+    assert all(_head.logits_pay(n, 152064, 3584) for n in (384, 256, 1024))
     h, w, t, mask, adv, old, ref = make(4, 256, 3584, 152064, seed=6)
     B, S, D = h.shape
     out_a = ko.fused_linear_grpo_step(h, w, t, old, adv, mask, ref, chunk_tokens=384, **KW)
     out_b = ko.fused_linear_grpo_step(h, w, t, old, adv, mask, ref, chunk_tokens=1024, **KW)
     assert abs(out_a[0].item() - out_b[0].item()) <= 1e-5 * max(1.0, abs(out_b[0].item()))
-    h2 = h.view(-1, D)
-    full = torch.mm(h2, w.t())
-    chunked = torch.cat([torch.mm(h2[n0:n0 + 384], w.t()) for n0 in range(0, B * S, 384)])
-    dx = (full.float() - chunked.float()).abs().amax(dim=-1).view(B, S)
-    del full, chunked
     for a, b in zip(out_a[1:], out_b[1:]):
-        assert torch.all((a - b).abs() <= 2 * dx + 2e-5)
+        assert torch.all((a - b).abs() <= 2e-5)
 
 
 def test_default_chunking_is_one_chunk_when_it_fits():

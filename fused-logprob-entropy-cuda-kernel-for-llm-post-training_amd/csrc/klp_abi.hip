@@ -507,9 +507,9 @@ int grpo_setup(const float* logp, const float* old_logp, const float* ref_logp,
 //   1280                  209 / 231      250 / 286      38 / 33
 // and 256 or 128, as the rule without 192 chose / the rule:
 //   N     [152064, 3584]  [151936, 2048]  [32000, 4096]  [100000, 1024]
-//   260   429-432 / 373   238 / 201
-//   320   432 / 368                       106 / 92       86 / 86
-//   560   603 / 517                                      129 / 111
+//   260   428-432 / 373   238 / 201                      (330) 86 / 86
+//   320   432 / 368                       106 / 92
+//   560   603 / 517                                      (550) 129 / 111
 //   1100  958 / 940                                      224 / 206
 struct LmhPlan {
     int block_tokens;

@@ -596,9 +596,9 @@ int head_gemm_check(int dtype, const void* d_logits, int64_t ld_d, int64_t n_tok
         return fail(KLP_EINVAL,
                     "row strides must be multiples of 8 elements, at least dim and vocab rounded "
                     "up to 8");
-    if (ld_d > INT32_MAX / 512 || ld_other > INT32_MAX / 512)
-        return fail(KLP_EINVAL, "row strides above %d elements are not supported",
-                    INT32_MAX / 512);
+    if (ld_d > klp::kLmhMaxStride || ld_other > klp::kLmhMaxStride)
+        return fail(KLP_EINVAL, "row strides above %lld elements are not supported",
+                    static_cast<long long>(klp::kLmhMaxStride));
     if (n_tokens > INT32_MAX / 2 || vocab > INT32_MAX / 2 || dim > INT32_MAX / 2)
         return fail(KLP_EINVAL, "n_tokens, vocab and dim must be below 2^30");
     if (n_tokens == 0) return KLP_OK;
@@ -1185,10 +1185,11 @@ size_t klp_lmh_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t dim) {
 }
 
 // Checks shared by klp_lmh_fwd and klp_lmh_bwd_logits; fills the GEMM part
-// of `p`.  Returns KLP_OK, or an error (after fail()).
+// of `p`.  `far_rows`: row strides of any size are taken.  Returns KLP_OK, or
+// an error (after fail()).
 int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t ld_weight,
               int64_t n_tokens, int64_t vocab, int64_t dim, const int64_t* targets,
-              float temperature, klp::LmhParams* p) {
+              float temperature, bool far_rows, klp::LmhParams* p) {
     if (n_tokens < 0) return fail(KLP_EINVAL, "n_tokens must be >= 0");
     if (vocab < 1) return fail(KLP_EINVAL, "vocab must be >= 1, got %lld",
                                static_cast<long long>(vocab));
@@ -1197,10 +1198,10 @@ int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
                     static_cast<long long>(dim));
     if (ld_hidden < dim || ld_weight < dim || ld_hidden % 8 != 0 || ld_weight % 8 != 0)
         return fail(KLP_EINVAL, "row strides must be >= dim and multiples of 8 elements");
-    // The kernels address 256 rows with 32-bit byte offsets.
-    if (ld_hidden > INT32_MAX / 512 || ld_weight > INT32_MAX / 512)
-        return fail(KLP_EINVAL, "row strides above %d elements are not supported",
-                    INT32_MAX / 512);
+    p->far = ld_hidden > klp::kLmhMaxStride || ld_weight > klp::kLmhMaxStride;
+    if (p->far && !far_rows)
+        return fail(KLP_EINVAL, "row strides above %lld elements are not supported",
+                    static_cast<long long>(klp::kLmhMaxStride));
     if (n_tokens > (int64_t{1} << 31) - 1 || vocab > (int64_t{1} << 31) - 1)
         return fail(KLP_EINVAL, "n_tokens and vocab must be below 2^31");
     float scale;
@@ -1222,8 +1223,8 @@ int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
     p->targets = targets;
     p->scale = scale;
     const LmhPlan plan = lmh_plan(n_tokens, vocab);
-    p->block_tokens = plan.block_tokens;
-    p->n_tblocks = (n_tokens + plan.block_tokens - 1) / plan.block_tokens;
+    p->block_tokens = p->far ? 256 : plan.block_tokens;
+    p->n_tblocks = ceil_div(n_tokens, p->block_tokens);
     p->n_vtiles = klp::lmh_vocab_tiles(vocab);
     p->tiles_per_chunk = plan.tiles_per_chunk;
     p->n_chunks = plan.n_chunks;
@@ -1244,7 +1245,7 @@ static int lmh_bwd_impl(int dtype, bool rounded, const void* hidden, int64_t ld_
                         void* d_logits, int64_t ld_d, int64_t pad, void* stream) {
     klp::LmhParams p;
     int rc = lmh_setup(hidden, ld_hidden, weight, ld_weight, n_tokens, vocab, dim, targets,
-                       temperature, &p);
+                       temperature, dtype == KLP_BF16 && !rounded, &p);
     if (rc != KLP_OK) return rc;
     if (n_tokens == 0) return ok();
     if ((rc = check_f32(lse, "lse")) != KLP_OK) return rc;
@@ -1315,7 +1316,7 @@ int klp_lmh_logits(int dtype, const void* hidden, int64_t ld_hidden, const void*
     klp::LmhParams p;
     static const int64_t no_targets = 0;  // not read
     rc = lmh_setup(hidden, ld_hidden, weight, ld_weight, n_tokens, vocab, dim, &no_targets, 1.0f,
-                   &p);
+                   false, &p);
     if (rc != KLP_OK) return rc;
     if (n_tokens == 0) return ok();
     p.targets = nullptr;
@@ -1420,7 +1421,7 @@ static int lmh_fwd_impl(int dtype, bool rounded, const void* hidden, int64_t ld_
                         void* stream) {
     klp::LmhParams p;
     int rc = lmh_setup(hidden, ld_hidden, weight, ld_weight, n_tokens, vocab, dim, targets,
-                       temperature, &p);
+                       temperature, dtype == KLP_BF16 && !rounded, &p);
     if (rc != KLP_OK) return rc;
     if (n_tokens == 0) return ok();
     if ((rc = check_f32(logprob, "logprob")) != KLP_OK) return rc;

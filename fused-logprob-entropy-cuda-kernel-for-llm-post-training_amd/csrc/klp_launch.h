@@ -220,6 +220,7 @@ struct LmhParams {
     float scale;             // 1 / temperature
     float* partials;         // [n_chunks, n_tokens] float4 (m, z, t, unused)
     float* target_logit;     // [n_tokens], behind the partials; written where a target is valid
+    bool far;                // a row stride above kLmhMaxStride: bf16, float32 logits
     int block_tokens;        // tokens per workgroup: 256, 192 or 128
     int64_t n_tblocks;       // ceil(n_tokens / block_tokens)
     int64_t n_vtiles;        // ceil(vocab / 256)
@@ -242,6 +243,8 @@ struct LmhParams {
     int out_align;
 };
 int64_t lmh_vocab_tiles(int64_t vocab);
+// The longest row stride whose 256 rows 32-bit byte offsets reach.
+constexpr int64_t kLmhMaxStride = INT32_MAX / 512;
 // `rounded`: logits rounded once to `dtype` (bf16 or fp16); otherwise bf16
 // operands and float32 logits.
 hipError_t launch_lmh_fwd(int dtype, bool rounded, const LmhParams& p, hipStream_t stream);

@@ -89,7 +89,10 @@ enum : int { kFold = 0, kGradient = 1, kLogits = 2 };
 // rounded to DT before it is scaled and used, as a GEMM that writes DT does.
 // kTokBlocks: 16-token blocks per wave, 8, 6 or 4 (256, 192 or 128 tokens a
 // workgroup).
-template <int DT, int kMode, bool kRound, bool kScaled, int kTokBlocks>
+// kFar: row strides of any size (the others address a block's rows with 32-bit
+// offsets): every lane copies from a 64-bit address of its own, and rows past
+// the matrix's end are its last one instead of zeros.
+template <int DT, int kMode, bool kRound, bool kScaled, int kTokBlocks, bool kFar>
 __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     constexpr int kTokSide = 16 * kTokBlocks;  // a wave's tokens
     constexpr int kBT = 2 * kTokSide;          // the workgroup's
@@ -149,10 +152,20 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
     int64_t w_tile = tile_first;
     int w_k = 0, w_slot = 0, h_k = 0, h_slot = 0;
     __amdgpu_buffer_rsrc_t w_rs = tile_rsrc(w_tile);
+    // kFar: this lane's 16 bytes of `row` (or of the last row), stage k.
+    auto copy_far = [&](const uint16_t* base, int64_t row, int64_t rows, int64_t ld, int k,
+                        unsigned char* to) {
+        if (row > rows - 1) row = rows - 1;
+        __builtin_amdgcn_global_load_lds(base + row * ld + k * kBK + cchunk * 8, (lds_void*)to, 16,
+                                         0, 0);
+    };
     auto copy_w = [&](int j) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            w_rs, (lds_void*)(lds + w_slot * kSlotBytes + (wave + 4 * j) * 1024), 16, w_off,
-            j * w_step + w_k * kRowBytes, 0, 0);
+        unsigned char* to = lds + w_slot * kSlotBytes + (wave + 4 * j) * 1024;
+        if constexpr (kFar)
+            copy_far(p.weight, w_tile * kBV + 32 * j + crow, p.vocab, p.ld_weight, w_k, to);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rs, (lds_void*)to, 16, w_off,
+                                                     j * w_step + w_k * kRowBytes, 0, 0);
         if (j == kCopies - 1) {
             if (++w_k == n_k) {
                 w_k = 0;
@@ -162,9 +175,12 @@ __global__ __launch_bounds__(kThreads) void klp_lmh_kernel(LmhParams p) {
         }
     };
     auto copy_h = [&](int j) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            h_rs, (lds_void*)(lds + kTokRing + h_slot * kTokSlot + (wave + 4 * j) * 1024), 16,
-            h_off, j * h_step + h_k * kRowBytes, 0, 0);
+        unsigned char* to = lds + kTokRing + h_slot * kTokSlot + (wave + 4 * j) * 1024;
+        if constexpr (kFar)
+            copy_far(p.hidden, tok0 + 32 * j + crow, p.n_tokens, p.ld_hidden, h_k, to);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(h_rs, (lds_void*)to, 16, h_off,
+                                                     j * h_step + h_k * kRowBytes, 0, 0);
         if (j == kTokBlocks - 1) {
             if (++h_k == n_k) h_k = 0;
             h_slot ^= 1;
@@ -475,13 +491,19 @@ static hipError_t launch_lmh_s(const LmhParams& p, hipStream_t stream) {
     // padding workgroups exit at once.
     const int64_t chunks8 = (p.n_chunks + 7) / 8 * 8;
     const dim3 grid(static_cast<unsigned>(chunks8 * p.n_tblocks));
+    if constexpr (DT == kBF16 && kMode != kLogits && !kRound) {
+        if (p.far)
+            return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 8, true>, grid,
+                                 dim3(kThreads), stream, p);
+    }
+    if (p.far) return hipErrorInvalidValue;
     if (p.block_tokens == 192)
-        return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 6>, grid, dim3(kThreads),
+        return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 6, false>, grid, dim3(kThreads),
                              stream, p);
     if (p.block_tokens == 128)
-        return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 4>, grid, dim3(kThreads),
+        return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 4, false>, grid, dim3(kThreads),
                              stream, p);
-    return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 8>, grid, dim3(kThreads),
+    return launch_kernel(klp_lmh_kernel<DT, kMode, kRound, kScaled, 8, false>, grid, dim3(kThreads),
                          stream, p);
 }
 

@@ -82,8 +82,8 @@ def _ld(t: torch.Tensor) -> int:
 
 
 def _rows_32bit(t: torch.Tensor) -> torch.Tensor:
-    """``t``, or its contiguous copy where the MFMA kernels' 32-bit offsets
-    within 256 rows would not reach (row strides above 4194303 elements)."""
+    """``t``, or its contiguous copy where the products' 32-bit offsets within
+    256 rows would not reach (row strides above 4194303 elements)."""
     return t if _ld(t) <= MAX_LD else t.contiguous()
 
 
@@ -385,7 +385,7 @@ def fused_linear_logprob_entropy_forward(hidden: torch.Tensor, weight: torch.Ten
     if not (T > 0.0 and T != float("inf")):
         raise RuntimeError(f"temperature must be finite and > 0, got {T}")
     if impl == "mfma":
-        _forward_mfma(_rows_32bit(h2), _rows_32bit(weight), t, T, False, out)
+        _forward_mfma(h2, weight, t, T, False, out)
     elif mfma_operands(h2, weight):
         if chunk_vocab is not None and chunk_vocab < 1:
             raise ValueError(f"chunk_vocab must be >= 1, got {chunk_vocab}")

@@ -485,7 +485,8 @@ int klp_lmh_bwd_logits(const void* hidden, int64_t ld_hidden, const void* weight
  * holds round_up(vocab, 8) columns; columns vocab .. round_up(vocab, 8) - 1
  * are written with 0.  klp_lmh_logits writes the rounded logits themselves
  * ([n_tokens, ld_logits], ld_logits >= vocab): the values the rounded forms
- * use, bit for bit.
+ * use, bit for bit.  Row strides of hidden and weight above 4194303 elements
+ * (32-bit byte offsets within 256 rows) are taken with `rounded` zero only.
  */
 int klp_lmh_fwd_as(int dtype, int rounded, const void* hidden, int64_t ld_hidden,
                    const void* weight, int64_t ld_weight, int64_t n_tokens, int64_t vocab,

@@ -660,6 +660,28 @@ def test_lm_head_as_rejects_bad_arguments():
     assert lib.klp_lmh_logits(0, P, 64, P, 64, 4, 100, 64, P, 96, None) != 0 and ">= vocab" in error()
 
 
+def test_lm_head_takes_row_strides_of_any_size():
+    """Hidden states of one token a sequence, hidden[:, -1], have the whole
+    sequence as their row stride: klp_lmh_fwd and klp_lmh_bwd_logits get past
+    it to their next check; the rounded forms refuse it."""
+    from kernel_opt._library import lib
+
+    def error():
+        buf = ctypes.create_string_buffer(512)
+        lib.klp_last_error(buf, 512)
+        return buf.value.decode()
+
+    far = 8192 * 3584
+    for ld_h, ld_w in ((far, 64), (64, far)):
+        rc = lib.klp_lmh_fwd(P, ld_h, P, ld_w, 4, 100, 64, P, 1.0, P, P, P, None, 0, None)
+        assert rc != 0 and "workspace" in error()
+        rc = lib.klp_lmh_bwd_logits(P, ld_h, P, ld_w, 4, 100, 64, P, 1.0, None, P, P, P, P, P, 104,
+                                    None)
+        assert rc != 0 and "lse" in error()
+        rc = lib.klp_lmh_fwd_as(0, 1, P, ld_h, P, ld_w, 4, 100, 64, P, 1.0, P, P, P, None, 0, None)
+        assert rc != 0 and "not supported" in error()
+
+
 @pytest.mark.parametrize("kw,message", [
     (dict(dtype=3), "mask dtype"), (dict(mask=None), "mask"), (dict(dtype=2, mask=4), "mask"),
     (dict(mask_out=None), "mask_out"), (dict(B=0), "n_seqs"), (dict(loss=None), "loss")])

@@ -129,6 +129,37 @@ def test_strided_hidden_and_leading_dims():
     assert outs[0].shape == (3, 40)
 
 
+@pytest.mark.parametrize("which", ["hidden", "weight"])
+@pytest.mark.parametrize("N,V,D,T", [(2, 300, 64, None), (290, 600, 192, 0.7)])
+def test_row_strides_past_32_bits(N, V, D, T, which):
+    """256 rows further apart than 32-bit byte offsets reach: the bits of the
+    same rows side by side, forward, d_logits and gradients."""
+    import ctypes
+
+    from kernel_opt import fused_linear_logprob_entropy, fused_linear_logprob_entropy_forward
+    from kernel_opt._library import check_status, lib, stream_handle
+    h, w, t = (x.to(DEV) for x in make(N, V, D, seed=72))
+    ld = 4194304 + 8
+    near = h if which == "hidden" else w
+    far = torch.empty((near.size(0) - 1) * ld + D, dtype=near.dtype, device=DEV)
+    far = far.as_strided(near.shape, (ld, 1)).copy_(near)
+    P = lambda a: ctypes.c_void_p(a.data_ptr())  # noqa: E731
+    res = []
+    for x in (near, far):
+        hd, wd = (x, w) if which == "hidden" else (h, x)
+        outs = fused_linear_logprob_entropy_forward(hd, wd, t, T, impl="mfma")
+        d = torch.empty(N, V, dtype=torch.bfloat16, device=DEV)
+        check_status(lib.klp_lmh_bwd_logits(
+            P(hd), hd.stride(0), P(wd), wd.stride(0), N, V, D, P(t), T or 1.0, P(outs[2]),
+            P(outs[1]), P(outs[0]), P(outs[1]), P(outs[0]), P(d), V, stream_handle(0)))
+        ha, wa = hd.detach().requires_grad_(True), wd.detach().requires_grad_(True)
+        lp, ent, _ = fused_linear_logprob_entropy(ha, wa, t, T, impl="mfma")
+        grads = torch.autograd.grad((lp.sum() + ent.sum()), (ha, wa))
+        res.append((*outs, d, *grads))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
 def test_matches_unfused_path_up_to_bf16_logit_rounding():
     """The unfused path (bf16 matmul, then the logprob kernel) rounds every
     logit to bf16; the fused one does not.  Both stay within the bf16

@@ -1198,8 +1198,8 @@ int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
                     static_cast<long long>(dim));
     if (ld_hidden < dim || ld_weight < dim || ld_hidden % 8 != 0 || ld_weight % 8 != 0)
         return fail(KLP_EINVAL, "row strides must be >= dim and multiples of 8 elements");
-    p->far = ld_hidden > klp::kLmhMaxStride || ld_weight > klp::kLmhMaxStride;
-    if (p->far && !far_rows)
+    const bool far = ld_hidden > klp::kLmhMaxStride || ld_weight > klp::kLmhMaxStride;
+    if (far && !far_rows)
         return fail(KLP_EINVAL, "row strides above %lld elements are not supported",
                     static_cast<long long>(klp::kLmhMaxStride));
     if (n_tokens > (int64_t{1} << 31) - 1 || vocab > (int64_t{1} << 31) - 1)
@@ -1223,7 +1223,8 @@ int lmh_setup(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
     p->targets = targets;
     p->scale = scale;
     const LmhPlan plan = lmh_plan(n_tokens, vocab);
-    p->block_tokens = p->far ? 256 : plan.block_tokens;
+    p->far = far;
+    p->block_tokens = far ? 256 : plan.block_tokens;
     p->n_tblocks = ceil_div(n_tokens, p->block_tokens);
     p->n_vtiles = klp::lmh_vocab_tiles(vocab);
     p->tiles_per_chunk = plan.tiles_per_chunk;

@@ -130,7 +130,7 @@ def test_strided_hidden_and_leading_dims():
 
 
 @pytest.mark.parametrize("which", ["hidden", "weight"])
-@pytest.mark.parametrize("N,V,D,T", [(2, 300, 64, None), (290, 600, 192, 0.7)])
+@pytest.mark.parametrize("N,V,D,T", [(2, 300, 64, None), (290, 520, 192, 0.7)])
 def test_row_strides_past_32_bits(N, V, D, T, which):
     """256 rows further apart than 32-bit byte offsets reach: the bits of the
     same rows side by side, forward, d_logits and gradients."""
@@ -139,7 +139,7 @@ def test_row_strides_past_32_bits(N, V, D, T, which):
     from kernel_opt import fused_linear_logprob_entropy, fused_linear_logprob_entropy_forward
     from kernel_opt._library import check_status, lib, stream_handle
     h, w, t = (x.to(DEV) for x in make(N, V, D, seed=72))
-    ld = 4194304 + 8
+    ld = 4 * 4194304 + 8  # row 128 starts past 2^32 bytes
     near = h if which == "hidden" else w
     far = torch.empty((near.size(0) - 1) * ld + D, dtype=near.dtype, device=DEV)
     far = far.as_strided(near.shape, (ld, 1)).copy_(near)

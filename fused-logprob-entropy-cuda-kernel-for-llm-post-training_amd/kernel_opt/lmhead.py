@@ -95,7 +95,8 @@ def _rows_32bit(t: torch.Tensor) -> torch.Tensor:
 # while one chunk of logits would exceed CHUNK_MAX_BYTES, half of the 256 MB
 # Infinity Cache, so that the logprob pass over a chunk reads it from the
 # cache.  The library GEMM's speed at the chunk shape dominates, and it does
-# not follow the width monotonically.  Measured at Qwen2.5-7B's head
+# not follow the width monotonically.  Measured at Qwen2.5-7B's head in bf16
+# while it ran this path, which heads that the MFMA kernels take no longer do
 # (V = 152064, D = 3584; forward, forward + backward, ms; two runs):
 #   1024 tokens: 32768 columns 0.934-0.940, 4.75-4.76; balanced 15360
 #                0.975-0.979, 4.79; unfused 0.927-0.932, 3.84
@@ -166,12 +167,22 @@ def vocab_chunks(n_tokens: int, vocab: int, elem_bytes: int = 2,
 #                   4096       14.21-14.32 / 14.04-14.08 8192  34.7 / 29.1
 #   [100000, 1024]  2000         1.90 / 1.62-1.63
 #   [50240, 2048]   2048         1.59 / 1.47             1024  0.87-0.88 / 0.85-0.86
-MFMA_CHUNK_TOKENS = 1024
-MFMA_CHUNK_BYTES = 64 << 20
-MFMA_CHUNK_MAX_BYTES = 128 << 20
+# From about 8192 tokens on, 128 MiB are fewer than 8192 columns: each chunk
+# moves the accumulator and its slab (16 bytes a value of d_hidden) for a K that
+# shrinks as the batch grows.  A chunk then has about 8192 columns, in whole
+# rounds, whatever their bytes up to 8 GiB.  Forward + backward, ms, 128 MiB /
+# 8192 columns (in brackets the library path's chunks of 1024-4096 columns):
+#   [152064, 3584]  16384 tokens 67 / 58.6 [63]   65536  399-407 / 235 [291]
+#   [32000, 4096]  131072       326 / 110 [136]
+#   [50257, 768]   131072       146 / 40.7 [79]  400000  754 / 126 [205]
 # A chunk's columns are the row stride of its d_logits, which the products
 # address with 32-bit offsets: few tokens of millions of columns take several.
 MFMA_CHUNK_MAX_COLS = MAX_LD // 256 * 256
+MFMA_CHUNK_TOKENS = 1024
+MFMA_CHUNK_BYTES = 64 << 20
+MFMA_CHUNK_ROUNDS_BYTES = 128 << 20
+MFMA_CHUNK_MIN_TILES = 32
+MFMA_CHUNK_MAX_BYTES = 8 << 30
 
 
 def _mfma_chunks(n_tokens: int, vocab: int, chunk_vocab: int | None) -> list:
@@ -182,10 +193,14 @@ def _mfma_chunks(n_tokens: int, vocab: int, chunk_vocab: int | None) -> list:
         n_chunks = max(1, -(-(n_tokens * vocab * 2) // MFMA_CHUNK_BYTES))
         cols = -(-(-(-vocab // n_chunks)) // 256) * 256
     else:
-        tiles = MFMA_CHUNK_MAX_BYTES // (2 * n_tokens * 256)
+        tile_bytes = 2 * n_tokens * 256
+        tiles = MFMA_CHUNK_ROUNDS_BYTES // tile_bytes
         if tiles * 256 < vocab:
             token_blocks = -(-n_tokens // 256)
-            tiles = max(1, tiles * token_blocks // 256 * 256 // token_blocks)
+            tiles = tiles * token_blocks // 256 * 256 // token_blocks
+            if tiles < MFMA_CHUNK_MIN_TILES:
+                tiles = -(-MFMA_CHUNK_MIN_TILES * token_blocks // 256) * 256 // token_blocks
+            tiles = max(1, min(tiles, MFMA_CHUNK_MAX_BYTES // tile_bytes))
         cols = tiles * 256
     cols = min(cols, MFMA_CHUNK_MAX_COLS)
     return [(c0, min(cols, vocab - c0)) for c0 in range(0, vocab, cols)]
@@ -369,8 +384,9 @@ def fused_linear_logprob_entropy_forward(hidden: torch.Tensor, weight: torch.Ten
             multiple of 64, both row strides multiples of 8).
         chunk_vocab: columns per vocabulary chunk where a pass walks the
             vocabulary in chunks (the backward; the forward of heads without
-            MFMA kernels); default :func:`vocab_chunks`, or chunks of 64 MiB
-            of d_logits.
+            MFMA kernels); default :func:`vocab_chunks`, or, with them, chunks
+            of d_logits of 64 MiB up to 1024 tokens, 128 MiB above and 8192
+            columns from about 8192 tokens on.
 
     Returns ``(logprob, entropy, lse)``, float32, shaped like ``targets``.
     """

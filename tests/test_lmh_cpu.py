@@ -188,3 +188,18 @@ def test_mfma_backward_chunks_stay_within_the_row_stride(n_tokens, chunk_vocab):
     assert [c0 for c0, _ in plan] == [sum(n for _, n in plan[:i]) for i in range(len(plan))]
     assert sum(n for _, n in plan) == 9000001
     assert max(-(-n // 8) * 8 for _, n in plan) <= (2 ** 31 - 1) // 512
+
+
+@pytest.mark.parametrize("n_tokens", [7900, 8192, 8300, 16384, 70000, 400000])
+@pytest.mark.parametrize("vocab", [5000, 16384, 50257, 152064])
+def test_mfma_backward_chunks_of_large_batches_stay_wide(n_tokens, vocab):
+    """A chunk of few columns is a short K between two passes over d_hidden's
+    accumulator: 8192 columns at least, in whole rounds of the 256 CUs."""
+    from kernel_opt.lmhead import _mfma_chunks
+    plan = _mfma_chunks(n_tokens, vocab, None)
+    cols = plan[0][1]
+    assert cols == vocab or 8192 <= cols <= 8192 * 1.25
+    assert all(n == cols for _, n in plan[:-1])
+    if cols < vocab:
+        tiles = cols // 256 * -(-n_tokens // 256)
+        assert tiles / (-(-tiles // 256) * 256) > 0.95

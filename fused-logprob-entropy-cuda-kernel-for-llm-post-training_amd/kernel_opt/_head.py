@@ -27,6 +27,23 @@ of the chip idle there and d_hidden is two launches.  Ours against the library
     512   32000   4096  102 / 98
     512   50240   2048  92 / 101
     1024  152064  3584  843 / 902    971 / 1198   895 / 1475
+From 8192 tokens on the library's logits and, for vocabularies (or chunks of
+them) below 2^17, its d_hidden are ahead: it reaches 1450-1500 TFLOP/s there, ours
+1300-1400, one workgroup a CU whose tile's stores overlap with nothing (65536
+tokens of [16384, 1024]: the forward's fold of the same tiles 1740 us, writing
+them 2230; fewer token blocks at a time on an XCD changed neither by more than
+2%):
+    4096  16384   1024  114 / 115    107 / 134    124 / 154
+    4096  50264   768   316 / 361    289 / 357    324 / 526
+    4096  32000   4096  742 / 723    841 / 1031   840 / 791
+    4096  152064  3584  3220 / 3085  3515 / 4076  3643 / 4915
+    8192  16384   1024  265 / 215    201 / 252    224 / 263
+    8192  50264   768   700 / 581    593 / 657    673 / 590
+    8192  32000   4096  1573 / 1494  1668 / 2084  1660 / 1582
+    8192  152064  3584  6622 / 6119  7021 / 7971  7152 / 9235
+    16384 16384   1024  581 / 422    418 / 525    436 / 415
+    16384 128256  2048  6835 / 6316  6793 / 7761  6586 / 6533
+    65536 32000   4096  12.6 / 11.6  13.8 / 16.3  13.4 / 13.0 (ms)
 The logits' token blocks of 256 (192, 128) do a remainder's work in full: the
 library is ahead where fewer than 7/10 of the padded tokens are real ones.
 """
@@ -59,7 +76,7 @@ def mfma_operands(h2: torch.Tensor, weight: torch.Tensor) -> bool:
 def logits_pay(n_tokens: int, vocab: int, dim: int) -> bool:
     padded = -(-n_tokens // 256) * 256
     return (10 * n_tokens >= 7 * padded and n_tokens * vocab * dim >= 15 << 30
-            and vocab % 8 == 0)
+            and n_tokens <= 4096 and vocab % 8 == 0)
 
 
 def d_weight_pays(vocab: int, dim: int) -> bool:
@@ -67,7 +84,8 @@ def d_weight_pays(vocab: int, dim: int) -> bool:
 
 
 def d_hidden_pays(n_tokens: int, vocab: int, dim: int) -> bool:
-    return n_tokens * vocab * dim >= 1 << 29
+    return (n_tokens * vocab * dim >= 1 << 29
+            and (n_tokens <= 4096 or vocab >= 1 << 17))
 
 
 def logits_into(out: torch.Tensor, h2: torch.Tensor, weight: torch.Tensor, stream) -> None:

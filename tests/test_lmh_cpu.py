@@ -203,3 +203,14 @@ def test_mfma_backward_chunks_of_large_batches_stay_wide(n_tokens, vocab):
     if cols < vocab:
         tiles = cols // 256 * -(-n_tokens // 256)
         assert tiles / (-(-tiles // 256) * 256) > 0.95
+
+
+def test_large_batches_take_the_faster_products():
+    """The measured sides of the rules: logits through the kernels from 7/10
+    real tokens up to 4096, d_hidden up to 4096 or over 2^17 columns."""
+    from kernel_opt._head import d_hidden_pays, d_weight_pays, logits_pay
+    assert logits_pay(1024, 152064, 3584) and logits_pay(4096, 50264, 768)
+    assert not logits_pay(8192, 152064, 3584) and not logits_pay(65536, 16384, 1024)
+    assert d_hidden_pays(4096, 16384, 1024) and d_hidden_pays(8192, 152064, 3584)
+    assert not d_hidden_pays(8192, 32000, 4096) and not d_hidden_pays(65536, 8192, 4096)
+    assert d_weight_pays(32000, 4096) and not d_weight_pays(8192, 768)

@@ -40,8 +40,9 @@ constexpr int kGrpoThreads = 256;
 // it is instead of converted by a launch before.  Rows kernel and backward,
 // bool mask, us before -> after, with the conversion: [8, 512] 3.6 + 3.0 + 3.6
 // -> 4.3 + 3.2, [1, 4749] 9.8 + 7.5 + 3.6 -> 5.3 + 3.6, [64, 4096] 9.2 + 7.9 +
-// 3.9 -> 6.1 + 4.1; the call with its backward, which the host's launches
-// bound, 65.2 -> 61.4 at [16, 2048].
+// 3.9 -> 6.1 + 4.1.  The call with its backward is bound by the host's
+// launches: 65-68 -> 62-64 at [16, 2048], where runs of one build differ by up
+// to 11%.
 constexpr int kGrpoUnroll = 4;
 constexpr int kGrpoLongThreads = 1024;
 constexpr int64_t kGrpoShortRow = kGrpoThreads * kGrpoUnroll;

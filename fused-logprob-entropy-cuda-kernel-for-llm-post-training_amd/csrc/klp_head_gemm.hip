@@ -27,8 +27,8 @@
 //
 // Bound: power and, in d_weight, the output's 1.1 GB and short tiles.  1024
 // tokens of a bf16 [152064, 3584] head: d_weight 971 us (1150 TFLOP/s; the
-// library GEMM 1198), d_hidden 895 us with the sum (1248 TFLOP/s; the library
-// 1475).  d_weight with 7 consecutive d tiles of one row block a workgroup,
+// library GEMM 1198 us), d_hidden 895 us with the sum (1248 TFLOP/s; the
+// library 1475 us).  d_weight with 7 consecutive d tiles of one row block a workgroup,
 // and the short ring for d_logits: 1140 us, its MFMAs busy half of the time.
 #include "klp_launch.h"
 #include "klp_mfma.h"

@@ -21,9 +21,9 @@
 //    online softmax update runs lane-locally, with no cross-lane reduction
 //    until the end of the chunk;
 //  - K advances in stages of 64 columns, a whole 128-byte line of every row,
-//    so that no line is asked for in two halves (with 64-byte stages 40% of
-//    the CU's cycles went to requests waiting behind a pending miss of their
-//    own line);
+//    so that no line is asked for in two halves, the second waiting behind
+//    the first's pending miss (TCP_PENDING_STALL_CYCLES, 1024 tokens of
+//    [152064, 3584]: 1.5e8 a launch, 3.2e8 with 64-byte stages);
 //  - the stages go through LDS by direct copies (buffer_load_dwordx4 ... lds,
 //    no register staging), all 160 KB of it: a ring of 3 stages of weight
 //    rows (32 KB each), which come from HBM, and of 2 stages of hidden rows,

@@ -75,7 +75,7 @@ __device__ __forceinline__ float value(float acc) {
 }
 
 // The wait states between the last MFMA and a VALU read of its result (11 for
-// an MFMA of 8 passes), rounded up.
+// an MFMA of 8 passes; these are busy for 16 cycles, 4 passes), rounded up.
 __device__ __forceinline__ void drain() { asm volatile("s_nop 15\n\ts_nop 7"); }
 
 // Two floats rounded to DT and packed, the first in the low half.

@@ -31,8 +31,9 @@ From 8192 tokens on the library's logits and, for vocabularies (or chunks of
 them) below 2^17, its d_hidden are ahead: it reaches 1450-1500 TFLOP/s there, ours
 1300-1400, one workgroup a CU whose tile's stores overlap with nothing (65536
 tokens of [16384, 1024]: the forward's fold of the same tiles 1740 us, writing
-them 2230; fewer token blocks at a time on an XCD changed neither by more than
-2%):
+them 2230).  Fewer token blocks at a time on an XCD, for its L2: 8192 tokens of
+[50264, 768] 701 -> 591 us, of [152064, 3584] 6623 -> 6285, [16384, 1024] and
+[32000, 4096] unchanged; all behind the library still.
     4096  16384   1024  114 / 115    107 / 134    124 / 154
     4096  50264   768   316 / 361    289 / 357    324 / 526
     4096  32000   4096  742 / 723    841 / 1031   840 / 791
@@ -68,8 +69,8 @@ def _rows_ok(t: torch.Tensor) -> bool:
 def mfma_operands(h2: torch.Tensor, weight: torch.Tensor) -> bool:
     """True when the MFMA kernels take hidden ``[N, D]`` and weight ``[V, D]``
     (one dtype, one device, rows with unit stride)."""
-    return (h2.device == weight.device and h2.dtype in (torch.bfloat16, torch.float16) and h2.size(0) > 0
-            and h2.size(1) >= 64 and h2.size(1) % 64 == 0 and h2.stride(1) == 1
+    return (h2.device == weight.device and h2.dtype in (torch.bfloat16, torch.float16)
+            and h2.size(0) > 0 and h2.size(1) >= 64 and h2.size(1) % 64 == 0 and h2.stride(1) == 1
             and weight.stride(1) == 1 and _rows_ok(h2) and _rows_ok(weight))
 
 

@@ -34,23 +34,39 @@ namespace {
 constexpr int kGrpoThreads = 256;
 // What bounds the loss is latency: launches, and in few long rows (one
 // workgroup a row, for sums in a fixed order) the chain of loads a thread
-// waits for.  So a thread loads kGrpoUnroll tokens before it uses any, rows of
-// more than kGrpoShortRow tokens, which would take a second such step with
-// kGrpoThreads, have kGrpoLongThreads, and a bool or integer mask is read as
-// it is instead of converted by a launch before.  Rows kernel and backward,
-// bool mask, us before -> after, with the conversion: [8, 512] 3.6 + 3.0 + 3.6
-// -> 4.3 + 3.2, [1, 4749] 9.8 + 7.5 + 3.6 -> 5.3 + 3.6, [64, 4096] 9.2 + 7.9 +
-// 3.9 -> 6.1 + 4.1.  The call with its backward is bound by the host's
-// launches: 65-68 -> 62-64 at [16, 2048], where runs of one build differ by up
-// to 11%.
+// waits for.  So a thread loads kGrpoUnroll tokens before it uses any, long
+// rows have kGrpoLongThreads while the CUs have the room, and a bool or integer
+// mask is read as it is instead of converted by a launch before.  The call with
+// its backward is bound by the host's launches: 65-68 -> 62-64 us at [16, 2048],
+// where runs of one build differ by up to 11%.
 constexpr int kGrpoUnroll = 4;
 constexpr int kGrpoLongThreads = 1024;
 constexpr int64_t kGrpoShortRow = kGrpoThreads * kGrpoUnroll;
-// Millions of rows fill the chip as they are, and 2^22 workgroups of 1024
-// threads would pass a grid's 2^32 threads.
-static int row_threads(const GrpoParams& p) {
-    return p.S > kGrpoShortRow && p.B <= (1 << 20) ? kGrpoLongThreads : kGrpoThreads;
+// Threads of a row that one workgroup sums.  1024 while there is at most a row
+// a CU, in rows longer than `longer_than` (below, their merge costs more than
+// the loads they take over), and up to two rows a CU beyond 4096 tokens; more
+// rows fill the CUs with 256 threads each.  GPU time, us, 256 / 1024 threads:
+//   rows x tokens  forward, token level  sequence level  its backward
+//   64 x 1025      6.2 / 6.9             7.2 / 8.1       4.7 / 4.3
+//   64 x 2048      6.8 / 6.9             8.1 / 8.2       5.8 / 4.8
+//   64 x 3000      8.0 / 7.4             9.8 / 8.9       7.5 / 5.3
+//   256 x 8192     14.3 / 10.2           19.4 / 12.4     17.1 / 9.3
+//   300 x 3000     8.6 / 10.1            10.3 / 12.3     8.1 / 9.4
+//   512 x 5000     12.3 / 12.3           16.2 / 15.1     14.4 / 14.0
+//   512 x 8192     16.9 / 15.7           23.8 / 21.2     23.2 / 20.2
+//   1000 x 1025    8.6 / 15.4            9.9 / 20.3      6.2 / 13.8
+//   2000 x 4096    24.9 / 30.0           37.5 / 45.4     33.6 / 42.5
+static int row_threads(const GrpoParams& p, int64_t longer_than) {
+    constexpr int64_t kCus = 256;
+    const bool room = p.B <= kCus ? p.S > longer_than : p.B <= 2 * kCus && p.S > 4096;
+    return room ? kGrpoLongThreads : kGrpoThreads;
 }
+// Rows of the token-level backward from which a workgroup takes a whole row
+// rather than a piece of it: 100000 x 64 51.3 -> 30.4 us, 30000 x 128 20.3 ->
+// 14.8 (the pieces' count is one more scalar load in front of the others), and
+// 2000 x 1100 7.6 -> 7.1; 1000 x 8192 is equal, 512 x 8192 12.2 in pieces, 15.3
+// whole.
+constexpr int64_t kGrpoManyRows = 1024;
 
 __device__ __forceinline__ float adv_at(const GrpoParams& p, int64_t b, int64_t i) {
     return p.adv_per_token ? p.adv[i] : p.adv[b];
@@ -217,9 +233,9 @@ __global__ __launch_bounds__(kGrpoThreads) void klp_grpo_finish_kernel(GrpoParam
 
 // d loss / d lp for every token, times the upstream gradient of the loss
 // (a device scalar, or 1 when null).  Reads the row sums of the forward.
-// Token level: pieces of kThreads * kGrpoUnroll tokens of the row, dealt over
-// blockIdx.y; sequence level: one workgroup a row.
-template <int kThreads>
+// One workgroup a row, or, token level only, kPieces: pieces of kThreads *
+// kGrpoUnroll tokens of it, dealt over blockIdx.y.
+template <int kThreads, bool kSequence, bool kPieces>
 __global__ __launch_bounds__(kThreads) void klp_grpo_bwd_kernel(GrpoParams p) {
     const int64_t b = blockIdx.x;
     const bool has_ref = p.ref_logp != nullptr && p.beta != 0.0f;
@@ -234,7 +250,7 @@ __global__ __launch_bounds__(kThreads) void klp_grpo_bwd_kernel(GrpoParams p) {
         scale = 1.0f / p.norm_const;
     scale *= g;
 
-    if (p.level == KLP_GRPO_SEQUENCE) {
+    if constexpr (kSequence) {
         // Every token shares w = sum_s (lp - lo) m / max(sum m, 1): the
         // ratio term's gradient is (sum_s' scale m_s' dw_s') * m_s / max(sum m, 1).
         float w_row, m_row;
@@ -249,17 +265,20 @@ __global__ __launch_bounds__(kThreads) void klp_grpo_bwd_kernel(GrpoParams p) {
             const TokenLoss t = token_loss(p, w_row, in.adv, in.lp, in.lr, has_ref);
             p.d_logp[i] = row_term * in.m + t.dlp * in.m * scale;
         });
-        return;
+    } else {
+        auto gradient = [&](int64_t i, const TokenIn& in) {
+            const TokenLoss t = token_loss(p, in.lp - in.lo, in.adv, in.lp, in.lr, has_ref);
+            p.d_logp[i] = (t.dw + t.dlp) * in.m * scale;
+        };
+        if constexpr (kPieces) {
+            constexpr int64_t kSpan = kThreads * kGrpoUnroll;
+            for (int64_t first = blockIdx.y * kSpan; first < p.S; first += gridDim.y * kSpan)
+                for_tokens<float>(p, b, has_ref, first + threadIdx.x, kThreads,
+                                  first + kSpan < p.S ? first + kSpan : p.S, gradient);
+        } else {
+            for_tokens<float>(p, b, has_ref, threadIdx.x, kThreads, p.S, gradient);
+        }
     }
-    constexpr int64_t kSpan = kThreads * kGrpoUnroll;
-    for (int64_t first = blockIdx.y * kSpan; first < p.S; first += gridDim.y * kSpan)
-        for_tokens<float>(p, b, has_ref, first + threadIdx.x, kThreads,
-                          first + kSpan < p.S ? first + kSpan : p.S,
-                          [&](int64_t i, const TokenIn& in) {
-                              const TokenLoss t = token_loss(p, in.lp - in.lo, in.adv, in.lp,
-                                                             in.lr, has_ref);
-                              p.d_logp[i] = (t.dw + t.dlp) * in.m * scale;
-                          });
 }
 
 namespace {
@@ -471,7 +490,7 @@ hipError_t launch_grpo_token_weights(const TokenWeightsParams& p, hipStream_t st
 template <typename Mask>
 static hipError_t launch_grpo_rows(const GrpoParams& p, hipStream_t stream) {
     const dim3 rows(static_cast<unsigned>(p.B));
-    return row_threads(p) == kGrpoThreads
+    return row_threads(p, 2 * kGrpoShortRow) == kGrpoThreads
                ? launch_kernel(klp_grpo_rows_kernel<kGrpoThreads, Mask>, rows, dim3(kGrpoThreads),
                                stream, p)
                : launch_kernel(klp_grpo_rows_kernel<kGrpoLongThreads, Mask>, rows,
@@ -491,15 +510,18 @@ hipError_t launch_grpo_fwd(const GrpoParams& p, hipStream_t stream) {
 hipError_t launch_grpo_bwd(const GrpoParams& p, hipStream_t stream) {
     const unsigned rows = static_cast<unsigned>(p.B);
     if (p.level == KLP_GRPO_SEQUENCE)
-        return row_threads(p) == kGrpoThreads
-                   ? launch_kernel(klp_grpo_bwd_kernel<kGrpoThreads>, dim3(rows),
+        return row_threads(p, kGrpoShortRow) == kGrpoThreads
+                   ? launch_kernel(klp_grpo_bwd_kernel<kGrpoThreads, true, false>, dim3(rows),
                                    dim3(kGrpoThreads), stream, p)
-                   : launch_kernel(klp_grpo_bwd_kernel<kGrpoLongThreads>, dim3(rows),
+                   : launch_kernel(klp_grpo_bwd_kernel<kGrpoLongThreads, true, false>, dim3(rows),
                                    dim3(kGrpoLongThreads), stream, p);
+    if (p.S <= kGrpoShortRow || p.B >= kGrpoManyRows)
+        return launch_kernel(klp_grpo_bwd_kernel<kGrpoThreads, false, false>, dim3(rows),
+                             dim3(kGrpoThreads), stream, p);
     const int64_t span = int64_t{kGrpoThreads} * kGrpoUnroll;
     const int64_t pieces = p.S < 1 ? 1 : (p.S + span - 1) / span;
     // 65535: the grid's second dimension; longer rows loop.
-    return launch_kernel(klp_grpo_bwd_kernel<kGrpoThreads>,
+    return launch_kernel(klp_grpo_bwd_kernel<kGrpoThreads, false, true>,
                          dim3(rows, static_cast<unsigned>(pieces < 65535 ? pieces : 65535)),
                          dim3(kGrpoThreads), stream, p);
 }

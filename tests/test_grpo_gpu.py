@@ -92,6 +92,18 @@ def test_shapes(B, S):
           dict(beta=0.04, loss_type="grpo"))
 
 
+@pytest.mark.parametrize("level", ["token", "sequence"])
+@pytest.mark.parametrize("B,S", [(2, 2048), (2, 2049), (256, 2100), (257, 2100), (257, 4097),
+                                 (513, 4097), (1023, 1025), (1024, 1025)])
+def test_rows_and_tokens_where_the_launch_changes(B, S, level):
+    """Both sides of the rules for threads a row and pieces of a row (ratios
+    inside the clip range but for a few: up to 2 million tokens)."""
+    new, old, ref, adv, mask = case(B, S, seed=17, spread=0.05)
+    check(new, old, ref, adv, mask,
+          dict(beta=0.04, loss_type="grpo", importance_level=level),
+          dict(beta=0.04, loss_type="grpo", level=level))
+
+
 def test_no_mask_and_all_masked():
     new, old, ref, adv, _ = case(3, 100, seed=14)
     check(new, old, ref, adv, None, dict(loss_type="bnpo"), dict(loss_type="bnpo"))

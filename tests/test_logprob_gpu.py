@@ -466,11 +466,12 @@ def test_one_element_path_matches_vector_path(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("V", [1, 7, 9, 4097, 50257])
+@pytest.mark.parametrize("V", [1, 7, 9, 1024, 1025, 4097, 50257])
 def test_backward_rows_at_different_offsets_bitwise(dtype, V):
     """Rows of logits at every offset within 16 bytes from their gradient's
     rows give the bits of rows that share it, over row ends, one piece and
-    several, with and without a temperature."""
+    several, with and without a temperature, on both sides of the length up to
+    which such rows go one element a lane."""
     from kernel_opt import _C
     N = 8
     per = 16 // torch.empty((), dtype=dtype).element_size()

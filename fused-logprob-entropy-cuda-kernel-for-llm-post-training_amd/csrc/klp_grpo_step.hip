@@ -539,8 +539,12 @@ static int capacity(int64_t vocab) {
 //    where 1024 threads of 70 VGPRs and more fit one.  bf16 [300, 40000]
 //    13.1 / 15.6, [512, 50240] 18.6 / 22.4, [1552, 53440] 64.9 / 72.9, [512,
 //    77824] 27.1 / 31.9; [128, 50240], a row a CU, 10.6 / 9.7.  fp32 has half
-//    the arithmetic to hide: [512, 32000] 22.3 / 23.3, [512, 24576] 15.9 /
-//    18.5, but past 1024 rows of more than 96 KB 74.0 / 72.0 ([1552, 32000]).
+//    the arithmetic to hide, and fewer places where that pays: rows of up to 96
+//    KB up to 512 rows ([512, 17000] 10.9 / 11.3, [1000, 17000] 26.2 / 24.8,
+//    [2047, 17000] 51.2 / 48.7), up to 128 KB from 512 to 1024 rows ([300,
+//    32768] 14.1 / 13.1, [512, 32768] 19.7 / 21.0, [1024, 32768] 44.3 / 46.7,
+//    [1100, 32768] 51.4 / 50.8), longer ones up to 1024 rows ([257, 38912] 15.9
+//    / 20.4, [1024, 38912] 56.6 / 58.9, [1552, 38912] equal).
 constexpr int64_t kCus = 256;
 
 template <int DT>
@@ -550,9 +554,13 @@ static hipError_t launch_step_dt(const GrpoStepParams& p, hipStream_t stream) {
     if (nvec <= 4 * 512) return launch_row<DT, 4, 512>(p, stream);
     if (nvec > 8 * 512 && nvec <= kGrpoStepMaxVec * 512 && p.n_rows > kCus &&
         p.n_rows < kPersistMinRowsPerWorkgroup * kCus) {
-        if (nvec <= 12 * 512) return launch_row<DT, 12, 512>(p, stream);
-        if (DT != kFP32 || p.n_rows <= 1024) {
-            if (nvec <= 16 * 512) return launch_row<DT, 16, 512>(p, stream);
+        const bool f32 = DT == kFP32;
+        if (nvec <= 12 * 512) {
+            if (!f32 || p.n_rows <= 512) return launch_row<DT, 12, 512>(p, stream);
+        } else if (nvec <= 16 * 512) {
+            if (!f32 || (p.n_rows >= 512 && p.n_rows <= 1024))
+                return launch_row<DT, 16, 512>(p, stream);
+        } else if (!f32 || p.n_rows <= 1024) {
             return launch_row<DT, kGrpoStepMaxVec, 512>(p, stream);
         }
     }

@@ -576,7 +576,8 @@ def test_persistent_rows_match_one_row_per_workgroup(dtype, B, S, V, temperature
 
 # Rows (in 16-byte vectors) and row counts at the edges of the dispatch: 256
 # threads up to 1024 vectors, 512 up to 2048, 1024 beyond; 512 again for 4097
-# .. 9728 vectors and 257 .. 2047 rows (12, 16 and 19 vectors a thread).
+# .. 9728 vectors and 257 .. 2047 rows (12, 16 and 19 vectors a thread; fp32 up
+# to 512 rows, 512 to 1024, and up to 1024).
 @pytest.mark.parametrize("dtype,rows,nvec", [
     (torch.bfloat16, 3, 1), (torch.bfloat16, 9, 255), (torch.float16, 5, 1024),
     (torch.bfloat16, 7, 1025), (torch.float32, 6, 2048), (torch.bfloat16, 5, 2049),
@@ -584,6 +585,8 @@ def test_persistent_rows_match_one_row_per_workgroup(dtype, B, S, V, temperature
     (torch.float16, 300, 6144), (torch.bfloat16, 290, 6145), (torch.bfloat16, 300, 8192),
     (torch.bfloat16, 260, 8193), (torch.float16, 258, 9728), (torch.bfloat16, 258, 9729),
     (torch.float32, 1024, 6145), (torch.float32, 1025, 6145), (torch.float32, 1025, 6144),
+    (torch.float32, 512, 4097), (torch.float32, 513, 4097), (torch.float32, 511, 8192),
+    (torch.float32, 512, 8192), (torch.float32, 1025, 8193), (torch.float32, 257, 9728),
     (torch.bfloat16, 2047, 4100), (torch.bfloat16, 2048, 4100)])
 @pytest.mark.parametrize("temperature", [1.0, 0.7])
 def test_threads_per_row(dtype, rows, nvec, temperature):

@@ -515,6 +515,32 @@ def test_unaligned_rows_take_the_library(dtype, stride, first, which, oracle):
     _check_chunked_backward(h, w, t, hd, wd, 400, 0.7, True, oracle)
 
 
+def test_widest_chunk_of_the_backward():
+    """A chunk as wide as the products' row stride allows (256 rows of d_logits
+    just below 2^31 bytes) gives the gradients of the default chunks: d_weight's
+    bits, whose sums over the tokens are the same; d_hidden, summed over 4.2
+    million columns in another order (sqrt(V) 2^-24 = 1.2e-4 of its terms'
+    sum), within one more rounding to bf16."""
+    from kernel_opt import fused_linear_logprob_entropy
+    from kernel_opt.lmhead import MFMA_CHUNK_MAX_COLS, _mfma_chunks
+    N, V, D = 260, MFMA_CHUNK_MAX_COLS + 3001, 64
+    g = torch.Generator(device=DEV).manual_seed(73)
+    h = torch.randn(N, D, device=DEV, generator=g).to(torch.bfloat16)
+    w = (torch.randn(V, D, device=DEV, generator=g) * 0.25).to(torch.bfloat16)
+    t = torch.randint(0, V, (N,), device=DEV, generator=g)
+    t[-1] = V - 1
+    gl = torch.linspace(-1, 1, N, device=DEV)
+    assert [n for _, n in _mfma_chunks(N, V, V)] == [MFMA_CHUNK_MAX_COLS, 3001]
+    grads = []
+    for chunk in (None, V):
+        ha, wa = h.clone().requires_grad_(True), w.clone().requires_grad_(True)
+        lp, ent, _ = fused_linear_logprob_entropy(ha, wa, t, chunk_vocab=chunk)
+        grads.append(torch.autograd.grad((lp, ent), (ha, wa), (gl, 0.1 * gl)))
+    assert torch.equal(grads[0][1], grads[1][1])
+    a, b = grads[0][0].float(), grads[1][0].float()
+    assert torch.all((a - b).abs() <= 2.0 ** -7 * a.abs() + 1e-3 * a.abs().amax(1, keepdim=True))
+
+
 def test_chunked_holds_no_full_logits():
     """At 1024 tokens of Qwen2.5-7B's vocabulary (V = 152064, with D = 1024
     to keep the weight small) neither pass allocates anything near the
